@@ -41,6 +41,11 @@ struct LevelJob {
     int32_t H, V, F, E, C;
     int32_t cV, cU, cH, cE, cF;
     int32_t xcd_remap, uv_refine, rare_cap, erep_read, erep_write;
+    // the rare-vertex table (RareView): offsets and counts, and the
+    // workgroups its vertices take in front of the job's in the masked
+    // vertex launch (0 without a table)
+    int64_t rv_item, rv_ent, rv_bnd;
+    int32_t rv_n4, rv_n8, rv_n64, rv_nb, rare_blocks;
     LevelTab t;
 };
 
@@ -72,6 +77,17 @@ struct AdjJob {
 template <class T>
 __host__ __device__ __forceinline__ T *arena_ptr(char *base, int64_t off) {
     return off < 0 ? nullptr : reinterpret_cast<T *>(base + off);
+}
+
+template <class J>
+__host__ __device__ __forceinline__ RareView arena_rare(char *base, const J &j) {
+    RareView r;
+    r.item = arena_ptr<const int4>(base, j.rv_item);
+    r.ent = arena_ptr<const int2>(base, j.rv_ent);
+    r.bnd = arena_ptr<const int4>(base, j.rv_bnd);
+    r.n4 = j.rv_n4; r.n8 = j.rv_n8; r.n64 = j.rv_n64; r.nb = j.rv_nb;
+    r.on = j.rv_item >= 0;
+    return r;
 }
 
 template <class J>

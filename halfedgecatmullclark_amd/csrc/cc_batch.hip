@@ -125,8 +125,13 @@ __global__ __launch_bounds__(256, W) void k_batch_vertices_masked(const LevelJob
     FusedArgs a;
     DCage c;
     unpack_level(J, arena, a, c);
+    const uint32_t b = lb - (uint32_t)start[k];
+    if (b < (uint32_t)J.rare_blocks) {
+        rare_vertices_block<GATHER, CREASED>(a, arena_rare(arena, J), J.t, d, b);
+        return;
+    }
     const JobLevelPtrs lp{J.lp, arena};
-    const int32_t wave = (int32_t)(lb - (uint32_t)start[k]) * 4 + (int32_t)(threadIdx.x >> 6);
+    const int32_t wave = (int32_t)(b - (uint32_t)J.rare_blocks) * 4 + (int32_t)(threadIdx.x >> 6);
     level_vertices_masked<GATHER, CREASED>(a, c, J.t, lp, d, wave);
 }
 

@@ -30,6 +30,10 @@ struct ccb_Batch {
         // element offsets of the cage's ring lists in `rings` (-1: walk the cage)
         int64_t o_vro = -1, o_vr = -1, o_vb = -1, o_fro = -1, o_fr = -1, o_voo = -1, o_vo = -1;
         int64_t o_he = 0, o_cr = 0, o_pts = 0, o_fin = 0, o_def = 0, o_adjB = 0, o_adjW = 0, o_rare = 0;
+        // the cage's rare-vertex table in `rings` (-1: its rare vertices go
+        // through the rare list)
+        int64_t o_ritem = -1, o_rent = -1, o_rbnd = -1;
+        RareView rv;   // its counts
         int64_t o_adjVP = 0;   // VParam offset of levels 1..D-1's vertex-rule parameters
         int32_t rare_cap = 0;   // rare-vertex list entries (FusedArgs::rare), the count first
         int64_t o_erep = -1;    // word offset of the edge-representative bits (depth >= 4)
@@ -236,6 +240,18 @@ bool ccb_Batch::create(const cc_Mesh *const *meshes, const int32_t *depths, int3
             g.o_fr = put(r.fring);
             g.o_voo = put(r.ooff);
             g.o_vo = put(r.out);
+            const RareTable rt = build_rare_table(m, r);
+            if (rt.ok) {   // records of two and four ints, read whole
+                auto put16 = [&](const std::vector<int32_t> &v) {
+                    rings_host.resize((rings_host.size() + 3) & ~size_t(3), 0);
+                    return put(v);
+                };
+                g.o_ritem = put16(rt.item);
+                g.o_rent = put16(rt.ent);
+                g.o_rbnd = put16(rt.bnd);
+                g.rv.n4 = rt.n4; g.rv.n8 = rt.n8; g.rv.n64 = rt.n64; g.rv.nb = rt.nb;
+                g.rv.on = 1;
+            }
         }
         g.o_he = tot_he; tot_he += g.n.cumH(g.D);
         g.o_cr = tot_cr; tot_cr += g.n.cumC(g.D);
@@ -443,8 +459,14 @@ bool ccb_Batch::build_tables() {
             j.ep = off(vp + g.n.V[d] + g.n.F[d]);
             j.defer_mask = off(defer_mask + g.o_def);
             j.owner_mask = cfg[d].kind == 1 && cfg[d].scan == 0 ? j.defer_mask : -1;
-            j.rare = j.owner_mask >= 0 ? off(rare + g.o_rare) : -1;
-            j.rare_cap = j.owner_mask >= 0 ? g.rare_cap : 0;
+            const bool listed = j.owner_mask >= 0 && !g.rv.on;
+            j.rare = listed ? off(rare + g.o_rare) : -1;
+            j.rare_cap = listed ? g.rare_cap : 0;
+            j.rv_item = g.rv.on ? off(rings + g.o_ritem) : -1;
+            j.rv_ent = g.rv.on ? off(rings + g.o_rent) : -1;
+            j.rv_bnd = g.rv.on ? off(rings + g.o_rbnd) : -1;
+            j.rv_n4 = g.rv.n4; j.rv_n8 = g.rv.n8; j.rv_n64 = g.rv.n64; j.rv_nb = g.rv.nb;
+            j.rare_blocks = j.owner_mask >= 0 && g.rv.on ? (int32_t)blocks_of(rare_waves(g.rv, d), 4) : 0;
             // edge-representative bits: the forward pass runs the fused
             // kernel on every level up to d, so levels 1..d are written in
             // the same pass before they are read
@@ -464,7 +486,7 @@ bool ccb_Batch::build_tables() {
             bd.push_back(blocks_of(blocks_of(blocks_of(g.n.H[d], 64), kDeferGroup), 4));
             bf.push_back(blocks_of(g.n.H[d], (int64_t)cfg[d].fb * cfg[d].ft));
             br.push_back(j.rare_cap > 0 ? blocks_of(j.rare_cap) : 0);
-            bv.push_back(cfg[d].scan == 0 ? blocks_of(blocks_of(blocks_of(g.n.H[d], 64), kOwnerWords), 4)
+            bv.push_back(cfg[d].scan == 0 ? j.rare_blocks + blocks_of(blocks_of(blocks_of(g.n.H[d], 64), kOwnerWords), 4)
                                           : blocks_of(g.n.H[d], 256 * cfg[d].scan));
         }
         tb.add(t_patch[d], jobs, bp);

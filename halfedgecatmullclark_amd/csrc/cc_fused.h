@@ -38,7 +38,7 @@ struct FusedArgs {
     uint64_t *owner_mask;
     // when set: the masked vertex kernel handles the vertices whose ring
     // follows from the child numbering and appends the others (cage-level
-    // and boundary fans) to this list, rare[0] their count (cleared by the
+    // and boundary fans; a cage with a rare-vertex table needs no list) to this list, rare[0] their count (cleared by the
     // fused kernel), rare[1 .. rare_cap] their representatives; the rare
     // kernel then finishes them
     int32_t *rare;
@@ -56,6 +56,29 @@ struct FusedArgs {
     // an unchanged topology), the fused kernel leaves them
     int owner_write = 1;
 };
+
+// The vertices of a cage's levels that no ring kernel takes, as cc_rare.h
+// reads them.  item: {vertex (a cage vertex, or V0 + face), first entry, n
+// halfedges, 1 on a boundary}, first the n4 items of at most 4 entries, then
+// the n8 of at most 8, then the n64 of at most 64; ent: {level-1 halfedge,
+// its level-1 edge, the sign bit set when its children 0 get odd edges} in
+// fan order, on a boundary followed by the edge of prev(last halfedge); bnd:
+// {h, next(h), edge(h), 0} of the nb boundary halfedges.  on: the table
+// stands in for the rare list.
+struct RareView {
+    const int4 *item = nullptr;
+    const int2 *ent = nullptr;
+    const int4 *bnd = nullptr;
+    int32_t n4 = 0, n8 = 0, n64 = 0, nb = 0, on = 0;
+};
+// waves (and workgroups of four waves, a multiple of 8 so that the
+// workgroups behind them keep their XCD) that level d's rare vertices take
+__host__ __device__ __forceinline__ int64_t rare_waves(const RareView &r, int d) {
+    return (r.n4 + (int64_t)r.nb * ((1 << d) - 1) + 15) / 16 + (r.n8 + 7) / 8 + r.n64;
+}
+__host__ __device__ __forceinline__ uint32_t rare_blocks(const RareView &r, int d) {
+    return r.on ? (uint32_t)((rare_waves(r, d) + 31) / 32 * 8) : 0u;
+}
 
 // topo: write child twin/edge/vertex IDs; uvMode: 0 leave uvIDs, 1 refine
 // them, 2 write 0; points: face and edge points of level d+1.
@@ -100,7 +123,10 @@ void launch_level_deferred(const FusedArgs &a, const DCage &c, const LevelTab &t
 // (scan: halfedges each thread of the compacted kernel tests, 2, 4 or 8;
 // 0: the owners marked in a.owner_mask by the fused kernel, with the masked
 // kernel compiled for `waves` waves per SIMD, 4, 6 or 8)
-void launch_level_vertices(const FusedArgs &a, const DCage &c, const LevelTab &t, const LevelPtrs &lp, int d,
-                           int gather, int creased, int fan, int scan, int waves, hipStream_t st);
+// rv: with on set, the masked kernel's launch also finishes the vertices of
+// the table, and a.rare may be null
+void launch_level_vertices(const FusedArgs &a, const DCage &c, const LevelTab &t, const LevelPtrs &lp,
+                           const RareView &rv, int d, int gather, int creased, int fan, int scan, int waves,
+                           hipStream_t st);
 
 }  // namespace cch

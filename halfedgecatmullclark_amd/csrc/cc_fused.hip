@@ -43,11 +43,17 @@ __global__ __launch_bounds__(NT) void k_level_fused(FusedArgs a, DCage c, LevelT
     }
 }
 
-// ring vertices only; the others to the rare list, then k_level_vertices_rare
+// ring vertices; the others in the first nr workgroups when the cage has a
+// rare-vertex table, else to the rare list and k_level_vertices_rare
 // (W waves per SIMD: 8 fit without spilling, 56 registers)
 template <int GATHER, int CREASED, int W>
-__global__ __launch_bounds__(256, W) void k_level_vertices_ring(FusedArgs a, DCage c, LevelTab t, LevelPtrs lp, int d) {
-    const uint32_t lb = xcd_block(blockIdx.x, gridDim.x, a.xcd_remap);
+__global__ __launch_bounds__(256, W) void k_level_vertices_ring(FusedArgs a, DCage c, LevelTab t, LevelPtrs lp, int d,
+                                                                RareView rv, uint32_t nr) {
+    if (blockIdx.x < nr) {
+        rare_vertices_block<GATHER, CREASED>(a, rv, t, d, blockIdx.x);
+        return;
+    }
+    const uint32_t lb = xcd_block(blockIdx.x - nr, gridDim.x - nr, a.xcd_remap);
     level_vertices_masked<GATHER, CREASED>(a, c, t, lp, d, (int32_t)(lb * 4 + (threadIdx.x >> 6)));
 }
 
@@ -305,15 +311,21 @@ static void launch_compact(const FusedArgs &a, const DCage &c, const LevelTab &t
 }
 
 template <int G, int C>
-static void launch_ring(const FusedArgs &a, const DCage &c, const LevelTab &t, const LevelPtrs &lp, int d, int waves,
-                        dim3 grid, hipStream_t st) {
-    if (waves == 4) hipLaunchKernelGGL((k_level_vertices_ring<G, C, 4>), grid, dim3(256), 0, st, a, c, t, lp, d);
-    else if (waves == 6) hipLaunchKernelGGL((k_level_vertices_ring<G, C, 6>), grid, dim3(256), 0, st, a, c, t, lp, d);
-    else hipLaunchKernelGGL((k_level_vertices_ring<G, C, kVertexWaves>), grid, dim3(256), 0, st, a, c, t, lp, d);
+static void launch_ring(const FusedArgs &a, const DCage &c, const LevelTab &t, const LevelPtrs &lp, int d,
+                        const RareView &rv, int waves, dim3 grid, hipStream_t st) {
+    const uint32_t nr = rare_blocks(rv, d);
+    grid.x += nr;
+    if (waves == 4)
+        hipLaunchKernelGGL((k_level_vertices_ring<G, C, 4>), grid, dim3(256), 0, st, a, c, t, lp, d, rv, nr);
+    else if (waves == 6)
+        hipLaunchKernelGGL((k_level_vertices_ring<G, C, 6>), grid, dim3(256), 0, st, a, c, t, lp, d, rv, nr);
+    else
+        hipLaunchKernelGGL((k_level_vertices_ring<G, C, kVertexWaves>), grid, dim3(256), 0, st, a, c, t, lp, d, rv, nr);
 }
 
-void launch_level_vertices(const FusedArgs &a, const DCage &c, const LevelTab &t, const LevelPtrs &lp, int d,
-                           int gather, int creased, int fan, int scan, int waves, hipStream_t st) {
+void launch_level_vertices(const FusedArgs &a, const DCage &c, const LevelTab &t, const LevelPtrs &lp,
+                           const RareView &rv, int d, int gather, int creased, int fan, int scan, int waves,
+                           hipStream_t st) {
     const dim3 block(256);
     const dim3 grid((unsigned)((a.H + 255) / 256));
     if (fan == 3) {
@@ -324,22 +336,22 @@ void launch_level_vertices(const FusedArgs &a, const DCage &c, const LevelTab &t
         else hipLaunchKernelGGL((k_level_vertices_direct<0, 0>), g3, block, 0, st, a, c, t, lp, d);
         return;
     }
-    if (fan == 2 && scan == 0 && a.owner_mask && a.rare) {   // owners marked by the fused kernel
+    if (fan == 2 && scan == 0 && a.owner_mask && (a.rare || rv.on)) {   // owners marked by the fused kernel
         const int64_t words = ((int64_t)a.H + 63) / 64;
-        const int64_t waves = (words + kOwnerWords - 1) / kOwnerWords;
-        const dim3 g0((unsigned)((waves + 3) / 4)), gr((unsigned)((a.rare_cap + 255) / 256));
+        const int64_t mask_waves = (words + kOwnerWords - 1) / kOwnerWords;
+        const dim3 g0((unsigned)((mask_waves + 3) / 4)), gr((unsigned)((a.rare_cap + 255) / 256));
         if (gather && creased) {
-            launch_ring<1, 1>(a, c, t, lp, d, waves, g0, st);
-            if (a.rare_cap > 0) hipLaunchKernelGGL((k_level_vertices_rare<1, 1>), gr, block, 0, st, a, c, t, lp, d);
+            launch_ring<1, 1>(a, c, t, lp, d, rv, waves, g0, st);
+            if (a.rare && a.rare_cap > 0) hipLaunchKernelGGL((k_level_vertices_rare<1, 1>), gr, block, 0, st, a, c, t, lp, d);
         } else if (gather) {
-            launch_ring<1, 0>(a, c, t, lp, d, waves, g0, st);
-            if (a.rare_cap > 0) hipLaunchKernelGGL((k_level_vertices_rare<1, 0>), gr, block, 0, st, a, c, t, lp, d);
+            launch_ring<1, 0>(a, c, t, lp, d, rv, waves, g0, st);
+            if (a.rare && a.rare_cap > 0) hipLaunchKernelGGL((k_level_vertices_rare<1, 0>), gr, block, 0, st, a, c, t, lp, d);
         } else if (creased) {
-            launch_ring<0, 1>(a, c, t, lp, d, waves, g0, st);
-            if (a.rare_cap > 0) hipLaunchKernelGGL((k_level_vertices_rare<0, 1>), gr, block, 0, st, a, c, t, lp, d);
+            launch_ring<0, 1>(a, c, t, lp, d, rv, waves, g0, st);
+            if (a.rare && a.rare_cap > 0) hipLaunchKernelGGL((k_level_vertices_rare<0, 1>), gr, block, 0, st, a, c, t, lp, d);
         } else {
-            launch_ring<0, 0>(a, c, t, lp, d, waves, g0, st);
-            if (a.rare_cap > 0) hipLaunchKernelGGL((k_level_vertices_rare<0, 0>), gr, block, 0, st, a, c, t, lp, d);
+            launch_ring<0, 0>(a, c, t, lp, d, rv, waves, g0, st);
+            if (a.rare && a.rare_cap > 0) hipLaunchKernelGGL((k_level_vertices_rare<0, 0>), gr, block, 0, st, a, c, t, lp, d);
         }
         return;
     }

@@ -7,6 +7,7 @@
 
 #include "../../include/CatmullClarkHIP.h"
 #include "cc_common.h"
+#include "cc_fused.h"
 
 namespace cch {
 
@@ -49,6 +50,8 @@ inline CageRings build_cage_rings(const cc_Mesh *m) {
     r.voff.assign((size_t)V + 1, 0);
     r.vbnd.assign((size_t)V, 0);
     r.foff.assign((size_t)F + 1, 0);
+    r.vring.reserve((size_t)H + 1);   // what a cage whose walks close needs
+    r.fring.reserve((size_t)H + 1);
     auto valid = [&](int32_t h) { return h >= 0 && h < H; };
     for (int32_t v = 0; v < V; ++v) {
         r.voff[v] = (int32_t)r.vring.size();
@@ -92,31 +95,91 @@ inline CageRings build_cage_rings(const cc_Mesh *m) {
     return r;
 }
 
-// True when every vertex of every level of this cage takes a structural ring
-// in the vertex passes (marked_ring_fan + structural_ring), so nothing is
-// left for the rare-vertex kernels: no boundary, every cage vertex with a
-// closed ring of four whose halfedges R have a twin with next(twin(R)) != R,
-// and every cage face a quad whose halfedges are f2h .. f2h+3 in next order.
-inline bool rings_without_rare(const cc_Mesh *m, const CageRings &r) {
-    const int32_t V = m->vertexCount, F = m->faceCount, H = m->halfedgeCount;
+// The rare-vertex table of a cage (RareView) as one run of int32s: items |
+// entries | boundary halfedges, item and boundary records of four ints,
+// entries of two.  `ok` is false when the cage does not fit it (walks that do
+// not close, links that contradict each other, a fan of more than 64
+// entries): its rare vertices then go through the rare list.
+struct RareTable {
+    std::vector<int32_t> item, ent, bnd;
+    int32_t n4 = 0, n8 = 0, n64 = 0, nb = 0;
+    bool ok = false;
+    bool empty() const { return n4 + n8 + n64 + nb == 0; }
+};
+
+inline RareTable build_rare_table(const cc_Mesh *m, const CageRings &r) {
+    RareTable t;
+    if (!r.ok) return t;
+    const int32_t V = m->vertexCount, F = m->faceCount, H = m->halfedgeCount, E = m->edgeCount;
     const CageHe *he = reinterpret_cast<const CageHe *>(m->halfedges);
-    for (int32_t h = 0; h < H; ++h)
-        if (he[h].twin < 0 || he[h].twin >= H) return false;
+    auto valid = [&](int32_t h) { return h >= 0 && h < H; };
+    for (int32_t h = 0; h < H; ++h) {
+        const CageHe &x = he[h];
+        if (!valid(x.next) || !valid(x.prev) || x.prev == h || x.next == h || he[x.next].prev != h ||
+            x.twin >= H || x.edge < 0 || x.edge >= E || x.face < 0 || x.face >= F)
+            return t;
+        if (x.twin >= 0 && (he[x.twin].twin != h || he[x.twin].edge != x.edge)) return t;
+    }
+    struct Item { int32_t v, first, n, boundary; };
+    std::vector<Item> items[3];
+    auto add_item = [&](int32_t v, int32_t n, int32_t boundary, size_t first) {
+        const int32_t entries = n + boundary;
+        const int k = entries <= 4 ? 0 : (entries <= 8 ? 1 : 2);
+        items[k].push_back({v, (int32_t)(first / 2), n, boundary});
+        return entries <= 64;
+    };
+    t.ent.resize(2 * (r.vring.size() + r.fring.size() + (size_t)V));
+    size_t used = 0;
+    auto add_ent = [&](int32_t h, int32_t e, bool odd) {
+        t.ent[used++] = h;
+        t.ent[used++] = odd ? (int32_t)((uint32_t)e | 0x80000000u) : e;
+    };
     for (int32_t v = 0; v < V; ++v) {
-        if (r.voff[v + 1] - r.voff[v] != 4 || r.vbnd[v] != 0) return false;
-        for (int32_t i = r.voff[v]; i < r.voff[v + 1]; ++i) {
-            const int32_t R = r.vring[i], w = he[R].twin;
-            const int32_t nt = he[w].next;
-            if (nt < 0 || nt >= H || nt == R) return false;
+        const int32_t o = r.voff[v], n = r.voff[v + 1] - o;
+        if (n == 0 || he[r.vring[o]].vert != v) continue;   // no halfedge represents v
+        const bool boundary = r.vbnd[v] != 0;
+        // A closed ring of four: marked_ring_fan and structural_ring take it
+        // (every entry has a twin w, and next(w) is the entry before it).
+        if (n == 4 && !boundary) continue;
+        const size_t first = used;
+        for (int32_t i = 0; i < n; ++i) {   // the ring's previous edge is the next entry's edge
+            const int32_t R = r.vring[o + i], w = he[R].twin;
+            const int32_t tw = w >= 0 ? 4 * he[w].next + 3 : -1;
+            add_ent(4 * R, 2 * he[R].edge + (R > w ? 0 : 1), 4 * R < tw);
         }
+        if (boundary) {
+            const int32_t R = r.vring[o + n - 1], p = he[R].prev;
+            add_ent(4 * R, 2 * he[p].edge + 1, true);
+        }
+        if (!add_item(v, n, boundary ? 1 : 0, first)) return t;
     }
     for (int32_t f = 0; f < F; ++f) {
-        const int32_t p = m->faceToHalfedgeIDs[f];
-        if (p < 0 || p + 3 >= H) return false;
-        if (he[p].next != p + 1 || he[p + 1].next != p + 2 || he[p + 2].next != p + 3 || he[p + 3].next != p)
-            return false;
+        const int32_t o = r.foff[f], n = r.foff[f + 1] - o;
+        if (n == 0 || he[r.fring[o]].face != f) continue;
+        const int32_t p = r.fring[o];
+        if (p + 3 < H && he[p].next == p + 1 && he[p + 1].next == p + 2 && he[p + 2].next == p + 3 &&
+            he[p + 3].next == p)
+            continue;
+        const size_t first = used;
+        for (int32_t i = 0; i < n; ++i) {
+            const int32_t q = r.fring[o + i], pr = he[q].prev;
+            add_ent(4 * q + 2, 2 * E + pr, 4 * q + 2 < 4 * pr + 1);
+        }
+        if (!add_item(V + f, n, 0, first)) return t;
     }
-    return true;
+    t.ent.resize(used);
+    for (const auto &group : items) {
+        const int32_t *p = reinterpret_cast<const int32_t *>(group.data());
+        t.item.insert(t.item.end(), p, p + 4 * group.size());
+    }
+    t.n4 = (int32_t)items[0].size();
+    t.n8 = (int32_t)items[1].size();
+    t.n64 = (int32_t)items[2].size();
+    for (int32_t h = 0; h < H; ++h)
+        if (he[h].twin < 0) t.bnd.insert(t.bnd.end(), {h, he[h].next, he[h].edge, 0});
+    t.nb = (int32_t)(t.bnd.size() / 4);
+    t.ok = true;
+    return t;
 }
 
 // host-memory view of a cage with the device-view type (for the O(depth) maps)

@@ -11,6 +11,7 @@
 
 #include "cc_fan.h"
 #include "cc_fused.h"
+#include "cc_rare.h"
 
 namespace cch {
 
@@ -395,8 +396,9 @@ __device__ __forceinline__ void mask_group(const uint64_t *mask, int32_t w0, int
 }
 
 // A marked owner whose ring follows from the child numbering: its vertex
-// point; any other goes to the rare list (no general fan code here, so the
-// kernel keeps fewer registers and runs more waves).
+// point; any other goes to the rare list when there is one, else its waves
+// of rare_vertices have it (no general fan code here, so the kernel keeps
+// fewer registers and runs more waves).
 template <int GATHER, int CREASED>
 struct RingVertexFn {
     const FusedArgs &a;
@@ -408,8 +410,10 @@ struct RingVertexFn {
         Fan f;
         int32_t v, r[4], e[4];
         if (!marked_ring_fan(h, d, c, t, lp.he, f, v) || !structural_ring(f, t, d, v, r, e, c)) {
-            const int32_t slot = atomicAdd(a.rare, 1);
-            if (slot < a.rare_cap) a.rare[1 + slot] = h;
+            if (a.rare) {
+                const int32_t slot = atomicAdd(a.rare, 1);
+                if (slot < a.rare_cap) a.rare[1 + slot] = h;
+            }
             return;
         }
         const FanPreloaded pre = closed_fan(a, r, e);
@@ -431,6 +435,17 @@ __device__ __forceinline__ void level_vertices_masked(const FusedArgs &a, const 
     const int32_t words = (a.H + 63) >> 6;
     mask_group<kOwnerWords>(a.owner_mask, wave * kOwnerWords, words, list[threadIdx.x >> 6],
                             RingVertexFn<GATHER, CREASED>{a, c, st, slp, d});
+}
+
+// workgroup `block` (four waves) of the level's rare vertices
+template <int GATHER, int CREASED>
+__device__ __forceinline__ void rare_vertices_block(const FusedArgs &a, const RareView &r, const LevelTab &t, int d,
+                                                    uint32_t block) {
+    __shared__ LevelTab st;
+    __shared__ RareLds x[4];
+    lds_fill(st, t);
+    __syncthreads();
+    rare_vertices<GATHER, CREASED>(a, r, st, d, (int32_t)(block * 4 + (threadIdx.x >> 6)), x[threadIdx.x >> 6]);
 }
 
 // the vertices the ring-only masked kernel listed, one thread each

@@ -38,9 +38,14 @@ struct ccd_Subd {
     int32_t *rare = nullptr;
     int32_t rare_cap = 0;
     bool rings_ok = false;
-    // no vertex of this cage can reach the rare lists (rings_without_rare):
-    // the vertex passes get a capacity of 0 and no rare kernel runs
+    // no vertex of this cage can reach the rare lists (an empty rare-vertex
+    // table): the vertex passes get a capacity of 0 and no rare kernel runs
     bool rare_free = false;
+    // the rare-vertex table (cch::RareView) in `rings`, rare_on when the cage
+    // fits it; offsets in ints
+    bool rare_on = false;
+    size_t o_ritem = 0, o_rent = 0, o_rbnd = 0;
+    int32_t rare_n4 = 0, rare_n8 = 0, rare_n64 = 0, rare_nb = 0;
     // levels 1..D, cumulative, laid out as cc_Subd's arrays
     cch::He *he = nullptr;
     cch::Crease *cr = nullptr;
@@ -103,6 +108,7 @@ struct ccd_Subd {
     cch::Lvl level_view(int d, const cch::P3 *levelPts, cch::P3 *nextPts) const;
     cch::FusedArgs fused_args(int d, const cch::P3 *points) const;
     cch::LevelPtrs level_ptrs() const;
+    cch::RareView rare_view() const;
     void cage_points(int32_t steps, const cch::P3 *cagePts, cch::P3 *out, hipStream_t st);
     bool refine(int32_t steps, int dmax, hipStream_t st);
     bool refine_graph(int32_t steps, hipStream_t st);

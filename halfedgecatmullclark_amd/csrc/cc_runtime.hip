@@ -156,7 +156,10 @@ bool ccd_Subd::upload_cage(const cc_Mesh *cage, hipStream_t st) {
     // vertex rings | face rings], each list padded by one entry
     const CageRings r = build_cage_rings(cage);
     rings_ok = r.ok;
-    rare_free = r.ok && rings_without_rare(cage, r);
+    const RareTable rt = build_rare_table(cage, r);
+    rare_free = rt.ok && rt.empty();
+    rare_on = rt.ok;
+    rare_n4 = rt.n4; rare_n8 = rt.n8; rare_n64 = rt.n64; rare_nb = rt.nb;
     if (!r.ok) return true;
     std::vector<int32_t> rings_host;
     auto put = [&](const std::vector<int32_t> &v) {
@@ -172,6 +175,15 @@ bool ccd_Subd::upload_cage(const cc_Mesh *cage, hipStream_t st) {
     o_fr = put(r.fring);
     o_voo = put(r.ooff);
     o_vo = put(r.out);
+    if (rt.ok) {   // records of two and four ints, read whole
+        auto put16 = [&](const std::vector<int32_t> &v) {
+            rings_host.resize((rings_host.size() + 3) & ~size_t(3), 0);
+            return put(v);
+        };
+        o_ritem = put16(rt.item);
+        o_rent = put16(rt.ent);
+        o_rbnd = put16(rt.bnd);
+    }
     if (rings_host.size() > rings_cap) {
         if (rings) (void)hipFree(rings);
         rings = nullptr;
@@ -199,6 +211,17 @@ DCage ccd_Subd::cage_view(const P3 *points) const {
     }
     c.V = V0; c.U = U0; c.H = H0; c.E = E0; c.F = F0;
     return c;
+}
+
+RareView ccd_Subd::rare_view() const {
+    RareView r;
+    if (!rare_on) return r;
+    r.item = reinterpret_cast<const int4 *>(rings + o_ritem);
+    r.ent = reinterpret_cast<const int2 *>(rings + o_rent);
+    r.bnd = reinterpret_cast<const int4 *>(rings + o_rbnd);
+    r.n4 = rare_n4; r.n8 = rare_n8; r.n64 = rare_n64; r.nb = rare_nb;
+    r.on = 1;
+    return r;
 }
 
 Lvl ccd_Subd::level_view(int d, const P3 *levelPts, P3 *nextPts) const {
@@ -338,8 +361,10 @@ void ccd_Subd::level_fused(int d, int32_t steps, int topo, int uvMode, P3 *point
     if (pts_ && opt_fan == 2 && cfg[d].scan == 0) {
         a.owner_mask = own_masks + own_off[d];
         a.owner_write = own_valid[d] && !topo ? 0 : 1;
-        a.rare = rare;
-        a.rare_cap = rare_free ? 0 : rare_cap;   // 0: the list stays empty, no rare kernel
+        if (!rare_on) {
+            a.rare = rare;
+            a.rare_cap = rare_free ? 0 : rare_cap;   // 0: the list stays empty, no rare kernel
+        }
     }
     // edge-representative bits: derive level d+1's while they are still
     // needed (levels up to D-2), read levels 1..d-1 in the owner test
@@ -364,7 +389,8 @@ void ccd_Subd::level_fused(int d, int32_t steps, int topo, int uvMode, P3 *point
     }
     if (pts_) {
         launch_timed("level_vertices", n.H[d], st, [&] {
-            launch_level_vertices(a, c, tab, level_ptrs(), d, gather, creased, opt_fan, cfg[d].scan, cfg[d].vw, st);
+            launch_level_vertices(a, c, tab, level_ptrs(), rare_view(), d, gather, creased, opt_fan, cfg[d].scan,
+                                  cfg[d].vw, st);
         });
     }
 }
