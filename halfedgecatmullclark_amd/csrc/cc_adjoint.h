@@ -37,12 +37,24 @@ struct AdjArgs {
     // after the vertex rule's shares (gEu, 3 E scalars)
     T *W;
     VParam<T> *VP;
+    // beside VP, a byte per vertex: 1 when its parameters are those of a
+    // smooth interior vertex of valence 4 (or null: read VP for every one)
+    uint8_t *plain = nullptr;
+    // the parent level's records and counts, to derive this level's records
+    // from (null: read them)
+    const He *par = nullptr;
+    int32_t pV = 0, pF = 0, pE = 0;
     T *gEu;
     // the face gradients after the quad pass (3 F scalars), or null: the
     // quad pass then updates gF in place
     T *gFu = nullptr;
     // edge-representative bits of levels 1..d-1 (FusedArgs::erep), or null
     const uint64_t *erep = nullptr;
+    // the tile pass: the weight and share of every border halfedge (4 H
+    // scalars, in the place of gEu and gFu), and two bits per halfedge: it is
+    // a border halfedge; it finishes its vertex
+    T *Cs = nullptr;
+    uint64_t *border = nullptr, *mark = nullptr;
     // when set: the vertex pass leaves the vertices whose ring does not
     // follow from the child numbering (cage vertices, cage faces other than
     // quads with consecutive halfedges, boundary edge vertices) to the rare
@@ -54,13 +66,13 @@ struct AdjArgs {
 };
 
 // scalars of adjoint scratch (AdjArgs::W) a cage refined to depth D needs:
-// the cage step's weights and every level's parameters and edge gradients
-// (face_out: and its face gradients, AdjArgs::gFu), a multiple of 4 so that
-// consecutive cages' scratch stays 16-byte aligned
-inline int64_t adj_scratch_scalars(const Counts &n, int D, bool face_out = false) {
+// the cage step's weights and every level's parameters and its edge
+// and face gradients, or the tile pass's shares (AdjArgs::Cs) with tiles set;
+// a multiple of 4 so that consecutive cages' scratch stays 16-byte aligned
+inline int64_t adj_scratch_scalars(const Counts &n, int D, bool tiles) {
     int64_t m = 4 * n.H[0];
     for (int d = 1; d < D; ++d) {
-        const int64_t need = 4 * n.V[d] + 3 * n.E[d] + (face_out ? 3 * n.F[d] : 0);
+        const int64_t need = 4 * n.V[d] + (tiles ? 4 * n.H[d] : 3 * n.E[d] + 3 * n.F[d]);
         if (need > m) m = need;
     }
     return (m + 3) & ~int64_t(3);
@@ -81,15 +93,20 @@ struct AdjPlan {
     // creases; vp_valid: they hold this topology's, so the parameter pass is
     // skipped (null: the parameters go to the scratch W, every call)
     void *vp_cache = nullptr;
+    uint8_t *vp_plain = nullptr;   // AdjArgs::plain of the same vertices
     bool vp_valid = false;
     // the vertex pass's rare-vertex list (AdjArgs::rare), or null
     int32_t *rare = nullptr;
     int32_t rare_cap = 0;
+    // the cage's rare-vertex table; with it on, quads and vertices run as one
+    // tile pass, with border and mark bits for the largest level below D
+    RareView rv;
+    uint64_t *border = nullptr, *mark = nullptr;
 };
 
 // dL/d(cage points) from dL/d(level-D points): V_D x 3 in (only read),
 // V_0 x 3 out.  bufA holds V_{D-2} x 3 scalars of scratch (V_D x 3 when
-// D = 1), bufB V_{D-1} x 3, W adj_scratch_scalars(n, D, true).
+// D = 1), bufB V_{D-1} x 3, W adj_scratch_scalars(n, D, rv.on).
 // When sharp is given (E_0 + Ccum(D-1) scalars) the sharpness of every level
 // is refined again in T and used instead of the float crease records.
 template <typename T>

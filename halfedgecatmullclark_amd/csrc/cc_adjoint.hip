@@ -25,6 +25,7 @@
 #include "cc_adjoint.h"
 #include "cc_batch.h"
 #include "cc_fan.h"
+#include "cc_rare.h"
 
 namespace cch {
 
@@ -55,7 +56,8 @@ __device__ __forceinline__ T sgnT(T x) { return x < (T)0 ? (T)-1 : (x > (T)0 ? (
 template <typename T>
 __device__ __forceinline__ T sharp_at(const AdjArgs<T> &a, int32_t e) {
     if (e >= a.C) return (T)0;
-    return a.sd ? a.sd[e] : (T)a.cr[e].sharp;
+    if (sizeof(T) == sizeof(double) && a.sd) return a.sd[e];   // never given in float
+    return (T)at3(a.cr, e)->sharp;
 }
 
 template <typename T>
@@ -71,7 +73,7 @@ struct RingT {
 
 // ---- level d >= 1, gather form -------------------------------------------------
 template <typename T>
-struct W4 { T a, b, g, dl; };
+struct alignas(16) W4 { T a, b, g, dl; };
 
 // The cage step's weights live as four arrays of the cage's H scalars,
 // a | b | g | dl, so that each pass reads only the one it needs.
@@ -215,18 +217,11 @@ __device__ __forceinline__ VParam<T> vparam_of(const RingT<T> &rp, bool creased)
 // g is -0, its b +0).
 template <typename T>
 __device__ __forceinline__ VW<T> vparam_weights(const VParam<T> &p, T ts, T ps, int32_t edge, bool creased) {
-    VW<T> w{0, 0, 0, 0};
+    VW<T> w{p.s1, (T)-4 * p.s2, p.s2, 0};   // the smooth rule: nearly every vertex
     const int rule = creased ? (p.nb >> 28) & 3 : 0;
-    if (rule == 0) {
-        w.a = p.s1;
-        w.b = (T)-4 * p.s2;
-        w.g = p.s2;
-        return w;
-    }
-    if (rule == 1) {
-        w.a = p.s1;
-        return w;
-    }
+    if (rule == 0) return w;
+    w.b = w.g = 0;
+    if (rule == 1) return w;
     const T n = (T)(p.nb & 0x0FFFFFFF);
     const bool boundary = ((p.nb >> 30) & 1) != 0;
     // two sharp ring edges: the sum of the sharpness this halfedge's walk
@@ -261,37 +256,34 @@ __device__ __forceinline__ void adj_params_fan(const AdjArgs<T> &a, const DCage 
     } else {
         rp = ring_params<T, CREASED>(a, c, f);
     }
-    a.VP[v] = vparam_of<T>(rp, CREASED);
+    const VParam<T> p = vparam_of<T>(rp, CREASED);
+    a.VP[v] = p;
+    if (a.plain) a.plain[v] = p.nb == 4 ? 1 : 0;   // smooth, interior, valence 4
 }
 
-// value held by the lane of the next halfedge of the same quad, for any
-// dword-sized record (DPP quad_perm)
-template <class S>
-__device__ __forceinline__ S quad_next_rec(const S &v) {
+// value held by another lane of the same quad, for any record of whole dwords
+// (DPP quad_perm CTRL)
+template <int CTRL, class S>
+__device__ __forceinline__ S quad_rel_rec(const S &v) {
     static_assert(sizeof(S) % 4 == 0, "whole dwords");
     S r;
 #pragma unroll
     for (int i = 0; i < (int)(sizeof(S) / 4); ++i)
-        reinterpret_cast<int *>(&r)[i] = quad_rel<kQuadNext>(reinterpret_cast<const int *>(&v)[i]);
-    return r;
-}
-template <int K, class S>
-__device__ __forceinline__ S quad_bcast_rec(const S &v) {
-    static_assert(sizeof(S) % 4 == 0, "whole dwords");
-    S r;
-#pragma unroll
-    for (int i = 0; i < (int)(sizeof(S) / 4); ++i)
-        reinterpret_cast<int *>(&r)[i] = quad_bcast<K>(reinterpret_cast<const int *>(&v)[i]);
+        reinterpret_cast<int *>(&r)[i] = quad_rel<CTRL>(reinterpret_cast<const int *>(&v)[i]);
     return r;
 }
 template <class S>
-__device__ __forceinline__ S quad_prev_rec(const S &v) {
-    static_assert(sizeof(S) % 4 == 0, "whole dwords");
-    S r;
-#pragma unroll
-    for (int i = 0; i < (int)(sizeof(S) / 4); ++i)
-        reinterpret_cast<int *>(&r)[i] = quad_rel<kQuadPrev>(reinterpret_cast<const int *>(&v)[i]);
-    return r;
+__device__ __forceinline__ S quad_next_rec(const S &v) { return quad_rel_rec<kQuadNext>(v); }
+template <class S>
+__device__ __forceinline__ S quad_prev_rec(const S &v) { return quad_rel_rec<kQuadPrev>(v); }
+
+// the sum of v over the four lanes of the quad, (0 + 1) + (2 + 3) in each
+template <typename T>
+__device__ __forceinline__ V3<T> quad_sum(V3<T> v) {
+    constexpr int kSwap1 = 0xB1, kSwap2 = 0x4E;   // quad_perm [1,0,3,2], [2,3,0,1]
+    const auto plus = [](V3<T> a, const auto &b) { return V3<T>{a.x + b.x, a.y + b.y, a.z + b.z}; };
+    v = plus(v, quad_rel_rec<kSwap1>(v));
+    return plus(v, quad_rel_rec<kSwap2>(v));
 }
 
 template <typename T>
@@ -309,16 +301,53 @@ __device__ __forceinline__ void add_w(V3<T> &acc, T w, const V3<T> &g) {
 // of each of its edges itself, in the order of the edge's larger halfedge
 // (both quads of an edge get the same bits), and from them and its corners
 // the updated gradient of its face; the larger halfedge stores its edge's.
+template <typename T>
+struct QuadParts {
+    int4 x;             // h's record
+    bool live, owner;   // owner: h is the larger halfedge of its pair
+    V3<T> gv, ge, gf;   // its vertex's gradient, its edge's and its face's updated ones
+    T wa, c0, c1;       // its weights in the vertex rule (on the vertex) and the edge rule (own, next vertex)
+};
+
+// What a halfedge's lane loads, in two rounds: its record (DERIVE: the parent
+// level's record it follows from), then everything the record leads to.  A
+// lane past the level's end reads quad 0 instead, so that no load of a round
+// waits behind a branch.
+template <typename T>
+struct QuadIn {
+    int4 x;
+    bool live, plain;
+    V3<T> gv, ge, gf;
+    T ts;
+};
+
+template <typename T, bool DERIVE>
+__device__ __forceinline__ void adj_quad_record(const AdjArgs<T> &a, int32_t h, QuadIn<T> &q) {
+    q.live = h < a.H;   // H is a multiple of 4: quads are whole
+    const int32_t g = q.live ? h : h & 3;
+    q.x = DERIVE ? he_gld(a.par, derived_from(g)) : he_gld(a.he, g);
+}
+
+template <typename T, int CREASED, bool DERIVE>
+__device__ __forceinline__ void adj_quad_gather(const AdjArgs<T> &a, int32_t h, QuadIn<T> &q) {
+    const int32_t g = q.live ? h : h & 3;
+    if (DERIVE) q.x = derived_record(q.x, g, a.pV, a.pF, a.pE);
+    q.gv = *at3(reinterpret_cast<const V3<T> *>(a.gV), q.x.z);
+    q.ge = *at3(reinterpret_cast<const V3<T> *>(a.gE), q.x.y);
+    q.gf = *at3(reinterpret_cast<const V3<T> *>(a.gF), g >> 2);
+    q.ts = CREASED ? sharp_at(a, q.x.y) : (T)0;
+    q.plain = sizeof(T) == sizeof(float) && a.plain && a.plain[q.x.z] != 0;
+}
+
 template <typename T, int CREASED>
-__device__ __forceinline__ void adj_quad_at(const AdjArgs<T> &a, int32_t h) {
-    if (a.rare && h == 0) a.rare[0] = 0;   // the vertex pass that follows appends
-    const bool live = h < a.H;   // H is a multiple of 4: quads are whole
-    const int4 x = live ? he_gld(a.he, h) : make_int4(0, 0, 0, 0);
-    const V3<T> *gV = reinterpret_cast<const V3<T> *>(a.gV);
-    const VParam<T> P = a.VP[x.z];   // a dead lane's record is all zeros: vertex 0
-    const V3<T> gv = gV[x.z];
-    const V3<T> ge0 = live ? reinterpret_cast<const V3<T> *>(a.gE)[x.y] : V3<T>{0, 0, 0};
-    const T ts = (CREASED && live) ? sharp_at(a, x.y) : (T)0;
+__device__ __forceinline__ QuadParts<T> adj_quad_parts(const AdjArgs<T> &a, int32_t h, const QuadIn<T> &in) {
+    const int4 x = in.x;
+    const bool live = in.live;
+    const V3<T> gv = in.gv, ge0 = in.ge;
+    const T ts = in.ts;
+    // the parameters vparam_of gives nearly every vertex, or the stored ones
+    VParam<T> P{(T)0.0625, (T)-0.0625, 4, -1};
+    if (!in.plain) P = a.VP[x.z];
     const T ps = CREASED ? quad_prev_rec(ts) : (T)0;
     const VW<T> w = vparam_weights<T>(P, ts, ps, x.y, CREASED);
     T c0, c1, cf;
@@ -351,27 +380,264 @@ __device__ __forceinline__ void adj_quad_at(const AdjArgs<T> &a, int32_t h) {
         add_w(ge, w.b, gv);
         add_w(ge, dlN, gvB);
     }
-    if (live && owner) reinterpret_cast<V3<T> *>(a.gEu)[x.y] = ge;
-    // the face: its corners' gamma shares and its edges' face shares, in
-    // halfedge order
+    // the face: its corners' gamma shares and its edges' face shares, summed
+    // over the quad by two exchanges (every lane gets the same bits)
     V3<T> pg{w.g * gv.x, w.g * gv.y, w.g * gv.z}, pe{cf * ge.x, cf * ge.y, cf * ge.z};
-    const V3<T> g0 = quad_bcast_rec<0>(pg), e0 = quad_bcast_rec<0>(pe);
-    const V3<T> g1 = quad_bcast_rec<1>(pg), e1 = quad_bcast_rec<1>(pe);
-    const V3<T> g2 = quad_bcast_rec<2>(pg), e2 = quad_bcast_rec<2>(pe);
-    const V3<T> g3 = quad_bcast_rec<3>(pg), e3 = quad_bcast_rec<3>(pe);
-    if (!live || (h & 3) != 0) return;
-    const V3<T> *gF = reinterpret_cast<const V3<T> *>(a.gF);
-    V3<T> *gFo = reinterpret_cast<V3<T> *>(a.gFu ? a.gFu : a.gF);
-    V3<T> gf = gF[h >> 2];
-    gf.x += g0.x; gf.y += g0.y; gf.z += g0.z;
-    gf.x += e0.x; gf.y += e0.y; gf.z += e0.z;
-    gf.x += g1.x; gf.y += g1.y; gf.z += g1.z;
-    gf.x += e1.x; gf.y += e1.y; gf.z += e1.z;
-    gf.x += g2.x; gf.y += g2.y; gf.z += g2.z;
-    gf.x += e2.x; gf.y += e2.y; gf.z += e2.z;
-    gf.x += g3.x; gf.y += g3.y; gf.z += g3.z;
-    gf.x += e3.x; gf.y += e3.y; gf.z += e3.z;
-    gFo[h >> 2] = gf;
+    V3<T> gf = in.gf;
+    const V3<T> sum = quad_sum(V3<T>{pg.x + pe.x, pg.y + pe.y, pg.z + pe.z});
+    gf.x += sum.x; gf.y += sum.y; gf.z += sum.z;
+    return QuadParts<T>{x, live, owner, gv, ge, gf, w.a, c0, c1};
+}
+
+// pass 2 by itself (cages without a rare-vertex table): the updated edge
+// gradient from the larger halfedge, the updated face gradient from the
+// quad's first lane
+template <typename T, int CREASED>
+__device__ __forceinline__ void adj_quad_at(const AdjArgs<T> &a, int32_t h) {
+    if (a.rare && h == 0) a.rare[0] = 0;   // the vertex pass that follows appends
+    QuadIn<T> in;
+    adj_quad_record<T, false>(a, h, in);
+    adj_quad_gather<T, CREASED, false>(a, h, in);
+    const QuadParts<T> q = adj_quad_parts<T, CREASED>(a, h, in);
+    if (q.live && q.owner) reinterpret_cast<V3<T> *>(a.gEu)[q.x.y] = q.ge;
+    if (!q.live || (h & 3) != 0) return;
+    reinterpret_cast<V3<T> *>(a.gFu ? a.gFu : a.gF)[h >> 2] = q.gf;
+}
+
+// ---- passes 2 and 3 in one, tile by tile ------------------------------------------
+// Passes 2 and 3 apart move 8.3 GB at level 7 of the 64 x 32 torus, 3.2 GB of
+// it the updated edge and face gradients on their way through memory, and
+// 2.15 GB the level's records.  A tile of
+// kAdjTile halfedges is a 16 x 16 patch of quads from level 6 on, and 225
+// of 256 vertices have their whole ring inside it.  So each lane forms its
+// halfedge's share of its vertex's gradient,
+//   c = c0 ge(h) + c1(prev h) ge(prev h) + gf / 4,
+// from registers, leaves it and its vertex-rule weight in LDS, and the
+// smallest halfedge of each ring of four that closes inside the tile adds
+// the ring's shares in ascending halfedge order and writes the vertex.  The
+// other halfedges ("border", an eighth) write their shares out, 16 bytes each,
+// and a bit, and one of each ring a second bit ("mark"), for adj_border and
+// adj_rare to finish.
+// What bounds it is the loads a wave has in flight: with one halfedge per
+// thread it took 1380 us at level 7 whatever was taken away (records derived
+// from the parent level's, 4.3 -> 2.2 GB read; a quarter of the instructions),
+// with two per thread, both records and then both sets of gathers issued
+// together, 968 us.  1024 threads of two 1165 us, 256 of four (128
+// registers) 1204; with tiles of 512 halfedges it takes the same and the
+// border kernel 50 us more.  Level 7 as a whole (this and the border kernel's
+// 247 us against the quad and vertex passes): 2018 -> 1215 us.
+constexpr int kAdjThreads = 512, kAdjPer = 2, kAdjTile = kAdjThreads * kAdjPer;
+
+// Border shares lie packed in each wave's 64 records, in halfedge order (in
+// place, half of every 64-byte segment near a tile's edge would be written
+// and every border vertex would read up to four 128-byte lines for 64
+// bytes): where halfedge h's is.
+__device__ __forceinline__ int32_t wave_rank(uint64_t m) {
+    return (int32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+template <typename T>
+__device__ __forceinline__ int32_t border_slot(const AdjArgs<T> &a, int32_t h) {
+    return (h & ~63) + __popcll(a.border[h >> 6] & ((1ull << (h & 63)) - 1ull));
+}
+
+// sorts r ascending (five exchanges)
+__device__ __forceinline__ void sort4(int32_t (&r)[4]) {
+    const auto order = [&](int i, int j) {
+        const int32_t lo = r[i] < r[j] ? r[i] : r[j], hi = r[i] < r[j] ? r[j] : r[i];
+        r[i] = lo;
+        r[j] = hi;
+    };
+    order(0, 1); order(2, 3); order(0, 2); order(1, 3); order(1, 2);
+}
+
+// a vertex's gradient from its summed weight and shares
+template <typename T>
+__device__ __forceinline__ void adj_vertex_store(const AdjArgs<T> &a, int32_t v, const V3<T> &gv, T alpha,
+                                                 const V3<T> &acc) {
+    *at3(reinterpret_cast<V3<T> *>(a.gP), v) = {alpha * gv.x + acc.x, alpha * gv.y + acc.y, alpha * gv.z + acc.z};
+}
+
+template <typename T, int CREASED, bool DERIVE>
+__device__ __forceinline__ void adj_tile(const AdjArgs<T> &a, int d, uint32_t tile) {
+    __shared__ T sc[4][kAdjTile];      // weight and share of every halfedge of the tile
+    __shared__ int32_t stw[kAdjTile];  // and its twin
+    const int32_t base = (int32_t)(tile * kAdjTile);
+    QuadIn<T> in[kAdjPer];
+#pragma unroll
+    for (int j = 0; j < kAdjPer; ++j) adj_quad_record<T, DERIVE>(a, base + j * kAdjThreads + (int)threadIdx.x, in[j]);
+#pragma unroll
+    for (int j = 0; j < kAdjPer; ++j)
+        adj_quad_gather<T, CREASED, DERIVE>(a, base + j * kAdjThreads + (int)threadIdx.x, in[j]);
+    int32_t rec_r1[kAdjPer];
+#pragma unroll
+    for (int j = 0; j < kAdjPer; ++j) {
+        const int t = j * kAdjThreads + (int)threadIdx.x;
+        const QuadParts<T> q = adj_quad_parts<T, CREASED>(a, base + t, in[j]);
+        const T c1p = quad_prev_rec(q.c1);
+        const V3<T> gep = quad_prev_rec(q.ge);
+        V3<T> c{0, 0, 0};
+        add_w(c, q.c0, q.ge);
+        add_w(c, c1p, gep);
+        add_w(c, (T)0.25, q.gf);
+        sc[0][t] = q.wa;
+        sc[1][t] = c.x;
+        sc[2][t] = c.y;
+        sc[3][t] = c.z;
+        stw[t] = q.live ? q.x.x : -1;
+        rec_r1[j] = quad_rel<kQuadPrev>(q.x.x);   // the ring: x -> twin(prev(x))
+    }
+    __syncthreads();
+    const auto here = [&](int32_t r) { return (uint32_t)(r - base) < (uint32_t)kAdjTile; };
+#pragma unroll
+    for (int j = 0; j < kAdjPer; ++j) {
+        const int t = j * kAdjThreads + (int)threadIdx.x;
+        const int32_t h = base + t;
+        const bool live = in[j].live;
+        const int32_t r1 = rec_r1[j];
+        bool ring = live && here(r1);
+        const int32_t r2 = ring ? stw[qprev(r1) - base] : -1;
+        ring = ring && here(r2);
+        const int32_t r3 = ring ? stw[qprev(r2) - base] : -1;
+        ring = ring && here(r3);
+        const int32_t r4 = ring ? stw[qprev(r3) - base] : -1;
+        ring = ring && r4 == h && r2 != h;   // four distinct halfedges
+        bool mark = false;
+        const uint64_t border = __ballot(live && !ring);
+        if (live && !ring) {
+            reinterpret_cast<W4<T> *>(a.Cs)[(h & ~63) + wave_rank(border)] = W4<T>{sc[0][t], sc[1][t], sc[2][t], sc[3][t]};
+            // one halfedge of the ring finishes the vertex.  Of a face vertex
+            // born at level >= 2 child 2 of its quad's first halfedge, of an
+            // interior edge vertex child 1 of the larger of the two parents p
+            // and w, here from r1 = 4 next(w) + 3 (both shifted by the levels
+            // since); the cage's vertices are left to the cage's maps.
+            const int k2 = 2 * zero_digits(h, d);
+            const int digit = (h >> k2) & 3;
+            const int32_t p = h >> (k2 + 2);
+            if (2 * (d - 1) == k2) mark = digit != 3;
+            else if (digit == 2) mark = (p & 3) == 0;
+            else if (digit == 1) mark = r1 >= 0 && p > qprev(r1 >> (k2 + 2));
+        }
+        const uint64_t m = __ballot(mark);
+        if ((t & 63) == 0 && live) {
+            a.border[h >> 6] = border;
+            a.mark[h >> 6] = m;
+        }
+        if (!ring || h > r1 || h > r2 || h > r3) continue;
+        int32_t r[4] = {h - base, r1 - base, r2 - base, r3 - base};
+        sort4(r);
+        T alpha = sc[0][r[0]];
+        V3<T> acc{sc[1][r[0]], sc[2][r[0]], sc[3][r[0]]};
+#pragma unroll
+        for (int k = 1; k < 4; ++k) {
+            alpha += sc[0][r[k]];
+            acc.x += sc[1][r[k]];
+            acc.y += sc[2][r[k]];
+            acc.z += sc[3][r[k]];
+        }
+        adj_vertex_store(a, in[j].x.z, in[j].gv, alpha, acc);
+    }
+}
+
+// The vertices whose ring of four leaves its tile: wave `wave` takes
+// kAdjBorderWords words of the mark bits (about two are set in each) and
+// finishes one vertex per lane, with the ring from the child numbering.
+constexpr int kAdjBorderWords = 16;
+constexpr int kAdjBorder = 4 * 64 * kAdjBorderWords;   // halfedges per workgroup
+
+template <typename T>
+struct BorderFn {
+    const AdjArgs<T> &a;
+    const DCage &c;
+    const LevelTab &t;
+    const LevelPtrs &lp;
+    int d;
+    __device__ void operator()(int32_t h) const {
+        Fan f;
+        int32_t v, r[4], e[4];
+        if (zero_digits(h, d) == d - 1 && !structural_owner(h, d, c, t, lp.he, nullptr)) return;
+        // other fans are the rare-vertex table's
+        if (!marked_ring_fan(h, d, c, t, lp.he, f, v) || !structural_ring(f, t, d, v, r, e, c)) return;
+        sort4(r);
+        const V3<T> gv = *at3(reinterpret_cast<const V3<T> *>(a.gV), v);
+        W4<T> s[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) s[k] = reinterpret_cast<const W4<T> *>(a.Cs)[border_slot(a, r[k])];
+        T alpha = s[0].a;
+        V3<T> acc{s[0].b, s[0].g, s[0].dl};
+#pragma unroll
+        for (int k = 1; k < 4; ++k) {
+            alpha += s[k].a;
+            acc.x += s[k].b; acc.y += s[k].g; acc.z += s[k].dl;
+        }
+        adj_vertex_store(a, v, gv, alpha, acc);
+    }
+};
+
+template <typename T, class LP>
+__device__ __forceinline__ void adj_border(const AdjArgs<T> &a, const DCage &c, const LevelTab &t, const LP &lp, int d,
+                                           uint32_t block) {
+    __shared__ LevelTab st;
+    __shared__ LevelPtrs slp;
+    __shared__ int32_t list[4][64 * kAdjBorderWords];
+    lds_fill(st, t);
+    lds_fill(slp, lp);
+    __syncthreads();
+    const int32_t wave = (int32_t)(block * 4 + (threadIdx.x >> 6));
+    mask_group<kAdjBorderWords>(a.mark, wave * kAdjBorderWords, (a.H + 63) >> 6, list[threadIdx.x >> 6],
+                                BorderFn<T>{a, c, st, slp, d});
+}
+
+// The vertices of the rare-vertex table, one lane per ring halfedge
+// (cc_rare.h); a closed ring of four inside one tile is done already.
+template <typename T>
+struct AdjRareLds {
+    T p[4][64];
+    int32_t h[64];
+};
+template <typename T>
+__device__ __forceinline__ void adj_rare(const AdjArgs<T> &a, const RareView &r, const LevelTab &t, int d,
+                                         int32_t wave, AdjRareLds<T> &x) {
+    const int lane = (int)(threadIdx.x & 63u);
+    const RareLane L = rare_lane(r, t, d, wave, lane);
+    const bool in = L.live && L.i < L.n;
+    W4<T> s{0, 0, 0, 0};
+    V3<T> gv{0, 0, 0};
+    x.h[lane] = L.h;
+    wave_lds_sync();
+    int rank = 0;
+    bool tile = L.n == 4 && !L.boundary;
+    for (int k = 0; k < L.n; ++k) {
+        const int32_t o = x.h[L.g0 + k];
+        rank += o < L.h ? 1 : 0;
+        tile = tile && o / kAdjTile == L.h / kAdjTile;
+    }
+    if (in && !tile) {
+        s = reinterpret_cast<const W4<T> *>(a.Cs)[border_slot(a, L.h)];
+        gv = reinterpret_cast<const V3<T> *>(a.gV)[L.v];
+        x.p[0][L.g0 + rank] = s.a;
+        x.p[1][L.g0 + rank] = s.b;
+        x.p[2][L.g0 + rank] = s.g;
+        x.p[3][L.g0 + rank] = s.dl;
+    }
+    wave_lds_sync();
+    if (!in || tile || L.i != 0) return;
+    T alpha = x.p[0][L.g0];
+    V3<T> acc{x.p[1][L.g0], x.p[2][L.g0], x.p[3][L.g0]};
+    for (int k = 1; k < L.n; ++k) {
+        alpha += x.p[0][L.g0 + k];
+        acc.x += x.p[1][L.g0 + k]; acc.y += x.p[2][L.g0 + k]; acc.z += x.p[3][L.g0 + k];
+    }
+    adj_vertex_store(a, L.v, gv, alpha, acc);
+}
+
+template <typename T>
+__device__ __forceinline__ void adj_rare_block(const AdjArgs<T> &a, const RareView &r, const LevelTab &t, int d,
+                                               uint32_t block) {
+    __shared__ LevelTab st;
+    __shared__ AdjRareLds<T> x[4];
+    lds_fill(st, t);
+    __syncthreads();
+    adj_rare<T>(a, r, st, d, (int32_t)(block * 4 + (threadIdx.x >> 6)), x[threadIdx.x >> 6]);
 }
 
 // pass 3: vertex v with fan f gathers alpha * gV[v] from the vertex rule
@@ -835,6 +1101,21 @@ __global__ __launch_bounds__(256) void k_adj_quads(AdjArgs<T> a) {
     adj_quad_at<T, CREASED>(a, (int32_t)(xcd_block(blockIdx.x, gridDim.x, 1) * blockDim.x + threadIdx.x));
 }
 
+// (float: 64 registers, so that two workgroups fit a CU)
+template <typename T, int CREASED, bool DERIVE>
+__global__ __launch_bounds__(kAdjThreads, sizeof(T) == 4 ? 8 : 4) void k_adj_tiles(AdjArgs<T> a, int d) {
+    adj_tile<T, CREASED, DERIVE>(a, d, xcd_block(blockIdx.x, gridDim.x, 1));
+}
+
+// after k_adj_tiles: the table's vertices in the first nr workgroups, the
+// other rings that leave their tile in the rest
+template <typename T>
+__global__ __launch_bounds__(256) void k_adj_border(AdjArgs<T> a, DCage c, LevelTab t, LevelPtrs lp, int d, RareView r,
+                                                    uint32_t nr) {
+    if (blockIdx.x < nr) adj_rare_block<T>(a, r, t, d, blockIdx.x);
+    else adj_border<T>(a, c, t, lp, d, xcd_block(blockIdx.x - nr, gridDim.x - nr, 1));
+}
+
 template <typename T, int CREASED, bool RING>
 __global__ __launch_bounds__(256) void k_adj_vertices(AdjArgs<T> a, DCage c, LevelTab t, LevelPtrs lp, int d) {
     owners_block<kAdjScan>(a.H, d, c, t, lp, xcd_block(blockIdx.x, gridDim.x, 1), a.erep,
@@ -973,6 +1254,14 @@ void adjoint_levels(const AdjPlan &pl, const T *gradFinest, T *gradCage, T *bufA
         a.VP = cache ? cache + n.offV[d] : reinterpret_cast<VParam<T> *>(W);
         a.gEu = W + 4 * n.V[d];
         a.gFu = W + 4 * n.V[d] + 3 * n.E[d];
+        a.Cs = W + 4 * n.V[d];   // (in place of gEu and gFu)
+        a.border = pl.border;
+        a.mark = pl.mark;
+        a.plain = cache && pl.vp_plain ? pl.vp_plain + n.offV[d] : nullptr;
+        if (pl.rv.on && d >= 2) {
+            a.par = pl.he + n.offH[d - 1];
+            a.pV = (int32_t)n.V[d - 1]; a.pF = (int32_t)n.F[d - 1]; a.pE = (int32_t)n.E[d - 1];
+        }
         a.erep = pl.erep;
         const dim3 g(grid_for(n.H[d])), gq(grid_for(n.H[d] / 4)), gv(grid_for(n.V[d])), b(256);
         const bool pv = n.V[d] <= pl.per_vertex_max;
@@ -981,25 +1270,28 @@ void adjoint_levels(const AdjPlan &pl, const T *gradFinest, T *gradCage, T *bufA
             a.rare_cap = pl.rare_cap;
         }
         const dim3 gr(grid_for(pl.rare_cap > 0 ? pl.rare_cap : 1));
-        if (creased) {
-            if (!params) {
-            } else if (pv) {
-                hipLaunchKernelGGL((k_adj_per_vertex<T, 1, 0>), gv, b, 0, st, a, pl.cage, pl.tab, pl.lp, d);
-            } else {
-                hipLaunchKernelGGL((k_adj_params<T, 1>), gq, b, 0, st, a, pl.cage, pl.tab, pl.lp, d);
-            }
+        const auto params_pass = [&](auto per_vertex, auto owners) {
+            if (!params) return;
+            if (pv) hipLaunchKernelGGL(per_vertex, gv, b, 0, st, a, pl.cage, pl.tab, pl.lp, d);
+            else hipLaunchKernelGGL(owners, gq, b, 0, st, a, pl.cage, pl.tab, pl.lp, d);
+        };
+        if (creased) params_pass(k_adj_per_vertex<T, 1, 0>, k_adj_params<T, 1>);
+        else params_pass(k_adj_per_vertex<T, 0, 0>, k_adj_params<T, 0>);
+        if (pl.rv.on) {
+            const dim3 tiles((unsigned)((n.H[d] + kAdjTile - 1) / kAdjTile)), tb(kAdjThreads);
+            const auto run = [&](auto kernel) { hipLaunchKernelGGL(kernel, tiles, tb, 0, st, a, d); };
+            if (a.par) run(creased ? k_adj_tiles<T, 1, true> : k_adj_tiles<T, 0, true>);
+            else run(creased ? k_adj_tiles<T, 1, false> : k_adj_tiles<T, 0, false>);
+            const unsigned nr = rare_blocks(pl.rv, d);
+            const dim3 gb(nr + (unsigned)((n.H[d] + kAdjBorder - 1) / kAdjBorder));
+            hipLaunchKernelGGL(k_adj_border<T>, gb, b, 0, st, a, pl.cage, pl.tab, pl.lp, d, pl.rv, nr);
+        } else if (creased) {
             hipLaunchKernelGGL((k_adj_quads<T, 1>), g, b, 0, st, a);
             if (pv) hipLaunchKernelGGL((k_adj_per_vertex<T, 1, 1>), gv, b, 0, st, a, pl.cage, pl.tab, pl.lp, d);
             else if (a.rare) hipLaunchKernelGGL((k_adj_vertices<T, 1, true>), gq, b, 0, st, a, pl.cage, pl.tab, pl.lp, d);
             else hipLaunchKernelGGL((k_adj_vertices<T, 1, false>), gq, b, 0, st, a, pl.cage, pl.tab, pl.lp, d);
             if (a.rare && a.rare_cap > 0) hipLaunchKernelGGL((k_adj_vertices_rare<T, 1>), gr, b, 0, st, a, pl.cage, pl.tab, pl.lp, d);
         } else {
-            if (!params) {
-            } else if (pv) {
-                hipLaunchKernelGGL((k_adj_per_vertex<T, 0, 0>), gv, b, 0, st, a, pl.cage, pl.tab, pl.lp, d);
-            } else {
-                hipLaunchKernelGGL((k_adj_params<T, 0>), gq, b, 0, st, a, pl.cage, pl.tab, pl.lp, d);
-            }
             hipLaunchKernelGGL((k_adj_quads<T, 0>), g, b, 0, st, a);
             if (pv) hipLaunchKernelGGL((k_adj_per_vertex<T, 0, 1>), gv, b, 0, st, a, pl.cage, pl.tab, pl.lp, d);
             else if (a.rare) hipLaunchKernelGGL((k_adj_vertices<T, 0, true>), gq, b, 0, st, a, pl.cage, pl.tab, pl.lp, d);
@@ -1123,6 +1415,41 @@ struct OpAdjCageFaces {
         adj_cage_faces_at<float>(a, c, (int32_t)i);
     }
 };
+// passes 2 and 3 of the jobs with a rare-vertex table, a workgroup per tile
+template <int CREASED, bool DERIVE>
+__global__ __launch_bounds__(kAdjThreads, 8) void k_batch_adj_tiles(const AdjJob *__restrict__ jobs,
+                                                                 const int32_t *__restrict__ start, int n, int d,
+                                                                 char *arena, char *adj) {
+    const uint32_t lb = xcd_block(blockIdx.x, gridDim.x, 1);
+    const int k = find_job(start, n, lb);
+    AdjArgs<float> a;
+    DCage c;
+    const AdjJob &J = jobs[k];
+    unpack_adj(J, arena, adj, a, c);
+    if (DERIVE) {
+        a.par = arena_ptr<const He>(arena, J.lp[d - 1]);
+        a.pV = J.t.V[d - 1]; a.pF = J.t.F[d - 1]; a.pE = J.t.E[d - 1];
+    }
+    adj_tile<float, CREASED, DERIVE>(a, d, lb - (uint32_t)start[k]);
+}
+
+// and the vertices they leave: job k's table's in its first rare_blocks
+// workgroups
+__global__ __launch_bounds__(256) void k_batch_adj_border(const AdjJob *__restrict__ jobs,
+                                                          const int32_t *__restrict__ start, int n, int d, char *arena,
+                                                          char *adj) {
+    const uint32_t lb = xcd_block(blockIdx.x, gridDim.x, 1);
+    const int k = find_job(start, n, lb);
+    const AdjJob &J = jobs[k];
+    AdjArgs<float> a;
+    DCage c;
+    unpack_adj(J, arena, adj, a, c);
+    const uint32_t b = lb - (uint32_t)start[k];
+    const JobLevelPtrs lp{J.lp, arena};
+    if (b < (uint32_t)J.rare_blocks) adj_rare_block<float>(a, arena_rare(arena, J), J.t, d, b);
+    else adj_border<float>(a, c, J.t, lp, d, b - (uint32_t)J.rare_blocks);
+}
+
 // the vertices job k's vertex pass listed, one thread each
 template <int CREASED>
 __global__ __launch_bounds__(256) void k_batch_adj_vertices_rare(const AdjJob *__restrict__ jobs,
@@ -1155,28 +1482,33 @@ struct OpAdjCageGather {
 
 }  // namespace
 
-// level d of every job: vertex parameters, quads (edges and faces) and
-// vertex gathers in turn; `quads` has one workgroup per 1024 halfedges of
-// each job (the owner passes), `halfedges` one per 256
-void batch_adj_level(const BatchTable &quads, const BatchTable &halfedges, const BatchTable &rare, char *arena, char *adj,
-                     int d, int creased, int params, hipStream_t st) {
-    const auto rare_pass = [&](auto kernel) {
-        if (rare.blocks == 0 || rare.n == 0) return;
-        hipLaunchKernelGGL(kernel, dim3(rare.blocks), dim3(256), 0, st, static_cast<const AdjJob *>(rare.jobs),
-                           rare.start, (int)rare.n, d, arena, adj);
+// level d of every job: vertex parameters, then the two tile launches for the
+// jobs with a rare-vertex table and quads, vertices and rare vertices in turn
+// for the others
+void batch_adj_level(const AdjLevelTables &t, char *arena, char *adj, int d, int creased, int params, hipStream_t st) {
+    const auto pass = [&](const BatchTable &b, unsigned threads, auto kernel, auto... args) {
+        if (b.blocks == 0 || b.n == 0) return;
+        hipLaunchKernelGGL(kernel, dim3(b.blocks), dim3(threads), 0, st, static_cast<const AdjJob *>(b.jobs), b.start,
+                           (int)b.n, args...);
     };
     if (creased) {
-        if (params) launch_batch<AdjJob>(quads, OpAdjParams<1>{d, arena, adj}, st);
-        launch_batch<AdjJob>(halfedges, OpAdjQuads<1>{arena, adj}, st);
-        launch_batch<AdjJob>(quads, OpAdjVertices<1>{d, arena, adj}, st);
-        rare_pass(k_batch_adj_vertices_rare<1>);
+        if (params) launch_batch<AdjJob>(t.params, OpAdjParams<1>{d, arena, adj}, st);
+        pass(t.tiles, kAdjThreads, d >= 2 ? k_batch_adj_tiles<1, true> : k_batch_adj_tiles<1, false>, d, arena, adj);
+        launch_batch<AdjJob>(t.halfedges, OpAdjQuads<1>{arena, adj}, st);
+        launch_batch<AdjJob>(t.vertices, OpAdjVertices<1>{d, arena, adj}, st);
+        pass(t.rare, 256, k_batch_adj_vertices_rare<1>, d, arena, adj);
     } else {
-        if (params) launch_batch<AdjJob>(quads, OpAdjParams<0>{d, arena, adj}, st);
-        launch_batch<AdjJob>(halfedges, OpAdjQuads<0>{arena, adj}, st);
-        launch_batch<AdjJob>(quads, OpAdjVertices<0>{d, arena, adj}, st);
-        rare_pass(k_batch_adj_vertices_rare<0>);
+        if (params) launch_batch<AdjJob>(t.params, OpAdjParams<0>{d, arena, adj}, st);
+        pass(t.tiles, kAdjThreads, d >= 2 ? k_batch_adj_tiles<0, true> : k_batch_adj_tiles<0, false>, d, arena, adj);
+        launch_batch<AdjJob>(t.halfedges, OpAdjQuads<0>{arena, adj}, st);
+        launch_batch<AdjJob>(t.vertices, OpAdjVertices<0>{d, arena, adj}, st);
+        pass(t.rare, 256, k_batch_adj_vertices_rare<0>, d, arena, adj);
     }
+    pass(t.border, 256, k_batch_adj_border, d, arena, adj);
 }
+
+int64_t adj_tile_blocks(int64_t H) { return (H + kAdjTile - 1) / kAdjTile; }
+int64_t adj_border_blocks(int64_t H) { return (H + kAdjBorder - 1) / kAdjBorder; }
 
 void batch_adj_cage_gather(const BatchTable &halfedges, const BatchTable &edges, const BatchTable &faces,
                            const BatchTable &vertices, char *arena, char *adj, int creased, hipStream_t st) {

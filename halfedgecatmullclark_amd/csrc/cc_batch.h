@@ -63,10 +63,16 @@ struct SpanJob {
 struct AdjJob {
     int64_t he, cr, gV, gF, gE, gP, W, erep;
     int64_t vp;   // the level's vertex-rule parameters (kept across calls), or -1: in W
+    int64_t plain;   // and their bytes (AdjArgs::plain), or -1
     int64_t gFu;  // the face gradients after the quad pass, or -1: in place (gF)
     int64_t rare; // the vertex pass's rare-vertex list (arena offset), or -1
     int32_t rare_cap;
     int32_t gin;
+    // the rare-vertex table as in LevelJob (rare_blocks: in front of the
+    // job's workgroups of the border launch), the border bits and, in the
+    // adjoint arena, the mark bits
+    int64_t rv_item, rv_ent, rv_bnd, border, mark;
+    int32_t rv_n4, rv_n8, rv_n64, rv_nb, rare_blocks;
     int64_t c_he, c_v2h, c_e2h, c_f2h, c_pts, c_uvs, c_cr, c_vro, c_vr, c_vb, c_fro, c_fr, c_voo, c_vo;
     int64_t lp[kMaxDepth + 1];
     int32_t H, C, V;
@@ -147,7 +153,10 @@ __host__ __device__ __forceinline__ void unpack_adj(const AdjJob &J, char *arena
     a.gP = arena_ptr<float>(adj, J.gP);
     a.W = arena_ptr<float>(adj, J.W);
     a.VP = J.vp >= 0 ? arena_ptr<VParam<float>>(adj, J.vp) : reinterpret_cast<VParam<float> *>(a.W);
-    a.gEu = a.W ? a.W + 4 * (int64_t)J.V : nullptr;
+    a.plain = arena_ptr<uint8_t>(adj, J.plain);
+    a.gEu = a.Cs = a.W ? a.W + 4 * (int64_t)J.V : nullptr;
+    a.border = arena_ptr<uint64_t>(arena, J.border);
+    a.mark = arena_ptr<uint64_t>(adj, J.mark);
     a.erep = arena_ptr<const uint64_t>(arena, J.erep);
     a.rare = arena_ptr<int32_t>(arena, J.rare);
     a.rare_cap = J.rare_cap;
@@ -215,12 +224,19 @@ void batch_level_vertices_rare(const BatchTable &t, char *arena, int d, int gath
 
 // adjoint launches (cc_adjoint.hip)
 // one level's adjoint: vertex parameters (when `params`; else the ones a
-// previous call left) and vertex gathers over `quads` (the owner passes scan
-// 4 halfedges per thread), the quad pass one thread per halfedge over
-// `halfedges`
-void batch_adj_level(const BatchTable &quads, const BatchTable &halfedges, const BatchTable &rare, char *arena, char *adj,
-                     int d, int creased,
-                     int params, hipStream_t st);
+// previous call left) over `params` (the owner passes scan 4 halfedges per
+// thread); jobs with a rare-vertex table: a workgroup per tile over `tiles`,
+// then the vertices left over `border`; the others: the quad pass one thread
+// per halfedge over `halfedges`, the vertex gathers over `vertices` and their
+// rare lists over `rare`
+struct AdjLevelTables {
+    BatchTable params, tiles, border, halfedges, vertices, rare;
+};
+void batch_adj_level(const AdjLevelTables &t, char *arena, char *adj, int d, int creased, int params, hipStream_t st);
+// workgroups a level of H halfedges takes in the two tile launches (the
+// table's vertices apart)
+int64_t adj_tile_blocks(int64_t H);
+int64_t adj_border_blocks(int64_t H);
 void batch_adj_cage(const BatchTable &t, char *arena, char *adj, int creased, hipStream_t st);
 // the cage step as ordered gathers (every cage has its ring lists): one
 // thread per cage halfedge, edge, face and vertex in turn

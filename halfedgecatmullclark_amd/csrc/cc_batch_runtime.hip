@@ -78,16 +78,18 @@ struct ccb_Batch {
     // adjoint calls (a batch's topology and creases never change); valid for
     // the creased (1) or uncreased (0) rules, -1 before the first call
     VParam<float> *adjVP = nullptr;
+    uint8_t *adjPlain = nullptr;   // AdjArgs::plain beside them
+    uint64_t *adjMark = nullptr;   // the tile pass's mark bits, laid out as defer_mask
     int adj_vp_key = -1;
     void *tables = nullptr;
     size_t tables_cap = 0;
     // launch tables
     BatchTable t_cage_he, t_cage_f, t_cage_e, t_cage_v, t_cage_h3, t_cage_zero, t_fin;
-    BatchTable t_cr[kMaxDepth + 1], t_patch[kMaxDepth + 1], t_def[kMaxDepth + 1], t_adj[kMaxDepth + 1];
+    BatchTable t_cr[kMaxDepth + 1], t_patch[kMaxDepth + 1], t_def[kMaxDepth + 1];
     BatchTable t_rare[kMaxDepth + 1];   // rare-vertex lists after the scan-0 vertex kernel
-    BatchTable t_fused[kMaxDepth + 1], t_vert[kMaxDepth + 1], t_adjq[kMaxDepth + 1];
-    BatchTable t_adjr[kMaxDepth + 1];   // the adjoint vertex pass's rare-vertex lists
-    BatchTable t_adjc_e, t_adjc_f, t_adjc_v;   // cage-step adjoint gathers: per edge, face, vertex
+    BatchTable t_fused[kMaxDepth + 1], t_vert[kMaxDepth + 1];
+    AdjLevelTables t_adj[kMaxDepth + 1];   // levels 1 ..
+    BatchTable t_adjc_h, t_adjc_e, t_adjc_f, t_adjc_v;   // cage-step adjoint gathers: per edge, face, vertex
     bool all_rings = true;                     // every cage has its ring lists
     // the adjoint's finest steps read the caller's gradient (its address in
     // the adjoint arena's first bytes); false when a cage is refined once:
@@ -212,6 +214,8 @@ DCage ccb_Batch::cage_view(int i) const {
 bool ccb_Batch::create(const cc_Mesh *const *meshes, const int32_t *depths, int32_t count) {
     N = count;
     cages.resize(count);
+    CageRings r;    // reused from cage to cage
+    RareTable rt;
     for (int i = 0; i < count; ++i) {
         const cc_Mesh *m = meshes[i];
         Cage &g = cages[i];
@@ -224,7 +228,7 @@ bool ccb_Batch::create(const cc_Mesh *const *meshes, const int32_t *depths, int3
         g.o_u0 = tot_u0; tot_u0 += g.U0;
         g.o_e0 = tot_e0; tot_e0 += g.E0;
         g.o_f0 = tot_f0; tot_f0 += g.F0;
-        const CageRings r = build_cage_rings(m);
+        build_cage_rings(m, r);
         all_rings = all_rings && r.ok;
         if (r.ok) {
             auto put = [&](const std::vector<int32_t> &v) {
@@ -240,7 +244,7 @@ bool ccb_Batch::create(const cc_Mesh *const *meshes, const int32_t *depths, int3
             g.o_fr = put(r.fring);
             g.o_voo = put(r.ooff);
             g.o_vo = put(r.out);
-            const RareTable rt = build_rare_table(m, r);
+            build_rare_table(m, r, rt);
             if (rt.ok) {   // records of two and four ints, read whole
                 auto put16 = [&](const std::vector<int32_t> &v) {
                     rings_host.resize((rings_host.size() + 3) & ~size_t(3), 0);
@@ -258,7 +262,7 @@ bool ccb_Batch::create(const cc_Mesh *const *meshes, const int32_t *depths, int3
         g.o_pts = tot_pts; tot_pts += g.n.cumV(g.D);
         g.o_fin = tot_fin; tot_fin += g.n.V[g.D];
         g.o_def = tot_def; tot_def += g.D >= 2 ? (g.n.H[g.D - 1] + 63) / 64 : 1;
-        {
+        if (!g.rv.on) {
             int64_t b0 = 0;
             const CageHe *ch = reinterpret_cast<const CageHe *>(m->halfedges);
             for (int32_t h = 0; h < g.H0; ++h) b0 += ch[h].twin < 0 ? 1 : 0;
@@ -271,7 +275,7 @@ bool ccb_Batch::create(const cc_Mesh *const *meshes, const int32_t *depths, int3
             tot_erep += g.tab.R[g.D - 1];
         }
         g.o_adjB = tot_adjB; tot_adjB += g.n.V[g.D - 1];
-        g.o_adjW = tot_adjW; tot_adjW += adj_scratch_scalars(g.n, g.D, true);
+        g.o_adjW = tot_adjW; tot_adjW += adj_scratch_scalars(g.n, g.D, g.rv.on);
         if (g.D == 1) gin_ok = false;
         g.o_adjVP = tot_adjVP; tot_adjVP += g.n.cumV(g.D - 1);
         Dmax = std::max(Dmax, g.D);
@@ -292,7 +296,7 @@ bool ccb_Batch::create(const cc_Mesh *const *meshes, const int32_t *depths, int3
         const size_t o_cr = cv.take(sizeof(Crease) * (size_t)tot_cr);
         const size_t o_pts = cv.take(sizeof(P3) * (size_t)tot_pts);
         const size_t o_def = cv.take(sizeof(uint64_t) * (size_t)tot_def);
-        const size_t o_rare = cv.take(sizeof(int32_t) * (size_t)tot_rare);
+        const size_t o_rare = cv.take(sizeof(int32_t) * (size_t)(tot_rare + 1));
         const size_t o_erep = cv.take(sizeof(uint64_t) * (size_t)(tot_erep + 1));
         CC_TRY(hipMalloc(&arena, cv.size), "hipMalloc(batch arena)");
         c_he = reinterpret_cast<CageHe *>(arena + o_che);
@@ -357,7 +361,11 @@ bool ccb_Batch::alloc_adjoint() {
     const size_t oW = cv.take(sizeof(float) * (size_t)tot_adjW);
     const size_t oC = cv.take(sizeof(float) * 3 * (size_t)tot_v0);
     const size_t oP = cv.take(sizeof(VParam<float>) * (size_t)tot_adjVP);
+    const size_t oL = cv.take((size_t)tot_adjVP);
+    const size_t oM = cv.take(sizeof(uint64_t) * (size_t)tot_def);
     CC_TRY(hipMalloc(&adj_arena, cv.size), "hipMalloc(batch adjoint arena)");
+    adjMark = reinterpret_cast<uint64_t *>(adj_arena + oM);
+    adjPlain = reinterpret_cast<uint8_t *>(adj_arena + oL);
     adjVP = reinterpret_cast<VParam<float> *>(adj_arena + oP);
     adjA = reinterpret_cast<float *>(adj_arena + oA);
     adjB = reinterpret_cast<float *>(adj_arena + oB);
@@ -501,7 +509,7 @@ bool ccb_Batch::build_tables() {
             // has written them
             const bool kept = d >= 2 && d - 1 <= erep_kept;
             std::vector<AdjJob> jobs;
-            std::vector<int64_t> b, bq, br, be, bf, bv;
+            std::vector<int64_t> b, bp, bt, bb, bh, bq, br, be, bf, bv;
             for (int i = 0; i < N; ++i) {
                 const Cage &g = cages[i];
                 if (g.D <= d) continue;
@@ -528,6 +536,7 @@ bool ccb_Batch::build_tables() {
                 }
                 j.W = aoff(adjW + g.o_adjW);
                 j.vp = d >= 1 ? aoff(adjVP + g.o_adjVP + g.n.offV[d]) : -1;
+                j.plain = d >= 1 ? aoff(adjPlain + g.o_adjVP + g.n.offV[d]) : -1;
                 j.erep = g.o_erep >= 0 && kept ? off(erep + g.o_erep) : -1;
                 j.gin = gin_ok && d == g.D - 1 ? 1 : 0;
                 if (j.gin) {   // byte offsets into the caller's gradient
@@ -542,23 +551,41 @@ bool ccb_Batch::build_tables() {
                 }
                 j.gFu = d >= 1 ? aoff(adjW + g.o_adjW + 4 * g.n.V[d] + 3 * g.n.E[d]) : -1;
                 // the forward's rare-vertex list, free between passes
-                j.rare = d >= 1 ? off(rare + g.o_rare) : -1;
-                j.rare_cap = d >= 1 ? g.rare_cap : 0;
+                const bool listed = d >= 1 && !g.rv.on, tiled = d >= 1 && g.rv.on;
+                j.rare = listed ? off(rare + g.o_rare) : -1;
+                j.rare_cap = listed ? g.rare_cap : 0;
+                j.rv_item = tiled ? off(rings + g.o_ritem) : -1;
+                j.rv_ent = tiled ? off(rings + g.o_rent) : -1;
+                j.rv_bnd = tiled ? off(rings + g.o_rbnd) : -1;
+                j.rv_n4 = g.rv.n4; j.rv_n8 = g.rv.n8; j.rv_n64 = g.rv.n64; j.rv_nb = g.rv.nb;
+                j.rare_blocks = tiled ? (int32_t)blocks_of(rare_waves(g.rv, d), 4) : 0;
+                j.border = off(defer_mask + g.o_def);   // the forward's bits, free between passes
+                j.mark = aoff(adjMark + g.o_def);
                 cage_offsets(i, j);
                 j.t = g.tab;
                 for (int k = 0; k <= kMaxDepth; ++k) j.lp[k] = (k >= 1 && k <= g.D) ? off(hb + g.n.offH[k]) : -1;
                 jobs.push_back(j);
                 b.push_back(blocks_of(j.H));
-                bq.push_back(blocks_of(j.H, 1024));
+                bp.push_back(blocks_of(j.H, 1024));
+                bt.push_back(tiled ? adj_tile_blocks(j.H) : 0);
+                bb.push_back(tiled ? j.rare_blocks + adj_border_blocks(j.H) : 0);
+                bh.push_back(listed ? blocks_of(j.H) : 0);
+                bq.push_back(listed ? blocks_of(j.H, 1024) : 0);
                 br.push_back(j.rare_cap > 0 ? blocks_of(j.rare_cap) : 0);
                 be.push_back(blocks_of(g.E0));
                 bf.push_back(blocks_of(g.F0));
                 bv.push_back(blocks_of(g.V0));
             }
-            tb.add(t_adj[d], jobs, b);
-            tb.add(t_adjq[d], jobs, bq);
-            tb.add(t_adjr[d], jobs, br);
-            if (d == 0) {
+            if (d >= 1) {
+                AdjLevelTables &t = t_adj[d];
+                tb.add(t.params, jobs, bp);
+                tb.add(t.tiles, jobs, bt);
+                tb.add(t.border, jobs, bb);
+                tb.add(t.halfedges, jobs, bh);
+                tb.add(t.vertices, jobs, bq);
+                tb.add(t.rare, jobs, br);
+            } else {
+                tb.add(t_adjc_h, jobs, b);
                 tb.add(t_adjc_e, jobs, be);
                 tb.add(t_adjc_f, jobs, bf);
                 tb.add(t_adjc_v, jobs, bv);
@@ -645,13 +672,13 @@ void ccb_Batch::record_adjoint(int flags, hipStream_t st) {
     hipLaunchKernelGGL(k_zero, dim3((unsigned)std::min<int64_t>((nc + 255) / 256, 65536)), dim3(256), 0, st, adjCage, nc);
     for (int d = Dmax - 1; d >= 1; --d)
         timed_launch("adj_level", d, st,
-                     [&] { batch_adj_level(t_adjq[d], t_adj[d], t_adjr[d], arena, adj_arena, d, creased, params, st); });
+                     [&] { batch_adj_level(t_adj[d], arena, adj_arena, d, creased, params, st); });
     if (all_rings)
         timed_launch("adj_cage", 0, st, [&] {
-            batch_adj_cage_gather(t_adj[0], t_adjc_e, t_adjc_f, t_adjc_v, arena, adj_arena, creased, st);
+            batch_adj_cage_gather(t_adjc_h, t_adjc_e, t_adjc_f, t_adjc_v, arena, adj_arena, creased, st);
         });
     else
-        timed_launch("adj_cage", 0, st, [&] { batch_adj_cage(t_adj[0], arena, adj_arena, creased, st); });
+        timed_launch("adj_cage", 0, st, [&] { batch_adj_cage(t_adjc_h, arena, adj_arena, creased, st); });
 }
 
 bool ccb_Batch::run(int32_t key, bool adjoint, int32_t steps, hipStream_t st) {

@@ -39,11 +39,18 @@ bool ref_counts_fit_int32(const cc_Mesh *cage, int32_t D, const char **why);
 // 4 H + V entries (a cage whose walks do not close): the kernels then walk.
 struct CageRings {
     std::vector<int32_t> voff, vring, vbnd, foff, fring, ooff, out;
+    std::vector<int32_t> fill;   // scratch
     bool ok = false;
+    // every listed halfedge leaves its ring's vertex and lies on its ring's face
+    bool own = true;
 };
 
-inline CageRings build_cage_rings(const cc_Mesh *m) {
-    CageRings r;
+// (into r, whose storage a caller with many cages reuses)
+inline void build_cage_rings(const cc_Mesh *m, CageRings &r) {
+    r.ok = false;
+    r.own = true;
+    r.vring.clear();
+    r.fring.clear();
     const int32_t V = m->vertexCount, F = m->faceCount, H = m->halfedgeCount;
     const CageHe *he = reinterpret_cast<const CageHe *>(m->halfedges);
     const size_t cap = 4 * (size_t)H + (size_t)V;
@@ -58,11 +65,13 @@ inline CageRings build_cage_rings(const cc_Mesh *m) {
         const int32_t p = m->vertexToHalfedgeIDs[v];
         if (!valid(p)) continue;
         r.vring.push_back(p);
+        r.own = r.own && he[p].vert == v;
         int32_t n = 1;
         int32_t g = valid(he[p].prev) ? he[he[p].prev].twin : -1;
         for (; g >= 0 && g != p && n < kWalkCap; ++n) {
-            if (!valid(g) || r.vring.size() >= cap) return r;
+            if (!valid(g) || r.vring.size() >= cap) return;
             r.vring.push_back(g);
+            r.own = r.own && he[g].vert == v;
             g = valid(he[g].prev) ? he[he[g].prev].twin : -1;
         }
         r.vbnd[v] = g < 0 ? 1 : 0;
@@ -73,10 +82,12 @@ inline CageRings build_cage_rings(const cc_Mesh *m) {
         const int32_t p = m->faceToHalfedgeIDs[f];
         if (!valid(p)) continue;
         r.fring.push_back(p);
+        r.own = r.own && he[p].face == f;
         int32_t n = 1;
         for (int32_t it = he[p].next; it != p && n < kWalkCap; it = he[it].next, ++n) {
-            if (!valid(it) || r.fring.size() >= cap) return r;
+            if (!valid(it) || r.fring.size() >= cap) return;
             r.fring.push_back(it);
+            r.own = r.own && he[it].face == f;
         }
     }
     r.foff[F] = (int32_t)r.fring.size();
@@ -84,64 +95,76 @@ inline CageRings build_cage_rings(const cc_Mesh *m) {
     r.ooff.assign((size_t)V + 1, 0);
     for (int32_t h = 0; h < H; ++h) {
         const int32_t v = he[h].vert;
-        if (v < 0 || v >= V) return r;
+        if (v < 0 || v >= V) return;
         ++r.ooff[(size_t)v + 1];
     }
     for (int32_t v = 0; v < V; ++v) r.ooff[(size_t)v + 1] += r.ooff[v];
     r.out.assign((size_t)H, 0);
-    std::vector<int32_t> fill(r.ooff.begin(), r.ooff.end() - 1);
-    for (int32_t h = 0; h < H; ++h) r.out[(size_t)fill[he[h].vert]++] = h;
+    r.fill.assign(r.ooff.begin(), r.ooff.end() - 1);
+    for (int32_t h = 0; h < H; ++h) r.out[(size_t)r.fill[he[h].vert]++] = h;
     r.ok = true;
-    return r;
 }
 
 // The rare-vertex table of a cage (RareView) as one run of int32s: items |
 // entries | boundary halfedges, item and boundary records of four ints,
 // entries of two.  `ok` is false when the cage does not fit it (walks that do
-// not close, links that contradict each other, a fan of more than 64
-// entries): its rare vertices then go through the rare list.
+// not close, links that contradict each other, a vertex, edge or face with
+// halfedges outside its one ring, a fan of more than 64 entries): its rare
+// vertices then go through the rare list.
 struct RareTable {
     std::vector<int32_t> item, ent, bnd;
     int32_t n4 = 0, n8 = 0, n64 = 0, nb = 0;
     bool ok = false;
     bool empty() const { return n4 + n8 + n64 + nb == 0; }
+    struct Item { int32_t v, first, n, boundary; };
+    std::vector<Item> items[3];   // scratch
+    std::vector<char> seen;
 };
 
-inline RareTable build_rare_table(const cc_Mesh *m, const CageRings &r) {
-    RareTable t;
-    if (!r.ok) return t;
+inline void build_rare_table(const cc_Mesh *m, const CageRings &r, RareTable &t) {
+    t.ok = false;
+    t.n4 = t.n8 = t.n64 = t.nb = 0;
+    for (std::vector<int32_t> *x : {&t.item, &t.ent, &t.bnd}) x->clear();
+    for (auto &x : t.items) x.clear();
     const int32_t V = m->vertexCount, F = m->faceCount, H = m->halfedgeCount, E = m->edgeCount;
+    if (!r.ok || !r.own || (int64_t)r.vring.size() != H || (int64_t)r.fring.size() != H) return;
     const CageHe *he = reinterpret_cast<const CageHe *>(m->halfedges);
     auto valid = [&](int32_t h) { return h >= 0 && h < H; };
+    t.seen.assign((size_t)E, 0);
+    int32_t pairs = 0;
     for (int32_t h = 0; h < H; ++h) {
         const CageHe &x = he[h];
         if (!valid(x.next) || !valid(x.prev) || x.prev == h || x.next == h || he[x.next].prev != h ||
             x.twin >= H || x.edge < 0 || x.edge >= E || x.face < 0 || x.face >= F)
-            return t;
-        if (x.twin >= 0 && (he[x.twin].twin != h || he[x.twin].edge != x.edge)) return t;
+            return;
+        if (x.twin >= 0 && (he[x.twin].twin != h || he[x.twin].edge != x.edge)) return;
+        if (h > x.twin) {   // one pair of halfedges, or one boundary halfedge, per edge
+            if (t.seen[x.edge]) return;
+            t.seen[x.edge] = 1;
+            ++pairs;
+            if (x.twin < 0) t.bnd.insert(t.bnd.end(), {h, x.next, x.edge, 0});
+        }
     }
-    struct Item { int32_t v, first, n, boundary; };
-    std::vector<Item> items[3];
+    if (pairs != E) return;
     auto add_item = [&](int32_t v, int32_t n, int32_t boundary, size_t first) {
         const int32_t entries = n + boundary;
         const int k = entries <= 4 ? 0 : (entries <= 8 ? 1 : 2);
-        items[k].push_back({v, (int32_t)(first / 2), n, boundary});
+        t.items[k].push_back({v, (int32_t)(first / 2), n, boundary});
         return entries <= 64;
     };
-    t.ent.resize(2 * (r.vring.size() + r.fring.size() + (size_t)V));
-    size_t used = 0;
     auto add_ent = [&](int32_t h, int32_t e, bool odd) {
-        t.ent[used++] = h;
-        t.ent[used++] = odd ? (int32_t)((uint32_t)e | 0x80000000u) : e;
+        t.ent.push_back(h);
+        t.ent.push_back(odd ? (int32_t)((uint32_t)e | 0x80000000u) : e);
     };
     for (int32_t v = 0; v < V; ++v) {
         const int32_t o = r.voff[v], n = r.voff[v + 1] - o;
-        if (n == 0 || he[r.vring[o]].vert != v) continue;   // no halfedge represents v
+        if (n != r.ooff[v + 1] - r.ooff[v]) return;
+        if (n == 0) continue;   // no halfedge leaves v
         const bool boundary = r.vbnd[v] != 0;
         // A closed ring of four: marked_ring_fan and structural_ring take it
         // (every entry has a twin w, and next(w) is the entry before it).
         if (n == 4 && !boundary) continue;
-        const size_t first = used;
+        const size_t first = t.ent.size();
         for (int32_t i = 0; i < n; ++i) {   // the ring's previous edge is the next entry's edge
             const int32_t R = r.vring[o + i], w = he[R].twin;
             const int32_t tw = w >= 0 ? 4 * he[w].next + 3 : -1;
@@ -151,35 +174,31 @@ inline RareTable build_rare_table(const cc_Mesh *m, const CageRings &r) {
             const int32_t R = r.vring[o + n - 1], p = he[R].prev;
             add_ent(4 * R, 2 * he[p].edge + 1, true);
         }
-        if (!add_item(v, n, boundary ? 1 : 0, first)) return t;
+        if (!add_item(v, n, boundary ? 1 : 0, first)) return;
     }
     for (int32_t f = 0; f < F; ++f) {
         const int32_t o = r.foff[f], n = r.foff[f + 1] - o;
-        if (n == 0 || he[r.fring[o]].face != f) continue;
+        if (n == 0) continue;
         const int32_t p = r.fring[o];
         if (p + 3 < H && he[p].next == p + 1 && he[p + 1].next == p + 2 && he[p + 2].next == p + 3 &&
             he[p + 3].next == p)
             continue;
-        const size_t first = used;
+        const size_t first = t.ent.size();
         for (int32_t i = 0; i < n; ++i) {
             const int32_t q = r.fring[o + i], pr = he[q].prev;
             add_ent(4 * q + 2, 2 * E + pr, 4 * q + 2 < 4 * pr + 1);
         }
-        if (!add_item(V + f, n, 0, first)) return t;
+        if (!add_item(V + f, n, 0, first)) return;
     }
-    t.ent.resize(used);
-    for (const auto &group : items) {
+    for (const auto &group : t.items) {
         const int32_t *p = reinterpret_cast<const int32_t *>(group.data());
         t.item.insert(t.item.end(), p, p + 4 * group.size());
     }
-    t.n4 = (int32_t)items[0].size();
-    t.n8 = (int32_t)items[1].size();
-    t.n64 = (int32_t)items[2].size();
-    for (int32_t h = 0; h < H; ++h)
-        if (he[h].twin < 0) t.bnd.insert(t.bnd.end(), {h, he[h].next, he[h].edge, 0});
+    t.n4 = (int32_t)t.items[0].size();
+    t.n8 = (int32_t)t.items[1].size();
+    t.n64 = (int32_t)t.items[2].size();
     t.nb = (int32_t)(t.bnd.size() / 4);
     t.ok = true;
-    return t;
 }
 
 // host-memory view of a cage with the device-view type (for the O(depth) maps)

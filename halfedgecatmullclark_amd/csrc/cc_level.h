@@ -370,31 +370,6 @@ __device__ __forceinline__ void level_vertices_compact_block(const FusedArgs &a,
 // halfedges, about a quarter of which represent a vertex.
 constexpr int kOwnerWords = 4;
 
-// Calls fn(h) once per bit set in mask words [w0, w0 + GW) of `words`, one
-// halfedge per lane in ascending order, in rounds of 64.  The wave lists the
-// marked halfedges in `list` (its own 64 GW slots of LDS): lane l of word w
-// writes w * 64 + l at the count of set bits before it (mbcnt).
-template <int GW, class Fn>
-__device__ __forceinline__ void mask_group(const uint64_t *mask, int32_t w0, int32_t words, int32_t *list,
-                                           const Fn &fn) {
-    const int lane = (int)(threadIdx.x & 63u);
-    int32_t total = 0;
-#pragma unroll
-    for (int j = 0; j < GW; ++j) {
-        const int32_t w = w0 + j;
-        const uint64_t m = w < words ? mask[w] : 0ull;   // the same word in every lane
-        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)m);
-        const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(m >> 32));
-        const uint32_t rank = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
-        if (((lane < 32 ? lo >> lane : hi >> (lane - 32)) & 1u) != 0u) list[total + (int32_t)rank] = w * 64 + lane;
-        total += __popc(lo) + __popc(hi);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    for (int32_t i = lane; i < total; i += 64) fn(list[i]);
-}
-
 // A marked owner whose ring follows from the child numbering: its vertex
 // point; any other goes to the rare list when there is one, else its waves
 // of rare_vertices have it (no general fan code here, so the kernel keeps

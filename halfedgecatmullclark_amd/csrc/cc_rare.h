@@ -31,12 +31,6 @@ struct RareLds {
     int32_t e[64], h[64];
 };
 
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // One lane's place in the table: entry i of a fan of n halfedges with m edge
 // entries (n, or n + 1 on a boundary: the last one is the edge of
 // prev(last halfedge)); h and e its halfedge and edge at the level.

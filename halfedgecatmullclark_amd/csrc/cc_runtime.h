@@ -74,6 +74,8 @@ struct ccd_Subd {
     uint64_t *erep = nullptr;
     bool erep_valid[cch::kMaxDepth + 1] = {};
     size_t adj_scalar = 0;
+    uint64_t *adj_mark = nullptr;   // AdjArgs::mark
+    bool adj_tiles = false;   // adj_w is sized for the adjoint's tile pass (rare_on)
     // halfedge normals (allocated on first use, H_D points each): the corner
     // normals the vertex normals sum, and the host entry points' output
     cch::P3 *nrm_tmp = nullptr, *nrm_out = nullptr;

@@ -105,7 +105,7 @@ bool ccd_Subd::alloc(const cc_Mesh *cage, int32_t depth) {
 void ccd_Subd::free_all() {
     DeviceGuard g(device);
     void *ptrs[] = {c_he, c_v2h, c_e2h, c_f2h, c_pts, c_uvs, c_cr, he, cr, pts, adj_a, adj_b, adj_w, adj_in, adj_out, adj_sharp,
-                    adj_vp, defer_mask, own_masks, rings, rare, erep, nrm_tmp, nrm_out};
+                    adj_vp, adj_mark, defer_mask, own_masks, rings, rare, erep, nrm_tmp, nrm_out};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     for (auto &t : timed) {
@@ -139,7 +139,17 @@ bool ccd_Subd::upload_cage(const cc_Mesh *cage, hipStream_t st) {
     CC_TRY(hipMemcpyAsync(c_pts, cage->vertexPoints, sizeof(P3) * (size_t)V0, hipMemcpyHostToDevice, st), "upload cage");
     if (U0 > 0) CC_TRY(hipMemcpyAsync(c_uvs, cage->uvs, sizeof(UV) * (size_t)U0, hipMemcpyHostToDevice, st), "upload cage");
     CC_TRY(hipMemcpyAsync(c_cr, cage->creases, sizeof(Crease) * (size_t)E0, hipMemcpyHostToDevice, st), "upload cage");
-    {   // the rare-vertex list: cage vertices, cage faces and boundary vertices
+    // ring lists: [vertex offsets | vertex boundary flags | face offsets |
+    // vertex rings | face rings], each list padded by one entry
+    CageRings r;
+    build_cage_rings(cage, r);
+    rings_ok = r.ok;
+    RareTable rt;
+    build_rare_table(cage, r, rt);
+    rare_free = rt.ok && rt.empty();
+    rare_on = rt.ok;
+    rare_n4 = rt.n4; rare_n8 = rt.n8; rare_n64 = rt.n64; rare_nb = rt.nb;
+    if (!rt.ok) {   // the rare-vertex list: cage vertices, cage faces and boundary vertices
         int64_t b0 = 0;
         const CageHe *ch = reinterpret_cast<const CageHe *>(cage->halfedges);
         for (int32_t h = 0; h < H0; ++h) b0 += ch[h].twin < 0 ? 1 : 0;
@@ -152,14 +162,6 @@ bool ccd_Subd::upload_cage(const cc_Mesh *cage, hipStream_t st) {
             rare_cap = (int32_t)cap;
         }
     }
-    // ring lists: [vertex offsets | vertex boundary flags | face offsets |
-    // vertex rings | face rings], each list padded by one entry
-    const CageRings r = build_cage_rings(cage);
-    rings_ok = r.ok;
-    const RareTable rt = build_rare_table(cage, r);
-    rare_free = rt.ok && rt.empty();
-    rare_on = rt.ok;
-    rare_n4 = rt.n4; rare_n8 = rt.n8; rare_n64 = rt.n64; rare_nb = rt.nb;
     if (!r.ok) return true;
     std::vector<int32_t> rings_host;
     auto put = [&](const std::vector<int32_t> &v) {
@@ -503,18 +505,24 @@ bool ccd_Subd::refine_graph(int32_t steps, hipStream_t st) {
 // Adjoint of the point refinement for the current topology and creases.
 bool ccd_Subd::adjoint(const void *gradFinest, void *gradCage, int32_t steps, hipStream_t st) {
     const size_t scalar = (steps & CCD_FP64) ? sizeof(double) : sizeof(float);
-    if (adj_scalar != scalar) {
+    if (adj_scalar != scalar || adj_tiles != rare_on) {
         if (adj_a) (void)hipFree(adj_a);
         if (adj_b) (void)hipFree(adj_b);
         if (adj_w) (void)hipFree(adj_w);
+        if (adj_mark) (void)hipFree(adj_mark);
         adj_a = adj_b = adj_w = nullptr;
+        adj_mark = nullptr;
         adj_scalar = 0;
         // level gradients: D-1 in adj_b, then D-2, D-3, ... alternating with
         // adj_a (a cage refined once copies the finest gradient to adj_a)
         CC_TRY(hipMalloc(&adj_a, 3 * scalar * (size_t)(D >= 2 ? n.V[D - 2] : n.V[D])), "hipMalloc(adjoint scratch)");
         CC_TRY(hipMalloc(&adj_b, 3 * scalar * (size_t)(D >= 1 ? n.V[D - 1] : 1)), "hipMalloc(adjoint scratch)");
-        CC_TRY(hipMalloc(&adj_w, scalar * (size_t)adj_scratch_scalars(n, D, true)), "hipMalloc(adjoint scratch)");
+        CC_TRY(hipMalloc(&adj_w, scalar * (size_t)adj_scratch_scalars(n, D, rare_on)),
+               "hipMalloc(adjoint scratch)");
+        if (rare_on && D >= 2)
+            CC_TRY(hipMalloc(&adj_mark, sizeof(uint64_t) * (size_t)((n.H[D - 1] + 63) / 64)), "hipMalloc(adjoint scratch)");
         adj_scalar = scalar;
+        adj_tiles = rare_on;
     }
     AdjPlan pl;
     pl.n = &n;
@@ -527,6 +535,9 @@ bool ccd_Subd::adjoint(const void *gradFinest, void *gradCage, int32_t steps, hi
     pl.per_vertex_max = opt_adj_vertex;
     pl.rare = rare;   // the forward's rare-vertex list, free between passes
     pl.rare_cap = rare_free ? 0 : rare_cap;
+    pl.rv = rare_view();
+    pl.border = defer_mask;   // the patch kernels' bits, free between passes
+    pl.mark = adj_mark;
     bool kept = erep != nullptr;
     for (int l = 1; l <= D - 2; ++l) kept = kept && erep_valid[l];
     pl.erep = kept ? erep : nullptr;
@@ -540,8 +551,10 @@ bool ccd_Subd::adjoint(const void *gradFinest, void *gradCage, int32_t steps, hi
                                (double *)adj_w, (double *)adj_sharp, creased, st);
     } else {
         if (!adj_vp && D >= 2)
-            CC_TRY(hipMalloc(&adj_vp, sizeof(VParam<float>) * (size_t)n.cumV(D - 1)), "hipMalloc(adjoint parameters)");
+            CC_TRY(hipMalloc(&adj_vp, (sizeof(VParam<float>) + 1) * (size_t)n.cumV(D - 1)), "hipMalloc(adjoint parameters)");
         pl.vp_cache = adj_vp;
+        if (D >= 2)   // a byte per vertex behind the records
+            pl.vp_plain = reinterpret_cast<uint8_t *>(static_cast<VParam<float> *>(adj_vp) + n.cumV(D - 1));
         pl.vp_valid = adj_vp_key == creased;
         adjoint_levels<float>(pl, (const float *)gradFinest, (float *)gradCage, (float *)adj_a, (float *)adj_b,
                               (float *)adj_w, nullptr, creased, st);
