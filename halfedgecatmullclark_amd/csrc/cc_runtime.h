@@ -21,16 +21,21 @@ struct ccd_Subd {
     int32_t D = 0, V0 = 0, U0 = 0, H0 = 0, E0 = 0, F0 = 0;
     cch::Counts n;
     cch::LevelTab tab;
-    // cage (level 0) on the device
+    // cage (level 0) on the device, with its ring lists and rare-vertex table
+    // in one allocation, packed in cage_host for the upload
+    char *cage_arena = nullptr;
+    size_t cage_cap = 0;
+    std::vector<char> cage_host;
+    cch::CageRings cage_rings;
+    cch::RareTable cage_rare;
     cch::CageHe *c_he = nullptr;
     int32_t *c_v2h = nullptr, *c_e2h = nullptr, *c_f2h = nullptr;
     cch::P3 *c_pts = nullptr;
     cch::UV *c_uvs = nullptr;
     cch::Crease *c_cr = nullptr;
-    // the cage's vertex and face ring lists (cch::DCage) in one device
-    // buffer; rings_ok false: the kernels walk the cage
+    // the cage's vertex and face ring lists (cch::DCage), at offsets in ints
+    // from the allocation's start; rings_ok false: the kernels walk the cage
     int32_t *rings = nullptr;
-    size_t rings_cap = 0;
     size_t o_vro = 0, o_vr = 0, o_vb = 0, o_fro = 0, o_fr = 0, o_voo = 0, o_vo = 0;
     // the masked vertex kernel's list of vertices without a ring from the
     // child numbering (FusedArgs::rare): at most V0 + F0 + (boundary
@@ -60,6 +65,7 @@ struct ccd_Subd {
     // (a topology or crease refinement, a cage upload)
     void *adj_vp = nullptr;
     int adj_vp_key = -1;
+    uint64_t *bits = nullptr;   // the three bit arrays that follow
     // deferred-vertex masks of the patch kernels, one word per 64 halfedges
     uint64_t *defer_mask = nullptr;
     // owner bits of levels 1..D-1 (FusedArgs::owner_mask; level d from word
