@@ -440,16 +440,6 @@ __device__ __forceinline__ int32_t border_slot(const AdjArgs<T> &a, int32_t h) {
     return (h & ~63) + __popcll(a.border[h >> 6] & ((1ull << (h & 63)) - 1ull));
 }
 
-// sorts r ascending (five exchanges)
-__device__ __forceinline__ void sort4(int32_t (&r)[4]) {
-    const auto order = [&](int i, int j) {
-        const int32_t lo = r[i] < r[j] ? r[i] : r[j], hi = r[i] < r[j] ? r[j] : r[i];
-        r[i] = lo;
-        r[j] = hi;
-    };
-    order(0, 1); order(2, 3); order(0, 2); order(1, 3); order(1, 2);
-}
-
 // a vertex's gradient from its summed weight and shares
 template <typename T>
 __device__ __forceinline__ void adj_vertex_store(const AdjArgs<T> &a, int32_t v, const V3<T> &gv, T alpha,
@@ -578,7 +568,7 @@ __device__ __forceinline__ void adj_border(const AdjArgs<T> &a, const DCage &c, 
                                            uint32_t block) {
     __shared__ LevelTab st;
     __shared__ LevelPtrs slp;
-    __shared__ int32_t list[4][64 * kAdjBorderWords];
+    __shared__ uint16_t list[4][64 * kAdjBorderWords];
     lds_fill(st, t);
     lds_fill(slp, lp);
     __syncthreads();

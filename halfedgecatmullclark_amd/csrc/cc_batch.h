@@ -35,7 +35,7 @@ struct CreaseJob {
 // compiler knows every address derived from it is global memory and emits
 // global rather than flat instructions); -1 marks an absent buffer.
 struct LevelJob {
-    int64_t he, out_he, cr, old, vp, fp, ep, defer_mask, owner_mask, rare, erep;
+    int64_t he, out_he, cr, old, vp, fp, ep, defer_mask, owner_mask, far, rare, erep;
     int64_t c_he, c_v2h, c_e2h, c_f2h, c_pts, c_uvs, c_cr, c_vro, c_vr, c_vb, c_fro, c_fr, c_voo, c_vo;
     int64_t lp[kMaxDepth + 1];
     int32_t H, V, F, E, C;
@@ -118,7 +118,9 @@ __host__ __device__ __forceinline__ DCage arena_cage(char *base, const J &j) {
 }
 
 // the kernel arguments of one cage's level from its job and the arena
-__host__ __device__ __forceinline__ void unpack_level(const LevelJob &J, char *arena, FusedArgs &a, DCage &c) {
+// (far: the masked kernel reads the tile kernel's marks)
+__host__ __device__ __forceinline__ void unpack_level(const LevelJob &J, char *arena, FusedArgs &a, DCage &c,
+                                                      int far = 0) {
     a.he = arena_ptr<const He>(arena, J.he);
     a.out_he = arena_ptr<He>(arena, J.out_he);
     a.cr = arena_ptr<const Crease>(arena, J.cr);
@@ -128,6 +130,7 @@ __host__ __device__ __forceinline__ void unpack_level(const LevelJob &J, char *a
     a.ep = arena_ptr<P3>(arena, J.ep);
     a.defer_mask = arena_ptr<uint64_t>(arena, J.defer_mask);
     a.owner_mask = arena_ptr<uint64_t>(arena, J.owner_mask);
+    a.far = far ? arena_ptr<uint64_t>(arena, J.far) : nullptr;
     a.rare = arena_ptr<int32_t>(arena, J.rare);
     a.rare_cap = J.rare_cap;
     a.erep = arena_ptr<uint64_t>(arena, J.erep);
@@ -216,8 +219,12 @@ void batch_level_deferred(const BatchTable &t, char *arena, int d, int gather, i
 // 16 mask words, kernel compiled for `waves` waves per SIMD)
 void batch_level_fused(const BatchTable &t, char *arena, int d, int gather, int creased, int topo, int remap, int nt,
                        int tiles, hipStream_t st);
+// (far: the vertices the tile kernel left, with scan 0)
 void batch_level_vertices(const BatchTable &t, char *arena, int d, int gather, int creased, int scan, int remap,
-                          int waves, hipStream_t st);
+                          int waves, int far, hipStream_t st);
+// points alone, tile by tile (one workgroup per tile of `quads` quads)
+void batch_level_points(const BatchTable &t, char *arena, int d, int gather, int creased, int remap, int quads,
+                        hipStream_t st);
 // after a scan-0 vertex launch: each job's rare list, one thread per entry
 // (`start` counts workgroups of 256 list entries)
 void batch_level_vertices_rare(const BatchTable &t, char *arena, int d, int gather, int creased, hipStream_t st);

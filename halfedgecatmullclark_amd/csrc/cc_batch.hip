@@ -5,6 +5,7 @@
 #include "cc_level.h"
 #include "cc_level0.h"
 #include "cc_patch.h"
+#include "cc_tile.h"
 
 namespace cch {
 
@@ -113,18 +114,35 @@ __global__ __launch_bounds__(NT) void k_batch_fused(const LevelJob *__restrict__
     }
 }
 
-// vertex points of the owners k_batch_fused marked (kOwnerWords mask words
-// per wave, four waves per workgroup; W waves per SIMD)
-template <int GATHER, int CREASED, int W>
-__global__ __launch_bounds__(256, W) void k_batch_vertices_masked(const LevelJob *__restrict__ jobs,
-                                                               const int32_t *__restrict__ start, int n, int d,
-                                                               int remap, char *arena) {
+// points alone of job k's level, tile by tile (workgroups of N threads)
+template <int GATHER, int CREASED, int N>
+__global__ __launch_bounds__(N, 8) void k_batch_points(const LevelJob *__restrict__ jobs,
+                                                       const int32_t *__restrict__ start, int n, int d, int remap,
+                                                       char *arena) {
     const uint32_t lb = xcd_block(blockIdx.x, gridDim.x, remap);
     const int k = find_job(start, n, lb);
     const LevelJob &J = jobs[k];
     FusedArgs a;
     DCage c;
-    unpack_level(J, arena, a, c);
+    unpack_level(J, arena, a, c, 1);
+    a.own_in = a.owner_mask;
+    a.par = arena_ptr<const He>(arena, J.lp[d - 1]);
+    a.pV = J.t.V[d - 1]; a.pF = J.t.F[d - 1]; a.pE = J.t.E[d - 1];
+    point_tile<GATHER, CREASED, N>(a, lb - (uint32_t)start[k]);
+}
+
+// vertex points of the owners k_batch_fused or k_batch_points marked (kOwnerWords mask words
+// per wave, four waves per workgroup; W waves per SIMD)
+template <int GATHER, int CREASED, int W>
+__global__ __launch_bounds__(256, W) void k_batch_vertices_masked(const LevelJob *__restrict__ jobs,
+                                                               const int32_t *__restrict__ start, int n, int d,
+                                                               int remap, int far, char *arena) {
+    const uint32_t lb = xcd_block(blockIdx.x, gridDim.x, remap);
+    const int k = find_job(start, n, lb);
+    const LevelJob &J = jobs[k];
+    FusedArgs a;
+    DCage c;
+    unpack_level(J, arena, a, c, far);
     const uint32_t b = lb - (uint32_t)start[k];
     if (b < (uint32_t)J.rare_blocks) {
         rare_vertices_block<GATHER, CREASED>(a, arena_rare(arena, J), J.t, d, b);
@@ -132,7 +150,7 @@ __global__ __launch_bounds__(256, W) void k_batch_vertices_masked(const LevelJob
     }
     const JobLevelPtrs lp{J.lp, arena};
     const int32_t wave = (int32_t)(b - (uint32_t)J.rare_blocks) * 4 + (int32_t)(threadIdx.x >> 6);
-    level_vertices_masked<GATHER, CREASED>(a, c, J.t, lp, d, wave);
+    level_vertices_masked<GATHER, CREASED, kOwnerWords>(a, c, J.t, lp, d, wave);
 }
 
 template <int GATHER, int CREASED>
@@ -171,17 +189,17 @@ void vertices_scan(const BatchTable &t, char *arena, int d, int remap, hipStream
 }
 
 template <int G, int C, int W>
-void vertices_masked(const BatchTable &t, char *arena, int d, int remap, hipStream_t st) {
+void vertices_masked(const BatchTable &t, char *arena, int d, int remap, int far, hipStream_t st) {
     hipLaunchKernelGGL((k_batch_vertices_masked<G, C, W>), dim3(t.blocks), dim3(256), 0, st,
-                       static_cast<const LevelJob *>(t.jobs), t.start, (int)t.n, d, remap, arena);
+                       static_cast<const LevelJob *>(t.jobs), t.start, (int)t.n, d, remap, far, arena);
 }
 
 template <int G, int C>
-void vertices_gc(const BatchTable &t, char *arena, int d, int scan, int remap, int waves, hipStream_t st) {
+void vertices_gc(const BatchTable &t, char *arena, int d, int scan, int remap, int waves, int far, hipStream_t st) {
     if (scan == 0) {
-        if (waves == 4) vertices_masked<G, C, 4>(t, arena, d, remap, st);
-        else if (waves == 6) vertices_masked<G, C, 6>(t, arena, d, remap, st);
-        else vertices_masked<G, C, kVertexWaves>(t, arena, d, remap, st);
+        if (waves == 4) vertices_masked<G, C, 4>(t, arena, d, remap, far, st);
+        else if (waves == 6) vertices_masked<G, C, 6>(t, arena, d, remap, far, st);
+        else vertices_masked<G, C, kVertexWaves>(t, arena, d, remap, far, st);
         return;
     }
     if (scan == 2) vertices_scan<G, C, 2>(t, arena, d, remap, st);
@@ -297,12 +315,30 @@ void batch_level_fused(const BatchTable &t, char *arena, int d, int gather, int 
 }
 
 void batch_level_vertices(const BatchTable &t, char *arena, int d, int gather, int creased, int scan, int remap,
-                          int waves, hipStream_t st) {
+                          int waves, int far, hipStream_t st) {
     if (t.blocks == 0 || t.n == 0) return;
-    if (gather && creased) vertices_gc<1, 1>(t, arena, d, scan, remap, waves, st);
-    else if (gather) vertices_gc<1, 0>(t, arena, d, scan, remap, waves, st);
-    else if (creased) vertices_gc<0, 1>(t, arena, d, scan, remap, waves, st);
-    else vertices_gc<0, 0>(t, arena, d, scan, remap, waves, st);
+    if (gather && creased) vertices_gc<1, 1>(t, arena, d, scan, remap, waves, far, st);
+    else if (gather) vertices_gc<1, 0>(t, arena, d, scan, remap, waves, far, st);
+    else if (creased) vertices_gc<0, 1>(t, arena, d, scan, remap, waves, far, st);
+    else vertices_gc<0, 0>(t, arena, d, scan, remap, waves, far, st);
+}
+
+template <int G, int C>
+static void points_gc(const BatchTable &t, char *arena, int d, int remap, int quads, hipStream_t st) {
+    const auto run = [&](auto k) {
+        hipLaunchKernelGGL(k, dim3(t.blocks), dim3((unsigned)quads), 0, st, static_cast<const LevelJob *>(t.jobs), t.start,
+                           (int)t.n, d, remap, arena);
+    };
+    run(quads == kTileBig ? k_batch_points<G, C, kTileBig> : k_batch_points<G, C, kTileSmall>);
+}
+
+void batch_level_points(const BatchTable &t, char *arena, int d, int gather, int creased, int remap, int quads,
+                        hipStream_t st) {
+    if (t.blocks == 0 || t.n == 0) return;
+    if (gather && creased) points_gc<1, 1>(t, arena, d, remap, quads, st);
+    else if (gather) points_gc<1, 0>(t, arena, d, remap, quads, st);
+    else if (creased) points_gc<0, 1>(t, arena, d, remap, quads, st);
+    else points_gc<0, 0>(t, arena, d, remap, quads, st);
 }
 
 void batch_level_vertices_rare(const BatchTable &t, char *arena, int d, int gather, int creased, hipStream_t st) {

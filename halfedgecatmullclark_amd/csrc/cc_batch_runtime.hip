@@ -40,6 +40,7 @@ struct ccb_Batch {
         RareView rv;   // its counts
         int64_t o_adjVP = 0;   // VParam offset of levels 1..D-1's vertex-rule parameters
         int32_t rare_cap = 0;   // rare-vertex list entries (FusedArgs::rare), the count first
+        int64_t o_own[kMaxDepth + 1] = {};   // word offsets of the levels' owner bits
         int64_t o_erep = -1;    // word offset of the edge-representative bits (depth >= 4)
     };
     struct Timed {
@@ -77,6 +78,12 @@ struct ccb_Batch {
     Crease *cr = nullptr;
     P3 *pts = nullptr;
     uint64_t *defer_mask = nullptr;   // deferred-vertex masks, per cage one word per 64 halfedges
+    // owner bits of every cage's levels 1..D-1 (FusedArgs::owner_mask), and
+    // from there tot_own words on the tile kernel's marks; own_done: a
+    // forward pass over the topology has written the owner bits of all levels
+    uint64_t *own_masks = nullptr;
+    int64_t tot_own = 0;
+    bool own_done = false;
     float *adjA = nullptr, *adjB = nullptr, *adjW = nullptr, *adjCage = nullptr;
     // every cage's vertex-rule parameters of levels 1..D-1, kept across
     // adjoint calls (a batch's topology and creases never change); valid for
@@ -92,6 +99,8 @@ struct ccb_Batch {
     BatchTable t_cr[kMaxDepth + 1], t_patch[kMaxDepth + 1], t_def[kMaxDepth + 1];
     BatchTable t_rare[kMaxDepth + 1];   // rare-vertex lists after the scan-0 vertex kernel
     BatchTable t_fused[kMaxDepth + 1], t_vert[kMaxDepth + 1];
+    BatchTable t_points[kMaxDepth + 1];   // points alone, tiles of tile_quads quads
+    int tile_quads[kMaxDepth + 1] = {};
     AdjLevelTables t_adj[kMaxDepth + 1];   // levels 1 ..
     BatchTable t_adjc_h, t_adjc_e, t_adjc_f, t_adjc_v;   // cage-step adjoint gathers: per edge, face, vertex
     bool all_rings = true;                     // every cage has its ring lists
@@ -113,7 +122,7 @@ struct ccb_Batch {
     int remap = 1, use_graph = 1;
     bool timing = false;
     std::vector<Timed> timed;
-    std::map<int32_t, hipGraphExec_t> graphs;   // forward: steps; adjoint: -1 - creased - 2 params
+    std::map<int32_t, hipGraphExec_t> graphs;   // forward: forward_key; adjoint: -1 - creased - 2 params
     bool topo_done = false, creases_done = false;
 
     bool create(const cc_Mesh *const *meshes, const int32_t *depths, int32_t count);
@@ -125,6 +134,10 @@ struct ccb_Batch {
     // flags: 1 creased rules, 2 run the parameter pass
     void record_adjoint(int flags, hipStream_t st);
     bool run(int32_t key, bool adjoint, int32_t steps, hipStream_t st);
+    void note_owners();
+    // the graph of a forward pass: points alone take other kernels once the
+    // owner bits are there
+    int32_t forward_key(int32_t steps) const { return steps | (!(steps & CCD_HALFEDGES) && own_done ? 1 << 30 : 0); }
     int32_t autotune(int32_t steps, hipStream_t st);
     void begin_timing();
     template <typename Fn>
@@ -305,6 +318,10 @@ bool ccb_Batch::create(const cc_Mesh *const *meshes, const int32_t *depths, int3
         g.o_cr = tot_cr; tot_cr += g.n.cumC(g.D);
         g.o_pts = tot_pts; tot_pts += g.n.cumV(g.D);
         g.o_fin = tot_fin; tot_fin += g.n.V[g.D];
+        for (int d = 1; d < g.D; ++d) {
+            g.o_own[d] = tot_own;
+            tot_own += (g.n.H[d] + 63) / 64;
+        }
         g.o_def = tot_def; tot_def += g.D >= 2 ? (g.n.H[g.D - 1] + 63) / 64 : 1;
         if (!g.rv.on) {
             int64_t b0 = 0;
@@ -340,6 +357,7 @@ bool ccb_Batch::create(const cc_Mesh *const *meshes, const int32_t *depths, int3
         const size_t o_cr = cv.take(sizeof(Crease) * (size_t)tot_cr);
         const size_t o_pts = cv.take(sizeof(P3) * (size_t)tot_pts);
         const size_t o_def = cv.take(sizeof(uint64_t) * (size_t)tot_def);
+        const size_t o_own = cv.take(sizeof(uint64_t) * (size_t)(2 * tot_own + 1));
         const size_t o_rare = cv.take(sizeof(int32_t) * (size_t)(tot_rare + 1));
         const size_t o_erep = cv.take(sizeof(uint64_t) * (size_t)(tot_erep + 1));
         CC_TRY(hipMalloc(&arena, cv.size), "hipMalloc(batch arena)");
@@ -355,6 +373,7 @@ bool ccb_Batch::create(const cc_Mesh *const *meshes, const int32_t *depths, int3
         cr = reinterpret_cast<Crease *>(arena + o_cr);
         pts = reinterpret_cast<P3 *>(arena + o_pts);
         defer_mask = reinterpret_cast<uint64_t *>(arena + o_def);
+        own_masks = reinterpret_cast<uint64_t *>(arena + o_own);
         rare = reinterpret_cast<int32_t *>(arena + o_rare);
         erep = reinterpret_cast<uint64_t *>(arena + o_erep);
     }
@@ -499,7 +518,15 @@ bool ccb_Batch::build_tables() {
         for (int l = 1; l < d; ++l) fused_below = fused_below && cfg[l].kind == 1;
         const bool fused_upto = fused_below && cfg[d].kind == 1;
         std::vector<LevelJob> jobs;
-        std::vector<int64_t> bp, bd, bf, bv, br;
+        std::vector<int64_t> bp, bd, bf, bv, br, bt;
+        // tiles of 1024 quads where they are mostly full and fill the chip
+        int64_t quads = 0, big = 0;
+        for (const Cage &g : cages) {
+            if (g.D <= d) continue;
+            quads += g.n.F[d];
+            big += blocks_of(g.n.F[d], kTileBig);
+        }
+        tile_quads[d] = quads >= kTileBigFrom && 4 * quads >= 3 * kTileBig * big ? kTileBig : kTileSmall;
         for (int i = 0; i < N; ++i) {
             const Cage &g = cages[i];
             if (g.D <= d) continue;
@@ -515,7 +542,8 @@ bool ccb_Batch::build_tables() {
             j.fp = off(vp + g.n.V[d]);
             j.ep = off(vp + g.n.V[d] + g.n.F[d]);
             j.defer_mask = off(defer_mask + g.o_def);
-            j.owner_mask = cfg[d].kind == 1 && cfg[d].scan == 0 ? j.defer_mask : -1;
+            j.owner_mask = cfg[d].kind == 1 && cfg[d].scan == 0 ? off(own_masks + g.o_own[d]) : -1;
+            j.far = off(own_masks + tot_own + g.o_own[d]);
             const bool listed = j.owner_mask >= 0 && !g.rv.on;
             j.rare = listed ? off(rare + g.o_rare) : -1;
             j.rare_cap = listed ? g.rare_cap : 0;
@@ -542,6 +570,7 @@ bool ccb_Batch::build_tables() {
             bp.push_back((tiles + cfg[d].hpt - 1) / cfg[d].hpt);
             bd.push_back(blocks_of(blocks_of(blocks_of(g.n.H[d], 64), kDeferGroup), 4));
             bf.push_back(blocks_of(g.n.H[d], (int64_t)cfg[d].fb * cfg[d].ft));
+            bt.push_back(blocks_of(g.n.F[d], tile_quads[d]));
             br.push_back(j.rare_cap > 0 ? blocks_of(j.rare_cap) : 0);
             bv.push_back(cfg[d].scan == 0 ? j.rare_blocks + blocks_of(blocks_of(blocks_of(g.n.H[d], 64), kOwnerWords), 4)
                                           : blocks_of(g.n.H[d], 256 * cfg[d].scan));
@@ -551,6 +580,7 @@ bool ccb_Batch::build_tables() {
         tb.add(t_fused[d], jobs, bf);
         tb.add(t_vert[d], jobs, bv);
         tb.add(t_rare[d], jobs, br);
+        tb.add(t_points[d], jobs, bt);
     }
     if (adj_arena) {   // adjoint steps d+1 -> d, d = 0 the cage step
         for (int d = 0; d < Dmax; ++d) {
@@ -700,13 +730,18 @@ void ccb_Batch::record_forward(int32_t steps, hipStream_t st) {
             timed_launch("level_deferred", d, st,
                          [&] { batch_level_deferred(t_def[d], arena, d, gather, creased, st); });
         } else {
-            timed_launch("level_fused", d, st,
+            // points alone, with the owner bits of an earlier pass: the tile kernel
+            const int tiles = !topo && d >= 2 && own_done && cfg[d].scan == 0 ? 1 : 0;
+            if (tiles) timed_launch("level_points", d, st, [&] {
+                batch_level_points(t_points[d], arena, d, gather, creased, remap, tile_quads[d], st);
+            });
+            else timed_launch("level_fused", d, st,
                          [&] {
                              batch_level_fused(t_fused[d], arena, d, gather, creased, topo, remap, cfg[d].fb,
                                                cfg[d].ft, st);
                          });
             timed_launch("level_vertices", d, st, [&] {
-                batch_level_vertices(t_vert[d], arena, d, gather, creased, cfg[d].scan, remap, cfg[d].vw, st);
+                batch_level_vertices(t_vert[d], arena, d, gather, creased, cfg[d].scan, remap, cfg[d].vw, tiles, st);
                 if (cfg[d].scan == 0) batch_level_vertices_rare(t_rare[d], arena, d, gather, creased, st);
             });
         }
@@ -763,6 +798,13 @@ bool ccb_Batch::run(int32_t key, bool adjoint, int32_t steps, hipStream_t st) {
     }
     CC_TRY(hipGraphLaunch(it->second, st), "hipGraphLaunch");
     return true;
+}
+
+// after a pass over the topology: has it written every level's owner bits?
+void ccb_Batch::note_owners() {
+    bool all = true;
+    for (int d = 1; d < Dmax; ++d) all = all && cfg[d].kind == 1 && cfg[d].scan == 0;
+    own_done = own_done || all;
 }
 
 // Times candidate kernel configurations on this batch with HIP events and
@@ -935,8 +977,11 @@ int32_t ccb_Refine(ccb_Batch *b, int32_t steps, void *stream) {
     if (steps & CCD_HALFEDGES) steps |= CCD_UVS;
     DeviceGuard g(b->device);
     hipStream_t st = (hipStream_t)stream;
-    if (!b->run(steps, false, steps, st)) return last_error();
-    if (steps & CCD_HALFEDGES) b->topo_done = true;
+    if (!b->run(b->forward_key(steps), false, steps, st)) return last_error();
+    if (steps & CCD_HALFEDGES) {
+        b->topo_done = true;
+        b->note_owners();
+    }
     if (steps & CCD_CREASES) b->creases_done = true;
     return 0;
 }
@@ -954,7 +999,7 @@ int32_t ccb_RefinePoints(ccb_Batch *b, const float *devCagePoints, int32_t steps
                    "ccb_RefinePoints"))
         return last_error();
     const int32_t s = CCD_POINTS | (steps & (CCD_GATHER | CCD_NOCREASES));
-    return b->run(s, false, s, st) ? 0 : last_error();
+    return b->run(b->forward_key(s), false, s, st) ? 0 : last_error();
 }
 
 int32_t ccb_FinestPoints(ccb_Batch *b, float *devOut, void *stream) {

@@ -107,6 +107,15 @@ __device__ __forceinline__ P3 face_rule(P3 p0, P3 p1, P3 p2, P3 p3, bool gather)
     return a;
 }
 
+// The same from each lane's own corner, by DPP; the quarters are taken before
+// the exchange, which then folds into the additions.
+template <int GATHER>
+__device__ __forceinline__ P3 quad_face_rule(P3 P) {
+    if (GATHER) return face_rule(quad_bcast3<0>(P), quad_bcast3<1>(P), quad_bcast3<2>(P), quad_bcast3<3>(P), true);
+    const P3 q = P3{P.x / 4.0f, P.y / 4.0f, P.z / 4.0f};
+    return add(add(add(add(zero3(), quad_bcast3<0>(q)), quad_bcast3<1>(q)), quad_bcast3<2>(q)), quad_bcast3<3>(q));
+}
+
 __device__ __forceinline__ P3 quad_face(const He *he, const P3 *old, int32_t quad_base, bool gather) {
     const HeView q4{he + quad_base};
     return face_rule(old[q4[0].z], old[q4[1].z], old[q4[2].z], old[q4[3].z], gather);
@@ -337,6 +346,16 @@ __device__ __forceinline__ void cage_face_fan(const DCage &c, int32_t face, int3
     f.n = n;
 }
 
+// sorts r ascending (five exchanges)
+__device__ __forceinline__ void sort4(int32_t (&r)[4]) {
+    const auto order = [&](int i, int j) {
+        const int32_t lo = r[i] < r[j] ? r[i] : r[j], hi = r[i] < r[j] ? r[j] : r[i];
+        r[i] = lo;
+        r[j] = hi;
+    };
+    order(0, 1); order(2, 3); order(0, 2); order(1, 3); order(1, 2);
+}
+
 // Is h the representative of its vertex (CatmullClark.h:1336)?  The test of
 // owner_fan without building the fan (no twin record is read).
 __device__ __forceinline__ bool owner_test(int32_t h, int32_t vert, int d, const DCage &c, const LevelTab &t,
@@ -440,10 +459,10 @@ __device__ __forceinline__ void wave_lds_sync() {
 
 // Calls fn(h) once per bit set in mask words [w0, w0 + GW) of `words`, one
 // halfedge per lane in ascending order, in rounds of 64.  The wave lists the
-// marked halfedges in `list` (its own 64 GW slots of LDS): lane l of word w
-// writes w * 64 + l at the count of set bits before it (mbcnt).
+// marked halfedges in `list` (its own 64 GW slots of LDS): lane l of its word
+// j writes j * 64 + l at the count of set bits before it (mbcnt).
 template <int GW, class Fn>
-__device__ __forceinline__ void mask_group(const uint64_t *mask, int32_t w0, int32_t words, int32_t *list,
+__device__ __forceinline__ void mask_group(const uint64_t *mask, int32_t w0, int32_t words, uint16_t *list,
                                            const Fn &fn) {
     const int lane = (int)(threadIdx.x & 63u);
     int32_t total = 0;
@@ -454,11 +473,11 @@ __device__ __forceinline__ void mask_group(const uint64_t *mask, int32_t w0, int
         const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)m);
         const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(m >> 32));
         const uint32_t rank = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
-        if (((lane < 32 ? lo >> lane : hi >> (lane - 32)) & 1u) != 0u) list[total + (int32_t)rank] = w * 64 + lane;
+        if (((lane < 32 ? lo >> lane : hi >> (lane - 32)) & 1u) != 0u) list[total + (int32_t)rank] = (uint16_t)(j * 64 + lane);
         total += __popc(lo) + __popc(hi);
     }
     wave_lds_sync();
-    for (int32_t i = lane; i < total; i += 64) fn(list[i]);
+    for (int32_t i = lane; i < total; i += 64) fn(w0 * 64 + (int32_t)list[i]);
 }
 
 // Is level-d halfedge h the representative of its vertex?  owner_test

@@ -18,6 +18,20 @@ constexpr int kFusedBlock = 1024;
 // needs 56 registers: 8 fit without spilling); the autotuner may pick 4 or 6
 constexpr int kVertexWaves = 8;
 
+// The tile kernel (cc_tile.h): quads, and threads, of a tile of a level with
+// F quads.  Large tiles leave fewer vertices to the masked kernel, small ones
+// spread a small level over the chip: at 2.1 M quads 40 us and 18 for the
+// vertices with 1024 against 41 and 23 with 256, at 33 thousand 6.3 + 10.6
+// against 5.2 + 12.7, at 12 thousand 7.6 + 17.4 against 4.7 + 17.4.  The line
+// is two tiles of 1024 per CU.
+constexpr int kTileBig = 1024, kTileSmall = 256;
+constexpr int64_t kTileBigFrom = 512 * kTileBig;
+// The masked kernel's mask words per wave behind it, where few bits are set:
+// 16 of large levels (at 134 M halfedges 374 us, with 8
+// words 397), else kOwnerWords (at 262 thousand halfedges 11.7 us with 16, 7.4
+// with 8).
+constexpr int kFarWords = 16;
+
 // Level-d inputs and level-(d+1) outputs of one fused launch.
 struct FusedArgs {
     const He *he;       // level d halfedges
@@ -55,6 +69,15 @@ struct FusedArgs {
     // 0: owner_mask already holds this level's bits (a points-only pass over
     // an unchanged topology), the fused kernel leaves them
     int owner_write = 1;
+    // the tile kernel (cc_tile.h): level d-1's records and counts, the
+    // level's owner bits and where the bits of the representatives it leaves
+    // to the masked kernel go.  These follow from the topology and creases
+    // alone, but every pass writes them before it reads them, so passes on
+    // several streams need no order between them (16 MB beside 2.5 GB).
+    const He *par = nullptr;
+    int32_t pV = 0, pF = 0, pE = 0;
+    const uint64_t *own_in = nullptr;
+    uint64_t *far = nullptr;
 };
 
 // The vertices of a cage's levels that no ring kernel takes, as cc_rare.h
@@ -88,6 +111,9 @@ __host__ __device__ __forceinline__ uint32_t rare_blocks(const RareView &r, int 
 // workgroup processes in turn, 1, 2 or 4
 void launch_level_fused(const FusedArgs &a, const DCage &c, const LevelTab &t, int d, int gather, int creased, int topo,
                         int uvMode, int points, int store, int nt, int tiles, hipStream_t st);
+// points of level d+1 alone, tile by tile (d >= 2); launch_level_vertices
+// finishes the vertices it marks in a.far
+void launch_level_points(const FusedArgs &a, int gather, int creased, hipStream_t st);
 // base pointers of the halfedges of every level (index 1..D)
 struct LevelPtrs {
     const He *he[kMaxDepth + 1];
@@ -125,6 +151,7 @@ void launch_level_deferred(const FusedArgs &a, const DCage &c, const LevelTab &t
 // kernel compiled for `waves` waves per SIMD, 4, 6 or 8)
 // rv: with on set, the masked kernel's launch also finishes the vertices of
 // the table, and a.rare may be null
+// with a.far set, the masked kernel reads the tile kernel's marks
 void launch_level_vertices(const FusedArgs &a, const DCage &c, const LevelTab &t, const LevelPtrs &lp,
                            const RareView &rv, int d, int gather, int creased, int fan, int scan, int waves,
                            hipStream_t st);

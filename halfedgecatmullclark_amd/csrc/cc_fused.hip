@@ -20,6 +20,7 @@
 // Blocks are remapped so that each XCD processes one contiguous range of
 // the level, keeping neighbouring quads in the same L2.
 #include "cc_level.h"
+#include "cc_tile.h"
 
 namespace cch {
 
@@ -43,10 +44,16 @@ __global__ __launch_bounds__(NT) void k_level_fused(FusedArgs a, DCage c, LevelT
     }
 }
 
+// (eight waves per SIMD: 55 registers, 64 by the gather rules)
+template <int GATHER, int CREASED, int N>
+__global__ __launch_bounds__(N, 8) void k_level_points(FusedArgs a) {
+    point_tile<GATHER, CREASED, N>(a, xcd_block(blockIdx.x, gridDim.x, a.xcd_remap));
+}
+
 // ring vertices; the others in the first nr workgroups when the cage has a
 // rare-vertex table, else to the rare list and k_level_vertices_rare
 // (W waves per SIMD: 8 fit without spilling, 56 registers)
-template <int GATHER, int CREASED, int W>
+template <int GATHER, int CREASED, int W, int WORDS>
 __global__ __launch_bounds__(256, W) void k_level_vertices_ring(FusedArgs a, DCage c, LevelTab t, LevelPtrs lp, int d,
                                                                 RareView rv, uint32_t nr) {
     if (blockIdx.x < nr) {
@@ -54,7 +61,7 @@ __global__ __launch_bounds__(256, W) void k_level_vertices_ring(FusedArgs a, DCa
         return;
     }
     const uint32_t lb = xcd_block(blockIdx.x - nr, gridDim.x - nr, a.xcd_remap);
-    level_vertices_masked<GATHER, CREASED>(a, c, t, lp, d, (int32_t)(lb * 4 + (threadIdx.x >> 6)));
+    level_vertices_masked<GATHER, CREASED, WORDS>(a, c, t, lp, d, (int32_t)(lb * 4 + (threadIdx.x >> 6)));
 }
 
 template <int GATHER, int CREASED>
@@ -315,12 +322,24 @@ static void launch_ring(const FusedArgs &a, const DCage &c, const LevelTab &t, c
                         const RareView &rv, int waves, dim3 grid, hipStream_t st) {
     const uint32_t nr = rare_blocks(rv, d);
     grid.x += nr;
-    if (waves == 4)
-        hipLaunchKernelGGL((k_level_vertices_ring<G, C, 4>), grid, dim3(256), 0, st, a, c, t, lp, d, rv, nr);
-    else if (waves == 6)
-        hipLaunchKernelGGL((k_level_vertices_ring<G, C, 6>), grid, dim3(256), 0, st, a, c, t, lp, d, rv, nr);
-    else
-        hipLaunchKernelGGL((k_level_vertices_ring<G, C, kVertexWaves>), grid, dim3(256), 0, st, a, c, t, lp, d, rv, nr);
+    const auto run = [&](auto k) { hipLaunchKernelGGL(k, grid, dim3(256), 0, st, a, c, t, lp, d, rv, nr); };
+    if (a.far && a.F >= kTileBigFrom) run(k_level_vertices_ring<G, C, kVertexWaves, kFarWords>);
+    else if (waves == 4) run(k_level_vertices_ring<G, C, 4, kOwnerWords>);
+    else if (waves == 6) run(k_level_vertices_ring<G, C, 6, kOwnerWords>);
+    else run(k_level_vertices_ring<G, C, kVertexWaves, kOwnerWords>);
+}
+
+template <int N>
+static void launch_points(const FusedArgs &a, int gather, int creased, hipStream_t st) {
+    const dim3 grid((unsigned)((a.F + (int64_t)N - 1) / N));
+    const auto run = [&](auto k) { hipLaunchKernelGGL(k, grid, dim3(N), 0, st, a); };
+    if (gather) run(creased ? k_level_points<1, 1, N> : k_level_points<1, 0, N>);
+    else run(creased ? k_level_points<0, 1, N> : k_level_points<0, 0, N>);
+}
+
+void launch_level_points(const FusedArgs &a, int gather, int creased, hipStream_t st) {
+    if (a.F >= kTileBigFrom) launch_points<kTileBig>(a, gather, creased, st);
+    else launch_points<kTileSmall>(a, gather, creased, st);
 }
 
 void launch_level_vertices(const FusedArgs &a, const DCage &c, const LevelTab &t, const LevelPtrs &lp,
@@ -338,7 +357,7 @@ void launch_level_vertices(const FusedArgs &a, const DCage &c, const LevelTab &t
     }
     if (fan == 2 && scan == 0 && a.owner_mask && (a.rare || rv.on)) {   // owners marked by the fused kernel
         const int64_t words = ((int64_t)a.H + 63) / 64;
-        const int64_t mask_waves = (words + kOwnerWords - 1) / kOwnerWords;
+        const int64_t per = a.far && a.F >= kTileBigFrom ? kFarWords : kOwnerWords, mask_waves = (words + per - 1) / per;
         const dim3 g0((unsigned)((mask_waves + 3) / 4)), gr((unsigned)((a.rare_cap + 255) / 256));
         if (gather && creased) {
             launch_ring<1, 1>(a, c, t, lp, d, rv, waves, g0, st);

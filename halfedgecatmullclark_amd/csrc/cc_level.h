@@ -396,20 +396,21 @@ struct RingVertexFn {
     }
 };
 
-// vertex points of the owners marked by the fused kernel; `wave` is the
-// index of this wave among the level's waves (kOwnerWords words each)
-template <int GATHER, int CREASED, class LP>
+// vertex points of the owners the fused kernel marked, or of the far ones the
+// tile kernel left; `wave` is the
+// index of this wave among the level's waves (WORDS words each)
+template <int GATHER, int CREASED, int WORDS, class LP>
 __device__ __forceinline__ void level_vertices_masked(const FusedArgs &a, const DCage &c, const LevelTab &t,
                                                       const LP &lp, int d, int32_t wave) {
     __shared__ LevelTab st;
     __shared__ LevelPtrs slp;
-    __shared__ int32_t list[4][64 * kOwnerWords];   // four waves per workgroup
+    __shared__ uint16_t list[4][64 * WORDS];   // four waves per workgroup
     lds_fill(st, t);
     lds_fill(slp, lp);
     __syncthreads();
     const int32_t words = (a.H + 63) >> 6;
-    mask_group<kOwnerWords>(a.owner_mask, wave * kOwnerWords, words, list[threadIdx.x >> 6],
-                            RingVertexFn<GATHER, CREASED>{a, c, st, slp, d});
+    mask_group<WORDS>(a.far ? a.far : a.owner_mask, wave * WORDS, words, list[threadIdx.x >> 6],
+                      RingVertexFn<GATHER, CREASED>{a, c, st, slp, d});
 }
 
 // workgroup `block` (four waves) of the level's rare vertices

@@ -65,7 +65,7 @@ struct ccd_Subd {
     // (a topology or crease refinement, a cage upload)
     void *adj_vp = nullptr;
     int adj_vp_key = -1;
-    uint64_t *bits = nullptr;   // the three bit arrays that follow
+    uint64_t *bits = nullptr;   // the bit arrays that follow
     // deferred-vertex masks of the patch kernels, one word per 64 halfedges
     uint64_t *defer_mask = nullptr;
     // owner bits of levels 1..D-1 (FusedArgs::owner_mask; level d from word
@@ -74,6 +74,9 @@ struct ccd_Subd {
     uint64_t *own_masks = nullptr;
     int64_t own_off[cch::kMaxDepth + 1] = {};
     bool own_valid[cch::kMaxDepth + 1] = {};
+    // likewise the representatives the tile kernel leaves to the vertex kernel
+    // (FusedArgs::far)
+    uint64_t *far_masks = nullptr;
     // edge-representative bits of levels 1..D-2 (FusedArgs::erep; the owner
     // test of level d reads levels up to d-1), and which levels hold bits of
     // the current cage's topology

@@ -83,18 +83,22 @@ bool ccd_Subd::alloc(const cc_Mesh *cage, int32_t depth) {
     CC_TRY(hipMalloc(&he, sizeof(He) * (size_t)n.cumH(D)), "hipMalloc(halfedges)");
     CC_TRY(hipMalloc(&cr, sizeof(Crease) * (size_t)n.cumC(D)), "hipMalloc(creases)");
     CC_TRY(hipMalloc(&pts, sizeof(P3) * (size_t)n.cumV(D)), "hipMalloc(points)");
-    // bit arrays: deferred vertices, edge representatives, vertex owners
+    // bit arrays: deferred vertices, edge representatives, vertex owners and
+    // those left to the vertex kernel
     const int64_t defer_words = D >= 2 ? (n.H[D - 1] + 63) / 64 : 1;
     const int64_t erep_words = D >= 4 ? tab.R[D - 1] : 0;
     int64_t words = defer_words + erep_words;
+    int64_t own_words = 0;
     for (int d = 1; d < D; ++d) {
-        own_off[d] = words - defer_words - erep_words;
-        words += (n.H[d] + 63) / 64;
+        own_off[d] = own_words;
+        own_words += (n.H[d] + 63) / 64;
     }
+    words += 2 * own_words;
     CC_TRY(hipMalloc(&bits, sizeof(uint64_t) * (size_t)(words + 1)), "hipMalloc(bit arrays)");
     defer_mask = bits;
     erep = D >= 4 ? bits + defer_words : nullptr;
     own_masks = bits + defer_words + erep_words;
+    far_masks = own_masks + own_words;
     return true;
 }
 
@@ -391,7 +395,16 @@ void ccd_Subd::level_fused(int d, int32_t steps, int topo, int uvMode, P3 *point
         a.erep_read = d >= 2 && below ? 1 : 0;
         a.erep_write = d + 1 <= D - 2 && (d == 1 || erep_valid[d]) ? 1 : 0;
     }
-    if (topo || uvMode == 1 || pts_) {
+    // points alone, with the owner bits of an earlier pass: the tile kernel,
+    // which marks the vertices it leaves
+    const bool tiles = a.owner_mask && !topo && uvMode == 0 && d >= 2 && own_valid[d];
+    if (tiles) {
+        a.own_in = a.owner_mask;
+        a.far = far_masks + own_off[d];
+        a.par = he + n.offH[d - 1];
+        a.pV = (int32_t)n.V[d - 1]; a.pF = (int32_t)n.F[d - 1]; a.pE = (int32_t)n.E[d - 1];
+        launch_timed("level_points", n.H[d], st, [&] { launch_level_points(a, gather, creased, st); });
+    } else if (topo || uvMode == 1 || pts_) {
         launch_timed(pts_ ? (topo ? "level_fused" : "level_points") : "level_fused", n.H[d], st,
                      [&] {
                          launch_level_fused(a, c, tab, d, gather, creased, topo, uvMode, pts_, opt_store, cfg[d].fb,
