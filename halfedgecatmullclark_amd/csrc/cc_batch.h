@@ -219,7 +219,10 @@ void batch_level_deferred(const BatchTable &t, char *arena, int d, int gather, i
 // 16 mask words, kernel compiled for `waves` waves per SIMD)
 void batch_level_fused(const BatchTable &t, char *arena, int d, int gather, int creased, int topo, int remap, int nt,
                        int tiles, hipStream_t st);
-// (far: the vertices the tile kernel left, with scan 0)
+// children and owner bits without points, for the tile kernel
+void batch_level_children(const BatchTable &t, char *arena, int d, int remap, int nt, int tiles, hipStream_t st);
+// (far, with scan 0: the vertices the tile kernel left; kFarWords: its table
+// counts that many mask words per wave)
 void batch_level_vertices(const BatchTable &t, char *arena, int d, int gather, int creased, int scan, int remap,
                           int waves, int far, hipStream_t st);
 // points alone, tile by tile (one workgroup per tile of `quads` quads)

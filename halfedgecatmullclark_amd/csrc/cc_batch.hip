@@ -93,7 +93,8 @@ __global__ __launch_bounds__(NT) void k_batch_patch(const LevelJob *__restrict__
 // children with face and edge points of job k's level (workgroups of NT
 // threads; MULTI: each processing `tiles` tiles of NT halfedges in turn, a
 // kernel of its own since the loop costs registers)
-template <int GATHER, int CREASED, int TOPO, int NT, int MULTI>
+// POINTS 0: children and owner bits alone
+template <int GATHER, int CREASED, int TOPO, int NT, int MULTI, int POINTS = 1>
 __global__ __launch_bounds__(NT) void k_batch_fused(const LevelJob *__restrict__ jobs, const int32_t *__restrict__ start,
                                                     int n, int d, int remap, int tiles, char *arena) {
     const uint32_t lb = xcd_block(blockIdx.x, gridDim.x, remap);
@@ -104,12 +105,12 @@ __global__ __launch_bounds__(NT) void k_batch_fused(const LevelJob *__restrict__
     unpack_level(J, arena, a, c);
     constexpr int UV = TOPO ? 3 : 0;
     if constexpr (!MULTI) {
-        level_fused_block<GATHER, CREASED, TOPO, UV, 1, kStoreLds, NT>(a, c, J.t, d, lb - (uint32_t)start[k]);
+        level_fused_block<GATHER, CREASED, TOPO, UV, POINTS, kStoreLds, NT>(a, c, J.t, d, lb - (uint32_t)start[k]);
     } else {
         const uint32_t tile0 = (lb - (uint32_t)start[k]) * (uint32_t)tiles;
         for (int q = 0; q < tiles; ++q) {
             if (q) __syncthreads();
-            level_fused_block<GATHER, CREASED, TOPO, UV, 1, kStoreLds, NT>(a, c, J.t, d, tile0 + (uint32_t)q);
+            level_fused_block<GATHER, CREASED, TOPO, UV, POINTS, kStoreLds, NT>(a, c, J.t, d, tile0 + (uint32_t)q);
         }
     }
 }
@@ -133,7 +134,7 @@ __global__ __launch_bounds__(N, 8) void k_batch_points(const LevelJob *__restric
 
 // vertex points of the owners k_batch_fused or k_batch_points marked (kOwnerWords mask words
 // per wave, four waves per workgroup; W waves per SIMD)
-template <int GATHER, int CREASED, int W>
+template <int GATHER, int CREASED, int W, int WORDS = kOwnerWords>
 __global__ __launch_bounds__(256, W) void k_batch_vertices_masked(const LevelJob *__restrict__ jobs,
                                                                const int32_t *__restrict__ start, int n, int d,
                                                                int remap, int far, char *arena) {
@@ -150,7 +151,7 @@ __global__ __launch_bounds__(256, W) void k_batch_vertices_masked(const LevelJob
     }
     const JobLevelPtrs lp{J.lp, arena};
     const int32_t wave = (int32_t)(b - (uint32_t)J.rare_blocks) * 4 + (int32_t)(threadIdx.x >> 6);
-    level_vertices_masked<GATHER, CREASED, kOwnerWords>(a, c, J.t, lp, d, wave);
+    level_vertices_masked<GATHER, CREASED, WORDS>(a, c, J.t, lp, d, wave);
 }
 
 template <int GATHER, int CREASED>
@@ -188,16 +189,17 @@ void vertices_scan(const BatchTable &t, char *arena, int d, int remap, hipStream
                        static_cast<const LevelJob *>(t.jobs), t.start, (int)t.n, d, remap, arena);
 }
 
-template <int G, int C, int W>
+template <int G, int C, int W, int WORDS = kOwnerWords>
 void vertices_masked(const BatchTable &t, char *arena, int d, int remap, int far, hipStream_t st) {
-    hipLaunchKernelGGL((k_batch_vertices_masked<G, C, W>), dim3(t.blocks), dim3(256), 0, st,
+    hipLaunchKernelGGL((k_batch_vertices_masked<G, C, W, WORDS>), dim3(t.blocks), dim3(256), 0, st,
                        static_cast<const LevelJob *>(t.jobs), t.start, (int)t.n, d, remap, far, arena);
 }
 
 template <int G, int C>
 void vertices_gc(const BatchTable &t, char *arena, int d, int scan, int remap, int waves, int far, hipStream_t st) {
     if (scan == 0) {
-        if (waves == 4) vertices_masked<G, C, 4>(t, arena, d, remap, far, st);
+        if (far == kFarWords) vertices_masked<G, C, kVertexWaves, kFarWords>(t, arena, d, remap, far, st);
+        else if (waves == 4) vertices_masked<G, C, 4>(t, arena, d, remap, far, st);
         else if (waves == 6) vertices_masked<G, C, 6>(t, arena, d, remap, far, st);
         else vertices_masked<G, C, kVertexWaves>(t, arena, d, remap, far, st);
         return;
@@ -312,6 +314,17 @@ void batch_level_fused(const BatchTable &t, char *arena, int d, int gather, int 
     else if (gather) fused_gc<1, 0>(t, arena, d, topo, remap, nt, tiles, st);
     else if (creased) fused_gc<0, 1>(t, arena, d, topo, remap, nt, tiles, st);
     else fused_gc<0, 0>(t, arena, d, topo, remap, nt, tiles, st);
+}
+
+void batch_level_children(const BatchTable &t, char *arena, int d, int remap, int nt, int tiles, hipStream_t st) {
+    if (t.blocks == 0 || t.n == 0) return;
+    const auto run = [&](auto k) {
+        hipLaunchKernelGGL(k, dim3(t.blocks), dim3((unsigned)nt), 0, st, static_cast<const LevelJob *>(t.jobs), t.start,
+                           (int)t.n, d, remap, tiles, arena);
+    };
+    if (nt == 256) run(tiles > 1 ? k_batch_fused<0, 0, 1, 256, 1, 0> : k_batch_fused<0, 0, 1, 256, 0, 0>);
+    else if (nt == 512) run(tiles > 1 ? k_batch_fused<0, 0, 1, 512, 1, 0> : k_batch_fused<0, 0, 1, 512, 0, 0>);
+    else run(tiles > 1 ? k_batch_fused<0, 0, 1, kFusedBlock, 1, 0> : k_batch_fused<0, 0, 1, kFusedBlock, 0, 0>);
 }
 
 void batch_level_vertices(const BatchTable &t, char *arena, int d, int gather, int creased, int scan, int remap,

@@ -99,7 +99,9 @@ struct ccb_Batch {
     BatchTable t_cr[kMaxDepth + 1], t_patch[kMaxDepth + 1], t_def[kMaxDepth + 1];
     BatchTable t_rare[kMaxDepth + 1];   // rare-vertex lists after the scan-0 vertex kernel
     BatchTable t_fused[kMaxDepth + 1], t_vert[kMaxDepth + 1];
-    BatchTable t_points[kMaxDepth + 1];   // points alone, tiles of tile_quads quads
+    // points by tiles of tile_quads quads, and behind tiles of kTileBig the
+    // vertices left, kFarWords mask words per wave
+    BatchTable t_points[kMaxDepth + 1], t_far[kMaxDepth + 1];
     int tile_quads[kMaxDepth + 1] = {};
     AdjLevelTables t_adj[kMaxDepth + 1];   // levels 1 ..
     BatchTable t_adjc_h, t_adjc_e, t_adjc_f, t_adjc_v;   // cage-step adjoint gathers: per edge, face, vertex
@@ -518,7 +520,7 @@ bool ccb_Batch::build_tables() {
         for (int l = 1; l < d; ++l) fused_below = fused_below && cfg[l].kind == 1;
         const bool fused_upto = fused_below && cfg[d].kind == 1;
         std::vector<LevelJob> jobs;
-        std::vector<int64_t> bp, bd, bf, bv, br, bt;
+        std::vector<int64_t> bp, bd, bf, bv, br, bt, bw;
         // tiles of 1024 quads where they are mostly full and fill the chip
         int64_t quads = 0, big = 0;
         for (const Cage &g : cages) {
@@ -571,6 +573,7 @@ bool ccb_Batch::build_tables() {
             bd.push_back(blocks_of(blocks_of(blocks_of(g.n.H[d], 64), kDeferGroup), 4));
             bf.push_back(blocks_of(g.n.H[d], (int64_t)cfg[d].fb * cfg[d].ft));
             bt.push_back(blocks_of(g.n.F[d], tile_quads[d]));
+            bw.push_back(j.rare_blocks + blocks_of(blocks_of(blocks_of(g.n.H[d], 64), kFarWords), 4));
             br.push_back(j.rare_cap > 0 ? blocks_of(j.rare_cap) : 0);
             bv.push_back(cfg[d].scan == 0 ? j.rare_blocks + blocks_of(blocks_of(blocks_of(g.n.H[d], 64), kOwnerWords), 4)
                                           : blocks_of(g.n.H[d], 256 * cfg[d].scan));
@@ -581,6 +584,7 @@ bool ccb_Batch::build_tables() {
         tb.add(t_vert[d], jobs, bv);
         tb.add(t_rare[d], jobs, br);
         tb.add(t_points[d], jobs, bt);
+        if (tile_quads[d] == kTileBig) tb.add(t_far[d], jobs, bw);
     }
     if (adj_arena) {   // adjoint steps d+1 -> d, d = 0 the cage step
         for (int d = 0; d < Dmax; ++d) {
@@ -730,8 +734,14 @@ void ccb_Batch::record_forward(int32_t steps, hipStream_t st) {
             timed_launch("level_deferred", d, st,
                          [&] { batch_level_deferred(t_def[d], arena, d, gather, creased, st); });
         } else {
-            // points alone, with the owner bits of an earlier pass: the tile kernel
-            const int tiles = !topo && d >= 2 && own_done && cfg[d].scan == 0 ? 1 : 0;
+            // the tile kernel: for points alone with the owner bits of an
+            // earlier pass, and behind the children of a large level
+            const bool masked = d >= 2 && cfg[d].scan == 0;
+            const bool split = topo && masked && tile_quads[d] == kTileBig;
+            const int tiles = split || (!topo && masked && own_done) ? 1 : 0;
+            if (split) timed_launch("level_fused", d, st, [&] {
+                batch_level_children(t_fused[d], arena, d, remap, cfg[d].fb, cfg[d].ft, st);
+            });
             if (tiles) timed_launch("level_points", d, st, [&] {
                 batch_level_points(t_points[d], arena, d, gather, creased, remap, tile_quads[d], st);
             });
@@ -741,7 +751,9 @@ void ccb_Batch::record_forward(int32_t steps, hipStream_t st) {
                                                cfg[d].ft, st);
                          });
             timed_launch("level_vertices", d, st, [&] {
-                batch_level_vertices(t_vert[d], arena, d, gather, creased, cfg[d].scan, remap, cfg[d].vw, tiles, st);
+                const bool big = tiles && tile_quads[d] == kTileBig;
+                batch_level_vertices(big ? t_far[d] : t_vert[d], arena, d, gather, creased, cfg[d].scan, remap,
+                                     cfg[d].vw, big ? kFarWords : tiles, st);
                 if (cfg[d].scan == 0) batch_level_vertices_rare(t_rare[d], arena, d, gather, creased, st);
             });
         }

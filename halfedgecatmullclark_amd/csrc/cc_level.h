@@ -174,7 +174,7 @@ __device__ __forceinline__ void level_fused_block(const FusedArgs &a, const DCag
     __shared__ int4 stage[kStaged ? kStageInt4 * NT : 1];
     __shared__ P3 spts[POINTS ? NT : 1];
     __shared__ LevelTab stab;   // for the owner test (read after the block's barrier)
-    if (POINTS && a.owner_mask) lds_fill(stab, tb);
+    if (a.owner_mask) lds_fill(stab, tb);
     if (POINTS && a.rare && lb == 0 && threadIdx.x == 0) a.rare[0] = 0;
     const int32_t base = (int32_t)(lb * NT);   // NT threads per block, one tile of NT halfedges
     const int32_t h = base + (int32_t)threadIdx.x;
@@ -299,8 +299,20 @@ __device__ __forceinline__ void level_fused_block(const FusedArgs &a, const DCag
             *at32(a.erep + (tb.R[d + 1] + (base >> 4)), threadIdx.x >> 4) = ((uint64_t)hi << 32) | lo;
     }
 
-    if (!POINTS) return;
-    if (!kStaged) __syncthreads();
+    // One bit per halfedge: is it the representative of its vertex?  (The
+    // face vertices born at this level, d >= 2, whose representatives are the
+    // children 2 of a quad's first halfedge, h % 16 = 2, leave no bit: they
+    // are finished without the vertex kernel.)
+    const auto owner_bits = [&]() {
+        const bool skip = d >= 2 && (h & 15) == 2;
+        const uint64_t m = __ballot(live && !skip && owner_test(h, x.z, d, cg, stab, a.erep_read ? a.erep : nullptr));
+        if ((threadIdx.x & 63u) == 0 && live) *at32(a.owner_mask + (base >> 6), threadIdx.x >> 6) = m;
+    };
+    if (!kStaged && (POINTS || a.owner_mask)) __syncthreads();
+    if (!POINTS) {
+        if (a.owner_mask) owner_bits();
+        return;
+    }
     if (!kSides) {
         v1 = P3{quad_relf<kQuadNext>(P.x), quad_relf<kQuadNext>(P.y), quad_relf<kQuadNext>(P.z)};
         F = face_rule(quad_bcast3<0>(P), quad_bcast3<1>(P), quad_bcast3<2>(P), quad_bcast3<3>(P), GATHER);
@@ -311,22 +323,12 @@ __device__ __forceinline__ void level_fused_block(const FusedArgs &a, const DCag
         level_fused_points<GATHER, CREASED, kSides>(a, h, x, P, v1, F, mine, owner, twin_here, base, spts, g2, g3, s,
                                                     Ev);
     if (a.owner_mask) {
-        // the face vertices born at this level are finished here: their
-        // representatives (children 2 of a quad's first halfedge, h % 16 = 2)
-        // leave no bit for the vertex kernel
-        const bool face_here = d >= 2;
-        if (face_here) face_vertex_in_row<GATHER, CREASED>(a, tb, d, h, base, live, P, F, Ev);
-        // one bit per halfedge: is it the representative of its vertex?  Last,
-        // so that the cage lookups of a few lanes overlap the wave's stores
-        if (a.owner_write) {
-            const bool skip = face_here && (h & 15) == 2;
-            const uint64_t m =
-                __ballot(live && !skip && owner_test(h, x.z, d, cg, stab, a.erep_read ? a.erep : nullptr));
-            if ((threadIdx.x & 63u) == 0 && live) *at32(a.owner_mask + (base >> 6), threadIdx.x >> 6) = m;
-        }
+        if (d >= 2) face_vertex_in_row<GATHER, CREASED>(a, tb, d, h, base, live, P, F, Ev);
+        // the bits last, so that the cage lookups of a few lanes overlap the
+        // wave's stores
+        if (a.owner_write) owner_bits();
     }
 }
-
 
 // Vertex points with owners compacted per block: a block scans
 // 256 * SCAN halfedges, collects the representatives in LDS, then every

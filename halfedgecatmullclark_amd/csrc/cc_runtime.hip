@@ -395,26 +395,35 @@ void ccd_Subd::level_fused(int d, int32_t steps, int topo, int uvMode, P3 *point
         a.erep_read = d >= 2 && below ? 1 : 0;
         a.erep_write = d + 1 <= D - 2 && (d == 1 || erep_valid[d]) ? 1 : 0;
     }
-    // points alone, with the owner bits of an earlier pass: the tile kernel,
-    // which marks the vertices it leaves
-    const bool tiles = a.owner_mask && !topo && uvMode == 0 && d >= 2 && own_valid[d];
-    if (tiles) {
-        a.own_in = a.owner_mask;
-        a.far = far_masks + own_off[d];
-        a.par = he + n.offH[d - 1];
-        a.pV = (int32_t)n.V[d - 1]; a.pF = (int32_t)n.F[d - 1]; a.pE = (int32_t)n.E[d - 1];
-        launch_timed("level_points", n.H[d], st, [&] { launch_level_points(a, gather, creased, st); });
-    } else if (topo || uvMode == 1 || pts_) {
-        launch_timed(pts_ ? (topo ? "level_fused" : "level_points") : "level_fused", n.H[d], st,
+    // Points by the tile kernel, which marks the vertices it leaves: of a
+    // points-only pass with the owner bits of an earlier one, and of a large
+    // level (kTileBigFrom) after a kernel for the children and owner bits.
+    // The fused kernel reads the records once less, but its vertices' points
+    // all come back from memory: level 7 of the 64 x 32 torus 2425 + 646 us,
+    // children, tiles and far vertices 1775 + 596 + 277; at 2.1 M halfedges,
+    // where it begins, 46 + 14 against 33 + 12 + 10, and below that the third
+    // launch costs more than it saves.
+    const bool split = a.owner_mask && topo && d >= 2 && n.F[d] >= kTileBigFrom;
+    const bool tiles = split || (a.owner_mask && !topo && uvMode == 0 && d >= 2 && own_valid[d]);
+    const bool fused_points = pts_ && !tiles;
+    if (topo || uvMode == 1 || fused_points) {
+        launch_timed(fused_points && !topo ? "level_points" : "level_fused", n.H[d], st,
                      [&] {
-                         launch_level_fused(a, c, tab, d, gather, creased, topo, uvMode, pts_, opt_store, cfg[d].fb,
-                                            cfg[d].ft, st);
+                         launch_level_fused(a, c, tab, d, gather, creased, topo, uvMode, fused_points, opt_store,
+                                            cfg[d].fb, cfg[d].ft, st);
                      });
         if (a.erep_write) {
             erep_valid[d + 1] = true;
             if (d == 1) erep_valid[1] = true;
         }
         if (a.owner_mask) own_valid[d] = true;
+    }
+    if (tiles) {
+        a.own_in = a.owner_mask;
+        a.far = far_masks + own_off[d];
+        a.par = he + n.offH[d - 1];
+        a.pV = (int32_t)n.V[d - 1]; a.pF = (int32_t)n.F[d - 1]; a.pE = (int32_t)n.E[d - 1];
+        launch_timed("level_points", n.H[d], st, [&] { launch_level_points(a, gather, creased, st); });
     }
     if (pts_) {
         launch_timed("level_vertices", n.H[d], st, [&] {
