@@ -103,6 +103,7 @@ struct ccb_Batch {
     // vertices left, kFarWords mask words per wave
     BatchTable t_points[kMaxDepth + 1], t_far[kMaxDepth + 1];
     int tile_quads[kMaxDepth + 1] = {};
+    bool tile_split[kMaxDepth + 1] = {};   // a full refinement takes them too (kSplitFrom)
     AdjLevelTables t_adj[kMaxDepth + 1];   // levels 1 ..
     BatchTable t_adjc_h, t_adjc_e, t_adjc_f, t_adjc_v;   // cage-step adjoint gathers: per edge, face, vertex
     bool all_rings = true;                     // every cage has its ring lists
@@ -529,6 +530,7 @@ bool ccb_Batch::build_tables() {
             big += blocks_of(g.n.F[d], kTileBig);
         }
         tile_quads[d] = quads >= kTileBigFrom && 4 * quads >= 3 * kTileBig * big ? kTileBig : kTileSmall;
+        tile_split[d] = tile_quads[d] == kTileBig && quads >= kSplitFrom;
         for (int i = 0; i < N; ++i) {
             const Cage &g = cages[i];
             if (g.D <= d) continue;
@@ -737,7 +739,7 @@ void ccb_Batch::record_forward(int32_t steps, hipStream_t st) {
             // the tile kernel: for points alone with the owner bits of an
             // earlier pass, and behind the children of a large level
             const bool masked = d >= 2 && cfg[d].scan == 0;
-            const bool split = topo && masked && tile_quads[d] == kTileBig;
+            const bool split = topo && masked && tile_split[d];
             const int tiles = split || (!topo && masked && own_done) ? 1 : 0;
             if (split) timed_launch("level_fused", d, st, [&] {
                 batch_level_children(t_fused[d], arena, d, remap, cfg[d].fb, cfg[d].ft, st);

@@ -18,6 +18,10 @@ constexpr int kFusedBlock = 1024;
 // needs 56 registers: 8 fit without spilling); the autotuner may pick 4 or 6
 constexpr int kVertexWaves = 8;
 
+// Owners per wave of the masked vertex kernel: kOwnerWords mask words of 64
+// halfedges, about a quarter of which represent a vertex.
+constexpr int kOwnerWords = 4;
+
 // The tile kernel (cc_tile.h): quads, and threads, of a tile of a level with
 // F quads.  Large tiles leave fewer vertices to the masked kernel, small ones
 // spread a small level over the chip: at 2.1 M quads 40 us and 18 for the
@@ -26,6 +30,13 @@ constexpr int kVertexWaves = 8;
 // is two tiles of 1024 per CU.
 constexpr int kTileBig = 1024, kTileSmall = 256;
 constexpr int64_t kTileBigFrom = 512 * kTileBig;
+// Quads from which a full refinement writes a level's children and owner bits
+// first and its points by tiles, instead of the fused kernel and a vertex
+// kernel that reads every point back: level 7 of the torus 2425 + 646 us
+// against 1775 + 620 + 276; 0.72 M quads 61 + 38 against 49 + 21 + 15; 0.52 M
+// 46 + 14 against 36 + 12 + 10; 0.58 M of 12-byte records 38 + 15 against 29 +
+// 14 + 10, and one launch more.
+constexpr int64_t kSplitFrom = 640 * 1024;
 // The masked kernel's mask words per wave behind it, where few bits are set:
 // 16 of large levels (at 134 M halfedges 374 us, with 8
 // words 397), else kOwnerWords (at 262 thousand halfedges 11.7 us with 16, 7.4

@@ -368,10 +368,6 @@ __device__ __forceinline__ void level_vertices_compact_block(const FusedArgs &a,
     }
 }
 
-// Owners per wave of the masked vertex kernel: kOwnerWords mask words of 64
-// halfedges, about a quarter of which represent a vertex.
-constexpr int kOwnerWords = 4;
-
 // A marked owner whose ring follows from the child numbering: its vertex
 // point; any other goes to the rare list when there is one, else its waves
 // of rare_vertices have it (no general fan code here, so the kernel keeps

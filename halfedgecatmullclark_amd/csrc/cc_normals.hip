@@ -8,9 +8,10 @@
 // with normalize(v) = v * (1 / sqrt(dot(v, v))), correctly rounded, in the
 // shaders' operation order (built with -ffp-contract=off).
 //
-// Two kernels: one thread per halfedge forms its corner normal from its
-// quad's points (exchanged by DPP within the quad); the vertex normals then
-// walk the ring over the stored corner normals.
+// Two kernels: tile by tile, one thread per quad, the corner normals and the
+// vertex normals of rings that close inside the tile; then the other vertices
+// from the corner normals the first stored.  Corner normals alone, and cages
+// without ring lists, take one thread per halfedge.
 #include <stdio.h>
 
 #include "cc_fan.h"
@@ -115,32 +116,114 @@ struct VertexNormalsFn {
     }
 };
 
-// vertex normals by owner: a block lists the owners among its 1024
-// halfedges in LDS (halfedge order), then each thread finishes one vertex
-__global__ __launch_bounds__(256) void k_vertex_normals_owners(DCage c, LevelTab t, LevelPtrs lp, int d, int32_t H,
-                                                               const P3 *__restrict__ corner, P3 *__restrict__ out) {
-    __shared__ int32_t owners[1024];
-    __shared__ int32_t nown;
-    __shared__ LevelTab st;
-    __shared__ LevelPtrs slp;
-    lds_fill(st, t);
-    lds_fill(slp, lp);
-    const int32_t base = (int32_t)(xcd_block(blockIdx.x, gridDim.x, 1) * 1024u);
-    if (threadIdx.x == 0) nown = 0;
-    __syncthreads();
+// Corner normals, and vertex normals where the ring of four closes inside a
+// tile of N quads (one thread per quad, corner normals in LDS).  Halfedges of
+// other rings leave their corner normal in `corner`, and one of each ring,
+// normal_owner's, a bit in `mask` for k_vertex_normals_far (a vertex born at
+// level 1 leaves one for every child 0, 1 and 2 of its ring: the far kernel
+// asks the cage).
+// Passing every corner normal through memory took 580 + 1298 us at level 7 of
+// the 64 x 32 torus, 134 M halfedges: 1.6 GB written and read back three
+// times over by the vertices' quads in different workgroups; what has to
+// move is the records, the points and the normals, 4.1 GB.
+template <int N>
+__global__ __launch_bounds__(N, 8) void k_normal_tiles(const He *__restrict__ he, const P3 *__restrict__ pts, int32_t F,
+                                                       int d, P3 *__restrict__ corner, uint64_t *__restrict__ mask,
+                                                       P3 *__restrict__ out) {
+    // halfedge h at (h & 3) N + its quad: consecutive lanes, consecutive words
+    __shared__ float sc[3][4 * N];
+    __shared__ uint16_t sr[4 * N];   // twin(prev), kOut outside the tile or on a boundary
+    constexpr int kOut = 0xffff;
+    const int q = (int)threadIdx.x;
+    const int32_t base = (int32_t)(xcd_block(blockIdx.x, gridDim.x, 1) * N), p = base + q;
+    const bool live = p < F;
+    const int32_t g = live ? p : 0;
+    int32_t nx[4];
+    P3 c[4];
+    {
+        int4 x[4];
+        P3 P[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x[k] = he_gld(he, 4 * g + k);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) P[k] = gld(at3(pts, x[k].z));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            nx[k] = x[(k + 3) & 3].x;
+            c[k] = normalize3(cross3(sub3(P[(k + 1) & 3], P[k]), sub3(P[(k + 3) & 3], P[k])));
+        }
+    }
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        const int32_t h = base + k * 256 + (int32_t)threadIdx.x;
-        if (h < H && normal_owner(h, d, c, slp.he)) owners[atomicAdd(&nown, 1)] = h;
+        const int i = k * N + q;
+        const uint32_t o = (uint32_t)((nx[k] >> 2) - base);   // a boundary's -1 >> 2 is no quad of the tile
+        sr[i] = (uint16_t)(live && nx[k] >= 0 && o < (uint32_t)N ? (nx[k] & 3) * N + (int)o : kOut);
+        sc[0][i] = c[k].x;
+        sc[1][i] = c[k].y;
+        sc[2][i] = c[k].z;
     }
     __syncthreads();
-    const int32_t count = nown;
-    const VertexNormalsFn fn{corner, out, c};
-    for (int32_t i = (int32_t)threadIdx.x; i < count; i += 256) {
+    uint32_t nib = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int i = k * N + q;
+        const int r1 = sr[i];
+        const int r2 = r1 != kOut ? sr[r1] : kOut;
+        const int r3 = r2 != kOut ? sr[r2] : kOut;
+        const int r4 = r3 != kOut ? sr[r3] : kOut;
+        if (!live) continue;
+        const int32_t h = 4 * p + k;
+        if (r4 == i && r2 != i) {   // four distinct halfedges, summed in walk order
+            P3 avg = zero3();
+            avg = add(avg, P3{sc[0][r1], sc[1][r1], sc[2][r1]});
+            avg = add(avg, P3{sc[0][r2], sc[1][r2], sc[2][r2]});
+            avg = add(avg, P3{sc[0][r3], sc[1][r3], sc[2][r3]});
+            *at3(out, h) = normalize3(add(c[k], avg));
+        } else {
+            *at3(corner, h) = c[k];
+            const int k2 = 2 * zero_digits(h, d);
+            const int digit = (h >> k2) & 3;
+            const int32_t pp = h >> (k2 + 2);
+            bool mark = false;
+            if (2 * (d - 1) == k2) mark = digit != 3;
+            else if (digit == 2) mark = (pp & 3) == 0;
+            else if (digit == 1) mark = nx[k] < 0 || pp > qprev(nx[k] >> (k2 + 2));
+            nib |= mark ? 1u << k : 0u;
+        }
+    }
+    const uint32_t sh = 4u * (uint32_t)(q & 7);
+    const uint32_t lo = row_or((q & 8) ? 0u : nib << sh);
+    const uint32_t hi = row_or((q & 8) ? nib << sh : 0u);
+    if ((q & 15) == 15 && (p & ~15) < F) mask[p >> 4] = ((uint64_t)hi << 32) | lo;
+}
+
+struct FarNormalsFn {
+    VertexNormalsFn fn;
+    const LevelTab &t;
+    const LevelPtrs &lp;
+    int d;
+    __device__ void operator()(int32_t h) const {
+        if (zero_digits(h, d) == d - 1 && !normal_owner(h, d, fn.c, lp.he)) return;
         Fan f;
-        (void)marked_fan(owners[i], d, c, st, slp.he, f);
+        (void)marked_fan(h, d, fn.c, t, lp.he, f);
         fn(f);
     }
+};
+
+// the vertices k_normal_tiles marked, WORDS mask words per wave
+template <int WORDS>
+__global__ __launch_bounds__(256) void k_vertex_normals_far(DCage c, LevelTab t, LevelPtrs lp, int d, int32_t H,
+                                                            const uint64_t *__restrict__ mask,
+                                                            const P3 *__restrict__ corner, P3 *__restrict__ out) {
+    __shared__ LevelTab st;
+    __shared__ LevelPtrs slp;
+    __shared__ uint16_t list[4][64 * WORDS];
+    lds_fill(st, t);
+    lds_fill(slp, lp);
+    __syncthreads();
+    const int32_t wave = (int32_t)(xcd_block(blockIdx.x, gridDim.x, 1) * 4 + (threadIdx.x >> 6));
+    mask_group<WORDS>(mask, wave * WORDS, (H + 63) >> 6, list[threadIdx.x >> 6],
+                      FarNormalsFn{{corner, out, c}, st, slp, d});
 }
 
 // vertex normals from the corner normals, one walk per halfedge
@@ -169,18 +252,33 @@ bool ccd_Subd::normals(P3 *out, bool smooth, hipStream_t st) {
     const P3 *lpts = pts + n.offV[D];
     P3 *corner = out;
     if (smooth) {
-        if (!nrm_tmp && hip_failed(hipMalloc(&nrm_tmp, sizeof(P3) * (size_t)H), "hipMalloc(corner normals)"))
+        // corner normals, and the tile kernel's bits behind them
+        if (!nrm_tmp && hip_failed(hipMalloc(&nrm_tmp, sizeof(P3) * (size_t)H + sizeof(uint64_t) * (size_t)((H + 63) / 64)),
+                                   "hipMalloc(corner normals)"))
             return false;
         corner = nrm_tmp;
     }
-    hipLaunchKernelGGL(k_corner_normals, dim3(blocks_for(H)), dim3(256), 0, st, lhe, lpts, (int32_t)H, corner);
     if (smooth && D >= 1 && rings_ok) {
-        // by owner: each ring's corner normals read once
-        hipLaunchKernelGGL(k_vertex_normals_owners, dim3((unsigned)((H + 1023) / 1024)), dim3(256), 0, st,
-                           cage_view(nullptr), tab, level_ptrs(), D, (int32_t)H, (const P3 *)corner, out);
-    } else if (smooth) {
-        hipLaunchKernelGGL(k_vertex_normals, dim3(blocks_for(H)), dim3(256), 0, st, lhe, (const P3 *)corner,
-                           (int32_t)H, out);
+        uint64_t *mask = reinterpret_cast<uint64_t *>(nrm_tmp + H);   // H is a multiple of 4: 8-byte aligned
+        const int32_t F = (int32_t)(H / 4);
+        const bool big = F >= kTileBigFrom;
+        const int64_t words = (H + 63) / 64, tile = big ? kTileBig : kTileSmall, per = 4 * (big ? kFarWords : kOwnerWords);
+        const dim3 grid((unsigned)((F + tile - 1) / tile)), far((unsigned)((words + per - 1) / per));
+        const auto tiles = [&](auto k) {
+            hipLaunchKernelGGL(k, grid, dim3((unsigned)tile), 0, st, lhe, lpts, F, D, corner, mask, out);
+        };
+        const auto rest = [&](auto k) {
+            hipLaunchKernelGGL(k, far, dim3(256), 0, st, cage_view(nullptr), tab, level_ptrs(), D, (int32_t)H,
+                               (const uint64_t *)mask, (const P3 *)corner, out);
+        };
+        tiles(big ? k_normal_tiles<kTileBig> : k_normal_tiles<kTileSmall>);
+        if (big) rest(k_vertex_normals_far<kFarWords>);
+        else rest(k_vertex_normals_far<kOwnerWords>);
+    } else {
+        hipLaunchKernelGGL(k_corner_normals, dim3(blocks_for(H)), dim3(256), 0, st, lhe, lpts, (int32_t)H, corner);
+        if (smooth)
+            hipLaunchKernelGGL(k_vertex_normals, dim3(blocks_for(H)), dim3(256), 0, st, lhe, (const P3 *)corner,
+                               (int32_t)H, out);
     }
     return !hip_failed(hipGetLastError(), "halfedge normals");
 }

@@ -397,13 +397,8 @@ void ccd_Subd::level_fused(int d, int32_t steps, int topo, int uvMode, P3 *point
     }
     // Points by the tile kernel, which marks the vertices it leaves: of a
     // points-only pass with the owner bits of an earlier one, and of a large
-    // level (kTileBigFrom) after a kernel for the children and owner bits.
-    // The fused kernel reads the records once less, but its vertices' points
-    // all come back from memory: level 7 of the 64 x 32 torus 2425 + 646 us,
-    // children, tiles and far vertices 1775 + 596 + 277; at 2.1 M halfedges,
-    // where it begins, 46 + 14 against 33 + 12 + 10, and below that the third
-    // launch costs more than it saves.
-    const bool split = a.owner_mask && topo && d >= 2 && n.F[d] >= kTileBigFrom;
+    // level after a kernel for the children and owner bits.
+    const bool split = a.owner_mask && topo && d >= 2 && n.F[d] >= kSplitFrom;
     const bool tiles = split || (a.owner_mask && !topo && uvMode == 0 && d >= 2 && own_valid[d]);
     const bool fused_points = pts_ && !tiles;
     if (topo || uvMode == 1 || fused_points) {
