@@ -130,9 +130,11 @@ template <int N>
 __global__ __launch_bounds__(N, 8) void k_normal_tiles(const He *__restrict__ he, const P3 *__restrict__ pts, int32_t F,
                                                        int d, P3 *__restrict__ corner, uint64_t *__restrict__ mask,
                                                        P3 *__restrict__ out) {
-    // halfedge h at (h & 3) N + its quad: consecutive lanes, consecutive words
-    __shared__ float sc[3][4 * N];
-    __shared__ uint16_t sr[4 * N];   // twin(prev), kOut outside the tile or on a boundary
+    // Halfedge k of quad q at k (N + 16) + q: without bank conflicts by quad
+    // (written) and by halfedge (read).
+    constexpr int kRow = N + 16;
+    __shared__ float sc[3][4 * kRow];
+    __shared__ uint16_t sr[4 * kRow];   // twin(prev), kOut outside the tile or on a boundary
     constexpr int kOut = 0xffff;
     const int q = (int)threadIdx.x;
     const int32_t base = (int32_t)(xcd_block(blockIdx.x, gridDim.x, 1) * N), p = base + q;
@@ -155,46 +157,50 @@ __global__ __launch_bounds__(N, 8) void k_normal_tiles(const He *__restrict__ he
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        const int i = k * N + q;
+        const int i = k * kRow + q;
         const uint32_t o = (uint32_t)((nx[k] >> 2) - base);   // a boundary's -1 >> 2 is no quad of the tile
-        sr[i] = (uint16_t)(live && nx[k] >= 0 && o < (uint32_t)N ? (nx[k] & 3) * N + (int)o : kOut);
+        sr[i] = (uint16_t)(live && nx[k] >= 0 && o < (uint32_t)N ? (nx[k] & 3) * kRow + (int)o : kOut);
         sc[0][i] = c[k].x;
         sc[1][i] = c[k].y;
         sc[2][i] = c[k].z;
     }
     __syncthreads();
-    uint32_t nib = 0;
+    // now a lane per halfedge, so that a wave's stores are consecutive
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        const int i = k * N + q;
+        const int l = k * N + q;
+        const int32_t h = 4 * base + l;
+        const int i = (l & 3) * kRow + (l >> 2);
         const int r1 = sr[i];
         const int r2 = r1 != kOut ? sr[r1] : kOut;
         const int r3 = r2 != kOut ? sr[r2] : kOut;
         const int r4 = r3 != kOut ? sr[r3] : kOut;
-        if (!live) continue;
-        const int32_t h = 4 * p + k;
-        if (r4 == i && r2 != i) {   // four distinct halfedges, summed in walk order
+        const bool in = (h >> 2) < F, ring = in && r4 == i && r2 != i;   // four distinct halfedges
+        const P3 cn = P3{sc[0][i], sc[1][i], sc[2][i]};
+        bool mark = false;
+        if (ring) {   // summed in walk order
             P3 avg = zero3();
             avg = add(avg, P3{sc[0][r1], sc[1][r1], sc[2][r1]});
             avg = add(avg, P3{sc[0][r2], sc[1][r2], sc[2][r2]});
             avg = add(avg, P3{sc[0][r3], sc[1][r3], sc[2][r3]});
-            *at3(out, h) = normalize3(add(c[k], avg));
-        } else {
-            *at3(corner, h) = c[k];
+            *at3(out, h) = normalize3(add(cn, avg));
+        } else if (in) {
+            *at3(corner, h) = cn;
             const int k2 = 2 * zero_digits(h, d);
             const int digit = (h >> k2) & 3;
             const int32_t pp = h >> (k2 + 2);
-            bool mark = false;
-            if (2 * (d - 1) == k2) mark = digit != 3;
-            else if (digit == 2) mark = (pp & 3) == 0;
-            else if (digit == 1) mark = nx[k] < 0 || pp > qprev(nx[k] >> (k2 + 2));
-            nib |= mark ? 1u << k : 0u;
+            if (2 * (d - 1) == k2) {
+                mark = digit != 3;
+            } else if (digit == 2) {
+                mark = (pp & 3) == 0;
+            } else if (digit == 1) {   // the parent's twin, from twin(prev(h)) = 4 next(twin) + 3
+                const int32_t nxt = he[qprev(h)].twin;
+                mark = nxt < 0 || pp > qprev(nxt >> (k2 + 2));
+            }
         }
+        const uint64_t m = __ballot(mark);
+        if ((q & 63) == 0 && in) mask[h >> 6] = m;
     }
-    const uint32_t sh = 4u * (uint32_t)(q & 7);
-    const uint32_t lo = row_or((q & 8) ? 0u : nib << sh);
-    const uint32_t hi = row_or((q & 8) ? nib << sh : 0u);
-    if ((q & 15) == 15 && (p & ~15) < F) mask[p >> 4] = ((uint64_t)hi << 32) | lo;
 }
 
 struct FarNormalsFn {
