@@ -49,8 +49,9 @@ struct LevelJob {
     LevelTab t;
 };
 
-// a range of n floats copied from src + src_off to dst + dst_off, the base
-// pointers being launch arguments
+// a range of n points copied from src + src_off to dst + dst_off, the base
+// pointers being launch arguments; a workgroup takes 256 * kCopyPer
+constexpr int kCopyPer = 4;
 struct SpanJob {
     int64_t src_off, dst_off, n;
 };

@@ -61,11 +61,20 @@ struct OpZeroCageVertices {
     }
 };
 
+// Points of a range, kCopyPer per thread with every load before the first
+// store (128 cages, 243 MB: one float per thread 188 us, this 94).
 struct OpCopy {
-    const float *src;
-    float *dst;
+    const P3 *src;
+    P3 *dst;
     __device__ void operator()(const SpanJob &J, int64_t i) const {
-        if (i < J.n) dst[J.dst_off + i] = src[J.src_off + i];
+        const int64_t first = (i >> 8) * (256 * kCopyPer) + (i & 255);
+        P3 p[kCopyPer];
+#pragma unroll
+        for (int j = 0; j < kCopyPer; ++j)
+            if (first + 256 * j < J.n) p[j] = src[J.src_off + first + 256 * j];
+#pragma unroll
+        for (int j = 0; j < kCopyPer; ++j)
+            if (first + 256 * j < J.n) dst[J.dst_off + first + 256 * j] = p[j];
     }
 };
 
@@ -294,7 +303,7 @@ void batch_zero_cage_vertices(const BatchTable &t, hipStream_t st) {
 }
 
 void batch_copy(const BatchTable &t, const float *src, float *dst, hipStream_t st) {
-    launch_batch<SpanJob>(t, OpCopy{src, dst}, st);
+    launch_batch<SpanJob>(t, OpCopy{reinterpret_cast<const P3 *>(src), reinterpret_cast<P3 *>(dst)}, st);
 }
 
 void batch_level_patch(const BatchTable &t, char *arena, int d, int gather, int creased, int topo, int nt, int hpt,

@@ -496,8 +496,8 @@ bool ccb_Batch::build_tables() {
         std::vector<int64_t> b(N);
         for (int i = 0; i < N; ++i) {
             const Cage &g = cages[i];
-            jobs[i] = {3 * (g.o_pts + g.n.offV[g.D]), 3 * g.o_fin, 3 * g.n.V[g.D]};
-            b[i] = blocks_of(jobs[i].n);
+            jobs[i] = {g.o_pts + g.n.offV[g.D], g.o_fin, g.n.V[g.D]};
+            b[i] = blocks_of(jobs[i].n, 256 * kCopyPer);
         }
         tb.add(t_fin, jobs, b);
     }
