@@ -52,7 +52,7 @@ HBM_PEAK_GBS = 8000.0
 METRIC = "refined halfedges/s + HBM GB/s at depth 8; fwd+adjoint and batched vs plain"
 
 
-def level_bytes(n, d, D=None, owner_bits=False):
+def level_bytes(n, d, D=None, owner_bits=False, points=True):
     """Algorithmic bytes of the fused level kernel d -> d+1: each input read
     once and each output written once.  Reads: the level-d halfedge records
     (16 B), level-d points (12 B), level-d creases (12 B); writes: the four
@@ -62,9 +62,12 @@ def level_bytes(n, d, D=None, owner_bits=False):
     edge-representative bits and, from level 2 on, writes the vertex points
     of the face vertices born at level d (12 B each, one per parent-level
     face); on levels d + 1 <= D - 2 it reads level d's bits and writes level
-    d+1's (one bit per halfedge each)."""
-    b = 16 * n["H"][d] + 12 * n["V"][d] + 12 * n["C"][d] + 64 * n["H"][d] + 12 * (n["F"][d] + n["E"][d])
-    if owner_bits and d >= 2:
+    d+1's (one bit per halfedge each).  points=False: the children and bits
+    alone, where the tile kernel follows for the points."""
+    b = 16 * n["H"][d] + 64 * n["H"][d]
+    if points:
+        b += 12 * n["V"][d] + 12 * n["C"][d] + 12 * (n["F"][d] + n["E"][d])
+    if points and owner_bits and d >= 2:
         b += 12 * n["F"][d - 1]
     if D is not None and D >= 4:
         if owner_bits:
@@ -423,12 +426,15 @@ def main():
 
     # dominant kernel: largest mean duration among the launches of one step;
     # the per-level kernels run in level order, each level starting with its
-    # fused or patch-local kernel
-    labelled, d = [], 0
+    # fused or patch-local kernel (a level's points may follow its children)
+    labelled, d, split, prev = [], 0, set(), None
     for (i, nm) in sorted(kern):
-        if nm in ("level_fused", "level_points", "level_patch"):
+        if nm == "level_points" and prev == "level_fused":
+            split.add(d)
+        elif nm in ("level_fused", "level_points", "level_patch"):
             d += 1
         labelled.append(((i, nm), d))
+        prev = nm
     ((idx, name), level) = max(labelled, key=lambda kv: sum(kern[kv[0]]) / len(kern[kv[0]]))
     # every launch of one step: (name, level, mean ms), the level a kernel
     # reads (0: cage step and creases)
@@ -436,7 +442,7 @@ def main():
     durs = kern[(idx, name)]
     mean_ms = sum(durs) / len(durs)
     if name == "level_fused":
-        nbytes = level_bytes(n, level, D, owner_bits=level_cfg[level - 1]["scan"] == 0)
+        nbytes = level_bytes(n, level, D, owner_bits=level_cfg[level - 1]["scan"] == 0, points=level not in split)
     elif name == "level_vertices":
         nbytes = vertex_kernel_bytes(n, level)
     elif name == "level_patch":
@@ -450,7 +456,9 @@ def main():
     prof = os.path.join(ROOT, "profiles", "traffic_torus64x32_d8.json")
     if os.path.exists(prof):
         try:
-            traffic = json.load(open(prof)).get("kernels", {}).get(f"{name}@{level}", {}).get("traffic_bytes")
+            traffic = json.load(open(prof)).get("kernels", {}).get(
+                f"level_children@{level}" if name == "level_fused" and level in split else f"{name}@{level}",
+                {}).get("traffic_bytes")
         except Exception:
             traffic = None
 

@@ -348,8 +348,9 @@ int32_t ccd_HalfedgeNormals(ccd_Subd *subd, float *devNormals, int32_t smooth, v
  *                      takes the vertex representatives the fused kernel
  *                      marked in a bit mask; 2, 4 or 8 scans that many
  *                      halfedges per thread for them
- *   CCD_OPT_ADJ_VERTEX the adjoint's two vertex passes run one thread per
- *                      vertex on levels with at most this many vertices
+ *   CCD_OPT_ADJ_VERTEX the adjoint's vertex passes (the parameters; the
+ *                      gathers of a cage without a rare-vertex table) run
+ *                      one thread per vertex on levels with at most this many
  *                      (default 1048576), else over the vertex owners in
  *                      halfedge order; both give the same bits
  *   CCD_OPT_FUSED_BLOCK threads (parent halfedges) per workgroup of the fused
