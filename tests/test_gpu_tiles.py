@@ -85,3 +85,26 @@ def test_points_not_finite(rule):
     want, got = tiled(c, 4, rule)
     for g in got:
         assert_bytes_equal(canonical(g), canonical(want), "not finite")
+
+
+@pytest.mark.parametrize("name,cage,depth",
+                         [("torus4x4_1", C.torus(4, 4), 1), ("torus5x3", C.torus(5, 3), 3), ("torus4x4", C.torus(4, 4), 3),
+                          ("grid1x1", grid(1, 1), 5), ("grid5x3", grid(5, 3), 4), ("irregular", C.irregular(1, seed=3), 4),
+                          ("torus65x33", C.torus(65, 33), 5)], ids=lambda x: x if isinstance(x, str) else "")
+def test_normal_tiles(name, cage, depth):
+    """vertex normals of the finest level, the oracle's bytes: one tile and
+    part of one, levels of 1024-quad tiles with a remainder (torus65x33),
+    boundaries, and vertices that are not regular"""
+    import torch
+    from halfedgecatmullclark_amd import capi
+    from oracle import oracle as O
+    st = torch.cuda.current_stream().cuda_stream
+    ds = capi.DeviceSubd(cage, depth)
+    ds.refine(15, st)
+    H = ds.n["H"][depth]
+    out = torch.full((H, 3), 7.0, device="cuda")
+    ds.halfedge_normals(out.data_ptr(), True, st)
+    got = out.cpu().numpy()
+    want = O.halfedge_normals(ds.download(), depth, True)
+    ds.close()
+    assert_bytes_equal(got, np.ascontiguousarray(want).reshape(got.shape), name)
