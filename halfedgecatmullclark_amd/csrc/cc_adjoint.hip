@@ -813,7 +813,7 @@ __device__ __forceinline__ void adj_vertices_rare(const AdjArgs<T> &a, const DCa
     if (i >= n) return;
     Fan f;
     const int32_t v = marked_fan(a.rare[1 + i], d, c, st, slp.he, f);
-    adj_gather_fan<T, CREASED>(a, c, st, d, f, v);
+    if (v >= 0) adj_gather_fan<T, CREASED>(a, c, st, d, f, v);
 }
 
 // ---- the cage step (level 0 -> 1) -----------------------------------------------

@@ -576,8 +576,8 @@ __device__ __forceinline__ bool marked_ring_fan(int32_t h, int d, const DCage &c
     return true;
 }
 
-// The fan and vertex ID of a level-d halfedge h known to be the
-// representative of its vertex (marked by the fused kernel).  A face or edge
+// The fan and vertex ID of a level-d halfedge h that represents its vertex
+// (marked by the fused kernel); -1, and no fan, when it does not.  A face or edge
 // vertex born at level lvl >= 2 takes its ID from the child numbering
 // (child 2 of p: V + face(p), child 1: V + F + edge(p), parent-level counts),
 // so only an edge vertex reads one record, its parent's (twin and edge);
@@ -617,8 +617,7 @@ __device__ __forceinline__ int32_t marked_fan(int32_t h, int d, const DCage &c, 
         return (int32_t)(t.V[lvl - 1] + t.F[lvl - 1]) + x.y;
     }
     const int32_t v = levels[d][h].vert;
-    owner_fan(h, v, d, c, t, levels, f);
-    return v;
+    return owner_fan(h, v, d, c, t, levels, f) ? v : -1;
 }
 
 // The owners of level-d vertices among 256 * SCAN halfedges (structural
@@ -652,7 +651,7 @@ __device__ __forceinline__ void owners_block(int32_t H, int d, const DCage &c, c
         } else {
             Fan f;
             const int32_t v = marked_fan(owners[i], d, c, st, slp.he, f);
-            fn(st, f, v);
+            if (v >= 0) fn(st, f, v);
         }
     }
 }

@@ -63,9 +63,11 @@ struct FusedArgs {
     uint64_t *owner_mask;
     // when set: the masked vertex kernel handles the vertices whose ring
     // follows from the child numbering and appends the others (cage-level
-    // and boundary fans; a cage with a rare-vertex table needs no list) to this list, rare[0] their count (cleared by the
-    // fused kernel), rare[1 .. rare_cap] their representatives; the rare
-    // kernel then finishes them
+    // and boundary fans; a cage with a rare-vertex table needs no list) to
+    // this list, rare[0] their count, rare[1 .. rare_cap] their
+    // representatives; the rare kernel then finishes them.  The list holds
+    // one level's: the kernel before the masked one, fused or tile, clears
+    // the count
     int32_t *rare;
     int32_t rare_cap;
     // Edge-representative bits of levels 1 .. (word offsets LevelTab::R):

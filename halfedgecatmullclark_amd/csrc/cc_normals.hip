@@ -211,8 +211,7 @@ struct FarNormalsFn {
     __device__ void operator()(int32_t h) const {
         if (zero_digits(h, d) == d - 1 && !normal_owner(h, d, fn.c, lp.he)) return;
         Fan f;
-        (void)marked_fan(h, d, fn.c, t, lp.he, f);
-        fn(f);
+        if (marked_fan(h, d, fn.c, t, lp.he, f) >= 0) fn(f);
     }
 };
 

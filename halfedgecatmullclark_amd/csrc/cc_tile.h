@@ -75,6 +75,9 @@ __device__ __forceinline__ void point_tile(const FusedArgs &a, uint32_t tile) {
     __shared__ int32_t nfar;
     const int q = (int)threadIdx.x;
     if (q == 0) nfar = 0;
+    // the masked kernel that follows appends; on this path no fused kernel
+    // with points has emptied the list of the level before
+    if (a.rare && tile == 0 && q == 0) a.rare[0] = 0;
     const int32_t base = (int32_t)(tile * N), p = base + q;
     const auto here = [&](int32_t r) { return (uint32_t)(r - base) < (uint32_t)N; };
     const auto sharp = [&](int32_t e) {
