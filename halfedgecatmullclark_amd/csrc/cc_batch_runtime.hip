@@ -107,6 +107,7 @@ struct ccb_Batch {
     AdjLevelTables t_adj[kMaxDepth + 1];   // levels 1 ..
     BatchTable t_adjc_h, t_adjc_e, t_adjc_f, t_adjc_v;   // cage-step adjoint gathers: per edge, face, vertex
     bool all_rings = true;                     // every cage has its ring lists
+    bool all_simple = true;                    // RareTable::simple of every cage
     // the adjoint's finest steps read the caller's gradient (its address in
     // the adjoint arena's first bytes); false when a cage is refined once:
     // its cage step updates the finest gradient in place, so every call
@@ -291,6 +292,7 @@ bool ccb_Batch::create(const cc_Mesh *const *meshes, const int32_t *depths, int3
         g.o_e0 = tot_e0; tot_e0 += g.E0;
         g.o_f0 = tot_f0; tot_f0 += g.F0;
         all_rings = all_rings && r.ok;
+        all_simple = all_simple && rt.simple;
         if (r.ok) {
             auto put = [&](const std::vector<int32_t> &v) {
                 const int64_t o = (int64_t)rings_host.size();
@@ -738,7 +740,7 @@ void ccb_Batch::record_forward(int32_t steps, hipStream_t st) {
         } else {
             // the tile kernel: for points alone with the owner bits of an
             // earlier pass, and behind the children of a large level
-            const bool masked = d >= 2 && cfg[d].scan == 0;
+            const bool masked = all_simple && d >= 2 && cfg[d].scan == 0;
             const bool split = topo && masked && tile_split[d];
             const int tiles = split || (!topo && masked && own_done) ? 1 : 0;
             if (split) timed_launch("level_fused", d, st, [&] {

@@ -107,14 +107,16 @@ inline void build_cage_rings(const cc_Mesh *m, CageRings &r) {
 
 // The rare-vertex table of a cage (RareView) as one run of int32s: items |
 // entries | boundary halfedges, item and boundary records of four ints,
-// entries of two.  `ok` is false when the cage does not fit it (walks that do
-// not close, links that contradict each other, a vertex, edge or face with
-// halfedges outside its one ring, a fan of more than 64 entries): its rare
-// vertices then go through the rare list.
+// entries of two.  `simple`: every walk closes, links agree, and every vertex,
+// edge and face has all its halfedges in its one ring; a tile pass, which
+// finishes a vertex from whichever ring closes inside a tile, takes no other
+// cage (of two rings at a vertex, both might write it).  `ok` is false when
+// the cage does not fit the table (not simple, or a fan of more than 64
+// entries): its rare vertices then go through the rare list.
 struct RareTable {
     std::vector<int32_t> item, ent, bnd;
     int32_t n4 = 0, n8 = 0, n64 = 0, nb = 0;
-    bool ok = false;
+    bool ok = false, simple = false;
     bool empty() const { return n4 + n8 + n64 + nb == 0; }
     struct Item { int32_t v, first, n, boundary; };
     std::vector<Item> items[3];   // scratch
@@ -122,7 +124,7 @@ struct RareTable {
 };
 
 inline void build_rare_table(const cc_Mesh *m, const CageRings &r, RareTable &t) {
-    t.ok = false;
+    t.ok = t.simple = false;
     t.n4 = t.n8 = t.n64 = t.nb = 0;
     for (std::vector<int32_t> *x : {&t.item, &t.ent, &t.bnd}) x->clear();
     for (auto &x : t.items) x.clear();
@@ -146,11 +148,12 @@ inline void build_rare_table(const cc_Mesh *m, const CageRings &r, RareTable &t)
         }
     }
     if (pairs != E) return;
+    bool fits = true;
     auto add_item = [&](int32_t v, int32_t n, int32_t boundary, size_t first) {
         const int32_t entries = n + boundary;
         const int k = entries <= 4 ? 0 : (entries <= 8 ? 1 : 2);
         t.items[k].push_back({v, (int32_t)(first / 2), n, boundary});
-        return entries <= 64;
+        fits = fits && entries <= 64;
     };
     auto add_ent = [&](int32_t h, int32_t e, bool odd) {
         t.ent.push_back(h);
@@ -174,7 +177,7 @@ inline void build_rare_table(const cc_Mesh *m, const CageRings &r, RareTable &t)
             const int32_t R = r.vring[o + n - 1], p = he[R].prev;
             add_ent(4 * R, 2 * he[p].edge + 1, true);
         }
-        if (!add_item(v, n, boundary ? 1 : 0, first)) return;
+        add_item(v, n, boundary ? 1 : 0, first);
     }
     for (int32_t f = 0; f < F; ++f) {
         const int32_t o = r.foff[f], n = r.foff[f + 1] - o;
@@ -188,8 +191,10 @@ inline void build_rare_table(const cc_Mesh *m, const CageRings &r, RareTable &t)
             const int32_t q = r.fring[o + i], pr = he[q].prev;
             add_ent(4 * q + 2, 2 * E + pr, 4 * q + 2 < 4 * pr + 1);
         }
-        if (!add_item(V + f, n, 0, first)) return;
+        add_item(V + f, n, 0, first);
     }
+    t.simple = true;
+    if (!fits) return;
     for (const auto &group : t.items) {
         const int32_t *p = reinterpret_cast<const int32_t *>(group.data());
         t.item.insert(t.item.end(), p, p + 4 * group.size());

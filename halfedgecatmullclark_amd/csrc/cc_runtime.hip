@@ -139,6 +139,7 @@ bool ccd_Subd::upload_cage(const cc_Mesh *cage, hipStream_t st) {
     build_rare_table(cage, r, rt);
     rare_free = rt.ok && rt.empty();
     rare_on = rt.ok;
+    simple = rt.simple;
     rare_n4 = rt.n4; rare_n8 = rt.n8; rare_n64 = rt.n64; rare_nb = rt.nb;
     if (!rt.ok) {   // the rare-vertex list: cage vertices, cage faces and boundary vertices
         int64_t b0 = 0;
@@ -398,8 +399,9 @@ void ccd_Subd::level_fused(int d, int32_t steps, int topo, int uvMode, P3 *point
     // Points by the tile kernel, which marks the vertices it leaves: of a
     // points-only pass with the owner bits of an earlier one, and of a large
     // level after a kernel for the children and owner bits.
-    const bool split = a.owner_mask && topo && d >= 2 && n.F[d] >= kSplitFrom;
-    const bool tiles = split || (a.owner_mask && !topo && uvMode == 0 && d >= 2 && own_valid[d]);
+    const bool tileable = a.owner_mask && simple && d >= 2;
+    const bool split = tileable && topo && n.F[d] >= kSplitFrom;
+    const bool tiles = split || (tileable && !topo && uvMode == 0 && own_valid[d]);
     const bool fused_points = pts_ && !tiles;
     if (topo || uvMode == 1 || fused_points) {
         launch_timed(fused_points && !topo ? "level_points" : "level_fused", n.H[d], st,

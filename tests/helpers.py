@@ -57,3 +57,16 @@ def assert_bits_equal(a: np.ndarray, b: np.ndarray, what: str, chunk: int = 1 <<
             rec = np.unique(bad // per)
             raise AssertionError(f"{what}: records differ from {rec[:5].tolist()} "
                                  f"({rec.size} in words {lo}..{lo + x.size}); first {a[rec[:3]]} vs {b[rec[:3]]}")
+
+
+def welded_tori(nu: int, nv: int, v: int = 0, w: int = 0):
+    """two tori that share one vertex (v of the first, w of the second): two
+    closed rings of four at it"""
+    a, b = (C.torus_mesh(nu, nv, seed=s) for s in (1, 2))
+    n = len(a[0])
+    faces = [list(f) for f in a[1]] + [[v if x == w else n + x for x in f] for f in b[1]]
+    pts = np.concatenate([np.asarray(a[0]), np.asarray(b[0]) + np.float32(0.5)]).astype(np.float32)
+    # without the vertex that nothing uses now
+    keep = np.delete(np.arange(2 * n), n + w)
+    remap = {int(x): i for i, x in enumerate(keep)}
+    return C.from_faces(pts[keep], [[remap[x] for x in f] for f in faces], creases=a[4])

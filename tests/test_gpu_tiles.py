@@ -108,3 +108,24 @@ def test_normal_tiles(name, cage, depth):
     want = O.halfedge_normals(ds.download(), depth, True)
     ds.close()
     assert_bytes_equal(got, np.ascontiguousarray(want).reshape(got.shape), name)
+
+
+@pytest.mark.parametrize("rule", [r[1] for r in RULES], ids=[r[0] for r in RULES])
+def test_two_rings_at_a_vertex(rule):
+    """both close inside one tile (level 2: the quads of 16 cage faces)"""
+    import torch
+    from halfedgecatmullclark_amd import capi
+    from tests.helpers import welded_tori
+    c, D = welded_tori(3, 3, 0, 4), 4
+    want, got = tiled(c, D, rule)
+    for g in got:
+        assert_bytes_equal(g, want, "welded")
+    b = capi.Batch([c, C.torus(4, 4)], [D, 3])
+    b.refine(15 | rule)
+    want = [b.download(i)["points"].copy() for i in range(2)]
+    for _ in range(2):
+        b.refine_points(None, rule)
+        torch.cuda.synchronize()
+        for i in range(2):
+            assert_bytes_equal(b.download(i)["points"], want[i], f"batch {i}")
+    b.close()

@@ -1,0 +1,41 @@
+"""Library internals that run on the host, compiled for the CPU alone."""
+import ctypes
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from halfedgecatmullclark_amd import build as B
+from halfedgecatmullclark_amd import cage as C
+from halfedgecatmullclark_amd.abi import MeshView
+from tests.helpers import welded_tori
+from tests.test_gpu_rare import bipyramid, cone, prism
+
+
+@pytest.fixture(scope="module")
+def checks(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("host_checks") / "host_checks.so")
+    src = os.path.join(os.path.dirname(os.path.abspath(__file__)), "host_checks.hip")
+    subprocess.run([B.hipcc(), "--offload-host-only", "-O1", "-std=c++17", "-fPIC", "-shared", "-x", "hip", src, "-o", so],
+                   check=True, capture_output=True)
+    return ctypes.CDLL(so)
+
+
+def crossed():
+    """a torus with the twins of two edges exchanged"""
+    c = C.torus(4, 3).copy()
+    e = np.flatnonzero(c.halfedges[:, 0] > np.arange(c.H))[:2]
+    t = c.halfedges[e, 0].copy()
+    c.halfedges[e, 0] = t[::-1]
+    return c
+
+
+# rings 1, simple 2, table 4
+@pytest.mark.parametrize("name,cage,want", [
+    ("torus", C.torus(4, 3), 7), ("irregular", C.irregular(1, seed=3), 7), ("prism64", prism(64), 7),
+    ("cone63", cone(63), 7), ("prism65", prism(65), 3), ("bipyramid65", bipyramid(65), 3), ("cone65", cone(65), 3),
+    ("welded", welded_tori(3, 3), 1), ("crossed", crossed(), 1)], ids=lambda x: x if isinstance(x, str) else "")
+def test_which_cages_take_the_table_and_the_tiles(checks, name, cage, want):
+    m = MeshView(cage.contiguous())
+    assert checks.check_rare_table(m.pointer) == want
