@@ -84,9 +84,11 @@ struct FusedArgs {
     int owner_write = 1;
     // the tile kernel (cc_tile.h): level d-1's records and counts, the
     // level's owner bits and where the bits of the representatives it leaves
-    // to the masked kernel go.  These follow from the topology and creases
-    // alone, but every pass writes them before it reads them, so passes on
-    // several streams need no order between them (16 MB beside 2.5 GB).
+    // to the masked kernel go.  These follow from the topology and, under the
+    // creased rules, from the creases, which keep a vertex with a sharp edge
+    // from its tile.  Every pass writes them before it reads them (16 MB
+    // beside 2.5 GB), and each rule has its own, so passes over one topology
+    // that overlap on several streams write the same words alike.
     const He *par = nullptr;
     int32_t pV = 0, pF = 0, pE = 0;
     const uint64_t *own_in = nullptr;

@@ -76,8 +76,8 @@ struct ccd_Subd {
     int64_t own_off[cch::kMaxDepth + 1] = {};
     bool own_valid[cch::kMaxDepth + 1] = {};
     // likewise the representatives the tile kernel leaves to the vertex kernel
-    // (FusedArgs::far)
-    uint64_t *far_masks = nullptr;
+    // (FusedArgs::far), of the uncreased (0) and the creased rules (1)
+    uint64_t *far_masks[2] = {};
     // edge-representative bits of levels 1..D-2 (FusedArgs::erep; the owner
     // test of level d reads levels up to d-1), and which levels hold bits of
     // the current cage's topology

@@ -84,7 +84,7 @@ bool ccd_Subd::alloc(const cc_Mesh *cage, int32_t depth) {
     CC_TRY(hipMalloc(&cr, sizeof(Crease) * (size_t)n.cumC(D)), "hipMalloc(creases)");
     CC_TRY(hipMalloc(&pts, sizeof(P3) * (size_t)n.cumV(D)), "hipMalloc(points)");
     // bit arrays: deferred vertices, edge representatives, vertex owners and
-    // those left to the vertex kernel
+    // those left to the vertex kernel by either rule
     const int64_t defer_words = D >= 2 ? (n.H[D - 1] + 63) / 64 : 1;
     const int64_t erep_words = D >= 4 ? tab.R[D - 1] : 0;
     int64_t words = defer_words + erep_words;
@@ -93,12 +93,13 @@ bool ccd_Subd::alloc(const cc_Mesh *cage, int32_t depth) {
         own_off[d] = own_words;
         own_words += (n.H[d] + 63) / 64;
     }
-    words += 2 * own_words;
+    words += 3 * own_words;
     CC_TRY(hipMalloc(&bits, sizeof(uint64_t) * (size_t)(words + 1)), "hipMalloc(bit arrays)");
     defer_mask = bits;
     erep = D >= 4 ? bits + defer_words : nullptr;
     own_masks = bits + defer_words + erep_words;
-    far_masks = own_masks + own_words;
+    far_masks[0] = own_masks + own_words;
+    far_masks[1] = far_masks[0] + own_words;
     return true;
 }
 
@@ -417,7 +418,7 @@ void ccd_Subd::level_fused(int d, int32_t steps, int topo, int uvMode, P3 *point
     }
     if (tiles) {
         a.own_in = a.owner_mask;
-        a.far = far_masks + own_off[d];
+        a.far = far_masks[creased] + own_off[d];
         a.par = he + n.offH[d - 1];
         a.pV = (int32_t)n.V[d - 1]; a.pF = (int32_t)n.F[d - 1]; a.pE = (int32_t)n.E[d - 1];
         launch_timed("level_points", n.H[d], st, [&] { launch_level_points(a, gather, creased, st); });

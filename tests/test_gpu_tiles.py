@@ -129,3 +129,28 @@ def test_two_rings_at_a_vertex(rule):
         for i in range(2):
             assert_bytes_equal(b.download(i)["points"], want[i], f"batch {i}")
     b.close()
+
+
+def test_rules_on_two_streams():
+    """creased and uncreased passes of one subd, overlapping, each into its
+    own buffer: the vertices at sharp edges, which only the creased rules
+    leave to the vertex kernel, are written in every pass"""
+    import torch
+    from halfedgecatmullclark_amd import capi
+    c, D = C.torus(24, 16, ring_sharpness=((0, 5.0), (3, 2.5), (8, 4.0))), 6
+    ds = capi.DeviceSubd(c, D)
+    want = {}
+    for rule in (0, 32):
+        ds.refine(15 | rule)
+        want[rule] = torch.from_numpy(ds.download()["points"]).cuda()
+    streams = {rule: torch.cuda.Stream() for rule in want}
+    out = {rule: [torch.full((ds.n["Vcum"][D], 3), 7.0, device="cuda") for _ in range(12)] for rule in want}
+    torch.cuda.synchronize()
+    for k in range(12):
+        for rule, s in streams.items():
+            ds.refine_points(None, out[rule][k].data_ptr(), rule, s.cuda_stream)
+    torch.cuda.synchronize()
+    for rule in want:
+        for k, t in enumerate(out[rule]):
+            assert torch.equal(t.view(torch.int32), want[rule].view(torch.int32)), (rule, k)
+    ds.close()
