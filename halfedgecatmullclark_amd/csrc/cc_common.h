@@ -62,17 +62,29 @@ __host__ __device__ __forceinline__ T *at32(T *p, uint32_t i) {
     return reinterpret_cast<T *>(reinterpret_cast<char *>(p) + i * (uint32_t)sizeof(T));
 }
 // Element i >= 0 of an array of 12- or 24-byte records (points, creases,
-// gradients) gathered at a per-lane index: 3 i fits 32 bits for every ID
-// (counts stay below 2^31 / 2), so the address is a shift-add on that and a
-// 64-bit shift-add.  Left to itself the compiler takes a 64-bit
-// multiply-add (quarter rate) for each.  (For the adjoint, which is short of
-// issue slots; in the fused level kernel the same change moves the loads
-// behind the child stores: 2433 -> 2671 us at level 7 of the 64 x 32 torus.)
+// gradients, normals) gathered at a per-lane index: 3 i as one 64-bit
+// shift-add, the address as another.  Left to itself the compiler takes a
+// 64-bit multiply-add (quarter rate) for each.  (3 i in 32 bits does for the
+// edges, faces and halfedges of a level, below 2^30 by the limits on IDs, but
+// not for its vertices, which halfedges need not use; it is no faster: 2866
+// and 2884 us for a fit of the 64 x 32 torus at depth 8.)  For the adjoint,
+// the tile kernel and the normals, which are short of issue slots; in the
+// fused level kernel the same change moves the loads behind the child stores:
+// 2433 -> 2671 us at level 7 of that torus.
+__host__ __device__ __forceinline__ uint64_t times3(uint32_t i) {
+#ifdef __HIP_DEVICE_COMPILE__
+    uint64_t r;
+    asm("v_lshl_add_u64 %0, %1, 1, %1" : "=v"(r) : "v"((uint64_t)i));
+    return r;
+#else
+    return 3ull * i;
+#endif
+}
 template <class T>
 __host__ __device__ __forceinline__ T *at3(T *p, int32_t i) {
     static_assert(sizeof(T) == 12 || sizeof(T) == 24, "three words or three double words");
     using C = std::conditional_t<std::is_const_v<T>, const char, char>;
-    return reinterpret_cast<T *>(reinterpret_cast<C *>(p) + ((uint64_t)(3u * (uint32_t)i) << (sizeof(T) == 12 ? 2 : 3)));
+    return reinterpret_cast<T *>(reinterpret_cast<C *>(p) + (times3((uint32_t)i) << (sizeof(T) == 12 ? 2 : 3)));
 }
 __host__ __device__ __forceinline__ int4 he_load(const HeRec<12> *p, int64_t i) {
     const int32_t *q = reinterpret_cast<const int32_t *>(p) + 3 * i;
