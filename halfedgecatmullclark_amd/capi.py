@@ -83,6 +83,7 @@ def lib(variant: str = "uv") -> ctypes.CDLL:
         "ccd_SetOption": (i32, [vp, i32, i32]),
         "ccd_TimingCount": (i32, [vp]),
         "ccd_TimingName": (ctypes.c_char_p, [vp, i32]),
+        "ccd_TimingLevel": (i32, [vp, i32]),
         "ccd_TimingMs": (ctypes.c_float, [vp, i32]),
         "ccd_Autotune": (i32, [vp, i32, vp]),
         "ccd_TileOption": (i32, [vp, i32, i32]),
@@ -426,6 +427,10 @@ class DeviceSubd:
         n = self.L.ccd_TimingCount(self.handle)
         return [(self.L.ccd_TimingName(self.handle, i).decode(), float(self.L.ccd_TimingMs(self.handle, i)))
                 for i in range(n)]
+
+    def timing_levels(self) -> list[int]:
+        """the level of each of timings()"""
+        return [int(self.L.ccd_TimingLevel(self.handle, i)) for i in range(self.L.ccd_TimingCount(self.handle))]
 
     def close(self):
         if getattr(self, "handle", None):

@@ -14,6 +14,7 @@
 struct ccd_Subd {
     struct Timed {
         const char *name;
+        int level;   // the level it reads, 0 for the cage
         hipEvent_t start, stop;
     };
 
@@ -133,9 +134,9 @@ struct ccd_Subd {
     bool adjoint(const void *gradFinest, void *gradCage, int32_t steps, hipStream_t st);
     void zero(float *p, int64_t count, hipStream_t st);
     template <typename K, typename... Args>
-    void launch(const char *name, K kernel, int64_t threads, hipStream_t st, Args... args);
+    void launch(const char *name, int level, K kernel, int64_t threads, hipStream_t st, Args... args);
     template <typename Fn>
-    void launch_timed(const char *name, int64_t threads, hipStream_t st, Fn &&fn);
+    void launch_timed(const char *name, int level, int64_t threads, hipStream_t st, Fn &&fn);
     bool normals(cch::P3 *out, bool smooth, hipStream_t st);
 };
 

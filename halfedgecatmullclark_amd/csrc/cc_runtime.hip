@@ -267,10 +267,10 @@ void ccd_Subd::begin_timing() {
 }
 
 template <typename K, typename... Args>
-void ccd_Subd::launch(const char *name, K kernel, int64_t threads, hipStream_t st, Args... args) {
+void ccd_Subd::launch(const char *name, int level, K kernel, int64_t threads, hipStream_t st, Args... args) {
     if (threads <= 0) return;
     const unsigned grid = (unsigned)((threads + kBlock - 1) / kBlock);
-    Timed t{name, nullptr, nullptr};
+    Timed t{name, level, nullptr, nullptr};
     if (timing) {
         (void)hipEventCreate(&t.start);
         (void)hipEventCreate(&t.stop);
@@ -284,9 +284,9 @@ void ccd_Subd::launch(const char *name, K kernel, int64_t threads, hipStream_t s
 }
 
 template <typename Fn>
-void ccd_Subd::launch_timed(const char *name, int64_t threads, hipStream_t st, Fn &&fn) {
+void ccd_Subd::launch_timed(const char *name, int level, int64_t threads, hipStream_t st, Fn &&fn) {
     if (threads <= 0) return;
-    Timed t{name, nullptr, nullptr};
+    Timed t{name, level, nullptr, nullptr};
     if (timing) {
         (void)hipEventCreate(&t.start);
         (void)hipEventCreate(&t.stop);
@@ -341,16 +341,16 @@ bool ccd_Subd::refine_topology(int32_t steps, int dmax, hipStream_t st) {
     const int uvMode = uv_mode(steps, U0);
     if (topo || uvMode == 1) {
         const DCage c = cage_view(nullptr);
-        launch("cage_halfedges", k_cage_halfedges, H0, st, c, he, (int)topo, uvMode);
+        launch("cage_halfedges", 0, k_cage_halfedges, H0, st, c, he, (int)topo, uvMode);
         for (int d = 1; d < dmax; ++d) {
-            launch("level_halfedges", k_level_halfedges, n.H[d], st, (const He *)(he + n.offH[d]), he + n.offH[d + 1],
+            launch("level_halfedges", d, k_level_halfedges, n.H[d], st, (const He *)(he + n.offH[d]), he + n.offH[d + 1],
                    (int32_t)n.H[d], (int32_t)n.V[d], (int32_t)n.F[d], (int32_t)n.E[d], (int)topo, uvMode);
         }
     }
     if (steps & CCD_CREASES) {
-        launch("cage_creases", k_creases, E0, st, (const Crease *)c_cr, E0, cr);
+        launch("cage_creases", 0, k_creases, E0, st, (const Crease *)c_cr, E0, cr);
         for (int d = 1; d < dmax; ++d)
-            launch("level_creases", k_creases, n.C[d], st, (const Crease *)(cr + n.offC[d]), (int32_t)n.C[d], cr + n.offC[d + 1]);
+            launch("level_creases", d, k_creases, n.C[d], st, (const Crease *)(cr + n.offC[d]), (int32_t)n.C[d], cr + n.offC[d + 1]);
     }
     return true;
 }
@@ -364,9 +364,9 @@ void ccd_Subd::level_patch(int d, int32_t steps, int topo, int uvMode, P3 *point
     a.defer_mask = defer_mask;
     const DCage c = cage_view(nullptr);
     const LevelPtrs lp = level_ptrs();
-    launch_timed("level_patch", n.H[d], st,
+    launch_timed("level_patch", d, n.H[d], st,
                  [&] { launch_level_patch(a, c, tab, lp, d, gather, creased, topo, uvMode, cfg[d].nt, cfg[d].hpt, st); });
-    launch_timed("level_deferred", n.V[d], st, [&] { launch_level_deferred(a, c, tab, lp, d, gather, creased, st); });
+    launch_timed("level_deferred", d, n.V[d], st, [&] { launch_level_deferred(a, c, tab, lp, d, gather, creased, st); });
 }
 
 // one level of the fused kernels: children with face and edge points, then
@@ -405,7 +405,7 @@ void ccd_Subd::level_fused(int d, int32_t steps, int topo, int uvMode, P3 *point
     const bool tiles = split || (tileable && !topo && uvMode == 0 && own_valid[d]);
     const bool fused_points = pts_ && !tiles;
     if (topo || uvMode == 1 || fused_points) {
-        launch_timed(fused_points && !topo ? "level_points" : "level_fused", n.H[d], st,
+        launch_timed(fused_points && !topo ? "level_points" : "level_fused", d, n.H[d], st,
                      [&] {
                          launch_level_fused(a, c, tab, d, gather, creased, topo, uvMode, fused_points, opt_store,
                                             cfg[d].fb, cfg[d].ft, st);
@@ -421,10 +421,10 @@ void ccd_Subd::level_fused(int d, int32_t steps, int topo, int uvMode, P3 *point
         a.far = far_masks[creased] + own_off[d];
         a.par = he + n.offH[d - 1];
         a.pV = (int32_t)n.V[d - 1]; a.pF = (int32_t)n.F[d - 1]; a.pE = (int32_t)n.E[d - 1];
-        launch_timed("level_points", n.H[d], st, [&] { launch_level_points(a, gather, creased, st); });
+        launch_timed("level_points", d, n.H[d], st, [&] { launch_level_points(a, gather, creased, st); });
     }
     if (pts_) {
-        launch_timed("level_vertices", n.H[d], st, [&] {
+        launch_timed("level_vertices", d, n.H[d], st, [&] {
             launch_level_vertices(a, c, tab, level_ptrs(), rare_view(), d, gather, creased, opt_fan, cfg[d].scan,
                                   cfg[d].vw, st);
         });
@@ -437,12 +437,12 @@ void ccd_Subd::cage_points(int32_t steps, const P3 *cagePts, P3 *out, hipStream_
     const int creased = (steps & CCD_NOCREASES) ? 0 : 1;
     const DCage c = cage_view(cagePts);
     P3 *vp = out, *fp = out + V0, *ep = out + V0 + F0;
-    launch("cage_faces", k_cage_faces, F0, st, c, fp, (int)gather);
-    launch("cage_edges", k_cage_edges, E0, st, c, (const P3 *)fp, ep, (int)gather, creased);
+    launch("cage_faces", 0, k_cage_faces, F0, st, c, fp, (int)gather);
+    launch("cage_edges", 0, k_cage_edges, E0, st, c, (const P3 *)fp, ep, (int)gather, creased);
     if (gather) {
-        launch("cage_vertices", k_cage_vertices_gather, V0, st, c, (const P3 *)fp, (const P3 *)ep, vp, creased);
+        launch("cage_vertices", 0, k_cage_vertices_gather, V0, st, c, (const P3 *)fp, (const P3 *)ep, vp, creased);
     } else {
-        launch("cage_vertices", k_cage_vertices_scatter, V0, st, c, (const P3 *)fp, (const P3 *)ep, vp, creased);
+        launch("cage_vertices", 0, k_cage_vertices_scatter, V0, st, c, (const P3 *)fp, (const P3 *)ep, vp, creased);
     }
 }
 
@@ -461,14 +461,14 @@ bool ccd_Subd::refine_points(int32_t steps, int dmax, const P3 *cagePts, P3 *out
             continue;
         }
         const Lvl L = level_view(d, out + n.offV[d], out + n.offV[d + 1]);
-        launch("faces", k_faces, n.F[d], st, L, (int)gather);
+        launch("faces", d, k_faces, n.F[d], st, L, (int)gather);
         if (gather) {
-            launch("edges", k_edges_gather, n.E[d], st, L, c, tab, d, creased);
-            launch("vertices", k_vertices_gather, n.V[d], st, L, c, tab, d, creased);
+            launch("edges", d, k_edges_gather, n.E[d], st, L, c, tab, d, creased);
+            launch("vertices", d, k_vertices_gather, n.V[d], st, L, c, tab, d, creased);
         } else {
-            launch("edges", k_edges_scatter, n.H[d], st, L, creased);
+            launch("edges", d, k_edges_scatter, n.H[d], st, L, creased);
             zero(&L.vp->x, 3 * n.V[d], st);
-            launch("vertices", k_vertices_scatter, n.H[d], st, L, creased);
+            launch("vertices", d, k_vertices_scatter, n.H[d], st, L, creased);
         }
     }
     return true;
@@ -490,12 +490,12 @@ bool ccd_Subd::refine(int32_t steps, int dmax, hipStream_t st) {
     const bool points = (steps & CCD_POINTS) != 0;
     const int uvMode = uv_mode(steps, U0);
     if (steps & CCD_CREASES) {
-        launch("cage_creases", k_creases, E0, st, (const Crease *)c_cr, E0, cr);
+        launch("cage_creases", 0, k_creases, E0, st, (const Crease *)c_cr, E0, cr);
         for (int d = 1; d < dmax; ++d)
-            launch("level_creases", k_creases, n.C[d], st, (const Crease *)(cr + n.offC[d]), (int32_t)n.C[d], cr + n.offC[d + 1]);
+            launch("level_creases", d, k_creases, n.C[d], st, (const Crease *)(cr + n.offC[d]), (int32_t)n.C[d], cr + n.offC[d + 1]);
     }
     const DCage c = cage_view(nullptr);
-    if (topo || uvMode == 1) launch("cage_halfedges", k_cage_halfedges, H0, st, c, he, (int)topo, uvMode);
+    if (topo || uvMode == 1) launch("cage_halfedges", 0, k_cage_halfedges, H0, st, c, he, (int)topo, uvMode);
     if (points) cage_points(steps, nullptr, pts, st);
     for (int d = 1; d < dmax; ++d) {
         if (points && cfg[d].kind == 2) level_patch(d, steps, topo, uvMode, pts, st);
@@ -1045,7 +1045,8 @@ int32_t ccd_SetOption(ccd_Subd *s, int32_t key, int32_t value) {
 //      halfedges per thread;
 //   3. the patch-local kernel with tiles of 128, 256 or 512 halfedges.
 // Each candidate runs the given steps three times (the first discarded); a
-// level's time is that of its fused (or patch) and vertex kernels.
+// level's time is that of all its kernels but the creases': fused, patch,
+// tile, vertex and deferred ones.
 int32_t ccd_Subd::autotune(int32_t steps, hipStream_t st) {
     if (!(steps & CCD_POINTS) || opt_fused == 0 || D < 2) return 0;
     drop_graphs();
@@ -1062,18 +1063,11 @@ int32_t ccd_Subd::autotune(int32_t steps, hipStream_t st) {
             if (!refine(steps, D, st)) return false;
             if (hip_failed(hipStreamSynchronize(st), "autotune")) return false;
             if (rep == 0) continue;  // warm-up
-            // level d's kernels are the timed launches between its first
-            // kernel and the next level's; they come in level order
-            int d = 0;
             for (auto &t : timed) {
-                const bool first = !strcmp(t.name, "level_fused") || !strcmp(t.name, "level_points") ||
-                                   !strcmp(t.name, "level_patch");
-                const bool level_kernel = first || !strcmp(t.name, "level_vertices") || !strcmp(t.name, "level_deferred");
-                if (!level_kernel) continue;
-                if (first) ++d;
+                if (t.level < 1 || t.level > kMaxDepth || !strcmp(t.name, "level_creases")) continue;
                 float x = 0.0f;
                 (void)hipEventElapsedTime(&x, t.start, t.stop);
-                if (d >= 1 && d <= kMaxDepth) ms[d] += x;
+                ms[t.level] += x;
             }
         }
         return true;
@@ -1141,6 +1135,10 @@ int32_t ccd_TimingCount(const ccd_Subd *s) { return s ? (int32_t)s->timed.size()
 
 const char *ccd_TimingName(const ccd_Subd *s, int32_t i) {
     return (s && i >= 0 && i < (int32_t)s->timed.size()) ? s->timed[i].name : "";
+}
+
+int32_t ccd_TimingLevel(const ccd_Subd *s, int32_t i) {
+    return (s && i >= 0 && i < (int32_t)s->timed.size()) ? s->timed[i].level : -1;
 }
 
 float ccd_TimingMs(const ccd_Subd *s, int32_t i) {

@@ -379,10 +379,12 @@ int32_t ccd_Autotune(ccd_Subd *subd, int32_t steps, void *stream);
  * _FUSED_BLOCK, _FUSED_TILES or _VERTEX_WAVES used at one level, or -1 */
 int32_t ccd_TileOption(const ccd_Subd *subd, int32_t key, int32_t level);
 /* per-kernel timing with HIP events on the launch stream: enable, run, then
- * read the kernel names and mean milliseconds of the last ccd_Refine. */
+ * read the kernel names, the levels they read (0: the cage) and the
+ * milliseconds of the last ccd_Refine. */
 int32_t ccd_SetTiming(ccd_Subd *subd, int32_t enable);
 int32_t ccd_TimingCount(const ccd_Subd *subd);
 const char *ccd_TimingName(const ccd_Subd *subd, int32_t i);
+int32_t ccd_TimingLevel(const ccd_Subd *subd, int32_t i);
 float ccd_TimingMs(const ccd_Subd *subd, int32_t i);
 
 /* ---- batched refinement (extension; no counterpart in the reference) ------

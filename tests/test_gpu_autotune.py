@@ -112,3 +112,32 @@ def test_option_values_refused(capi):
                 obj.set_option(key, bad)
     ds.close()
     b.close()
+
+
+def test_launches_of_a_split_level(capi):
+    """The launches of a level whose points follow its children (level 4:
+    671744 quads), which the tuner times, belong to that level."""
+    ds = capi.DeviceSubd(C.torus(64, 41), 5)
+    ds.set_timing(True)
+    ds.refine(capi.ALL)
+    ds.synchronize()
+    names = [n for n, _ in ds.timings()]
+    got = [x for x in zip(names, ds.timing_levels()) if x[0] not in ("level_creases", "cage_creases")]
+    ds.close()
+    want = [("cage_halfedges", 0), ("cage_faces", 0), ("cage_edges", 0), ("cage_vertices", 0)]
+    for d in (1, 2, 3):
+        want += [("level_fused", d), ("level_vertices", d)]
+    assert got == want + [("level_fused", 4), ("level_points", 4), ("level_vertices", 4)]
+
+
+def test_autotuned_split_level(capi):
+    cage, depth = C.torus(64, 41), 5
+    want = O.refine(cage, depth, O.ALL)
+    ds = capi.DeviceSubd(cage, depth)
+    ds.refine(capi.ALL)
+    ds.autotune(capi.ALL)
+    ds.refine(capi.ALL)
+    got = ds.download()
+    ds.close()
+    for k in ("halfedges", "creases", "points"):
+        assert_bytes_equal(got[k], want[k], f"autotuned {k}")
