@@ -198,19 +198,22 @@ void vertices_scan(const BatchTable &t, char *arena, int d, int remap, hipStream
                        static_cast<const LevelJob *>(t.jobs), t.start, (int)t.n, d, remap, arena);
 }
 
-template <int G, int C, int W, int WORDS = kOwnerWords>
-void vertices_masked(const BatchTable &t, char *arena, int d, int remap, int far, hipStream_t st) {
-    hipLaunchKernelGGL((k_batch_vertices_masked<G, C, W, WORDS>), dim3(t.blocks), dim3(256), 0, st,
-                       static_cast<const LevelJob *>(t.jobs), t.start, (int)t.n, d, remap, far, arena);
+template <int G, int C, int WORDS>
+void vertices_masked(const BatchTable &t, char *arena, int d, int remap, int waves, int far, hipStream_t st) {
+    const auto run = [&](auto k) {
+        hipLaunchKernelGGL(k, dim3(t.blocks), dim3(256), 0, st, static_cast<const LevelJob *>(t.jobs), t.start,
+                           (int)t.n, d, remap, far, arena);
+    };
+    if (waves == 4) run(k_batch_vertices_masked<G, C, 4, WORDS>);
+    else if (waves == 6) run(k_batch_vertices_masked<G, C, 6, WORDS>);
+    else run(k_batch_vertices_masked<G, C, kVertexWaves, WORDS>);
 }
 
 template <int G, int C>
 void vertices_gc(const BatchTable &t, char *arena, int d, int scan, int remap, int waves, int far, hipStream_t st) {
     if (scan == 0) {
-        if (far == kFarWords) vertices_masked<G, C, kVertexWaves, kFarWords>(t, arena, d, remap, far, st);
-        else if (waves == 4) vertices_masked<G, C, 4>(t, arena, d, remap, far, st);
-        else if (waves == 6) vertices_masked<G, C, 6>(t, arena, d, remap, far, st);
-        else vertices_masked<G, C, kVertexWaves>(t, arena, d, remap, far, st);
+        if (far == kFarWords) vertices_masked<G, C, kFarWords>(t, arena, d, remap, waves, far, st);
+        else vertices_masked<G, C, kOwnerWords>(t, arena, d, remap, waves, far, st);
         return;
     }
     if (scan == 2) vertices_scan<G, C, 2>(t, arena, d, remap, st);

@@ -260,7 +260,7 @@ __global__ __launch_bounds__(256) void k_level_vertices_direct(FusedArgs a, DCag
 template <int G, int C, int T, int U, int P, int S, int NT>
 static void launch_fused_tiles(const FusedArgs &a, const DCage &c, const LevelTab &t, int d, int tiles,
                                hipStream_t st) {
-    constexpr bool kMulti = S == kStoreLds && P == 1;
+    constexpr bool kMulti = S == kStoreLds;
     if (!kMulti) tiles = 1;
     const int64_t per = (int64_t)NT * tiles;
     const dim3 grid((unsigned)((a.H + per - 1) / per));
@@ -274,11 +274,11 @@ static void launch_fused_tiles(const FusedArgs &a, const DCage &c, const LevelTa
 }
 
 // 256 and 512 threads, and several tiles per workgroup, with LDS-staged
-// stores and points only; 1024 threads and one tile otherwise
+// stores only; 1024 threads and one tile otherwise
 template <int G, int C, int T, int U, int P, int S>
 static void launch_fused_nt(const FusedArgs &a, const DCage &c, const LevelTab &t, int d, int nt, int tiles,
                             hipStream_t st) {
-    if constexpr (S == kStoreLds && P == 1) {
+    if constexpr (S == kStoreLds) {
         if (nt == 256) return launch_fused_tiles<G, C, T, U, P, S, 256>(a, c, t, d, tiles, st);
         if (nt == 512) return launch_fused_tiles<G, C, T, U, P, S, 512>(a, c, t, d, tiles, st);
     }
@@ -294,10 +294,11 @@ static void launch_fused_nt(const FusedArgs &a, const DCage &c, const LevelTab &
 static void launch_fused_impl(const FusedArgs &a, const DCage &c, const LevelTab &t, int d, int gather, int creased,
                               int topo, int uvMode, int points, int store, int nt, int tiles, hipStream_t st) {
 #define CC_FUSED_STORES(G, C, T, U, P) CC_FUSED_CASE(G, C, T, U, P, kStoreDirect) CC_FUSED_CASE(G, C, T, U, P, kStoreLds)
-#define CC_FUSED_POINTS(G, C, T, U) CC_FUSED_STORES(G, C, T, U, 0) CC_FUSED_STORES(G, C, T, U, 1)
-#define CC_FUSED_UV(G, C, T) CC_FUSED_POINTS(G, C, T, 0) CC_FUSED_POINTS(G, C, T, 1) CC_FUSED_POINTS(G, C, T, 2)
-#define CC_FUSED_TOPO(G, C) CC_FUSED_UV(G, C, 0) CC_FUSED_UV(G, C, 1)
-    CC_FUSED_TOPO(0, 0) CC_FUSED_TOPO(0, 1) CC_FUSED_TOPO(1, 0) CC_FUSED_TOPO(1, 1)
+#define CC_FUSED_UV(G, C, T, P) CC_FUSED_STORES(G, C, T, 0, P) CC_FUSED_STORES(G, C, T, 1, P) CC_FUSED_STORES(G, C, T, 2, P)
+#define CC_FUSED_TOPO(G, C, P) CC_FUSED_UV(G, C, 0, P) CC_FUSED_UV(G, C, 1, P)
+    if (!points) gather = creased = 0;   // the rules of the points: one kernel for all
+    CC_FUSED_TOPO(0, 0, 0)
+    CC_FUSED_TOPO(0, 0, 1) CC_FUSED_TOPO(0, 1, 1) CC_FUSED_TOPO(1, 0, 1) CC_FUSED_TOPO(1, 1, 1)
 }
 
 void launch_level_fused(const FusedArgs &a, const DCage &c, const LevelTab &t, int d, int gather, int creased, int topo,
@@ -324,8 +325,11 @@ static void launch_ring(const FusedArgs &a, const DCage &c, const LevelTab &t, c
     const uint32_t nr = rare_blocks(rv, d);
     grid.x += nr;
     const auto run = [&](auto k) { hipLaunchKernelGGL(k, grid, dim3(256), 0, st, a, c, t, lp, d, rv, nr); };
-    if (a.far && a.F >= kTileBigFrom) run(k_level_vertices_ring<G, C, kVertexWaves, kFarWords>);
-    else if (waves == 4) run(k_level_vertices_ring<G, C, 4, kOwnerWords>);
+    if (a.far && a.F >= kTileBigFrom) {
+        if (waves == 4) run(k_level_vertices_ring<G, C, 4, kFarWords>);
+        else if (waves == 6) run(k_level_vertices_ring<G, C, 6, kFarWords>);
+        else run(k_level_vertices_ring<G, C, kVertexWaves, kFarWords>);
+    } else if (waves == 4) run(k_level_vertices_ring<G, C, 4, kOwnerWords>);
     else if (waves == 6) run(k_level_vertices_ring<G, C, 6, kOwnerWords>);
     else run(k_level_vertices_ring<G, C, kVertexWaves, kOwnerWords>);
 }

@@ -141,3 +141,36 @@ def test_autotuned_split_level(capi):
     ds.close()
     for k in ("halfedges", "creases", "points"):
         assert_bytes_equal(got[k], want[k], f"autotuned {k}")
+
+
+def kernels_of(fn):
+    """names of the kernels fn launches"""
+    import torch
+    from torch.profiler import ProfilerActivity, profile
+    torch.zeros(1, device="cuda")
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        fn()
+        torch.cuda.synchronize()
+    return [e.name for e in p.events()]
+
+
+@pytest.mark.parametrize("fb,ft,waves", [(256, 1, 6), (512, 2, 4), (1024, 4, 8)])
+def test_options_reach_split_levels(capi, fb, ft, waves):
+    """Every geometry of the children kernel and every build of the vertex
+    kernel behind large tiles can be chosen, and gives the same bytes."""
+    cage, depth = C.torus(64, 41), 5
+    want = O.refine(cage, depth, O.ALL)
+    ds, b = capi.DeviceSubd(cage, depth), capi.Batch([cage], [depth])
+    for obj, ring in ((ds, "k_level_vertices_ring<0, 1, %d, 16>"), (b, "k_batch_vertices_masked<0, 1, %d, 16>")):
+        set_all(obj, capi, fb, ft, 0, waves)
+        obj.set_option(capi.OPT_GRAPH, 0)
+        names = kernels_of(lambda: obj.refine(capi.ALL))
+        assert any(ring % waves in n for n in names), names
+        children = ("k_level_fused<0, 0, 1, 1, 0, 1, %d, %d>" if obj is ds else
+                    "k_batch_fused<0, 0, 1, %d, %d, 0>") % (fb, ft > 1)
+        assert any(children in n for n in names), names
+        got = ds.download() if obj is ds else b.download(0)
+        for k in ("halfedges", "creases", "points"):
+            assert_bytes_equal(got[k], want[k], k)
+    ds.close()
+    b.close()
