@@ -9,15 +9,13 @@
 #include <string.h>
 
 #include <algorithm>
-#include <atomic>
 #include <map>
 #include <new>
-#include <system_error>
-#include <thread>
 #include <vector>
 
 #include "cc_batch.h"
 #include "cc_internal.h"
+#include "cc_lists.h"
 #include "cc_kernels.h"
 #include "cc_level.h"
 #include "cc_patch.h"
@@ -203,43 +201,6 @@ struct TableBuilder {
 int64_t blocks_of(int64_t threads, int64_t per = 256) { return (threads + per - 1) / per; }
 
 // consecutive 256-byte aligned ranges of one allocation
-struct CageLists {
-    CageRings r;
-    RareTable rt;
-};
-
-// Every cage's ring lists and rare-vertex table.  The walks wait for one
-// cached halfedge after another (48 cages of 535 thousand halfedges: 22 ms on
-// one core), and the cages are independent: up to eight threads take them in
-// turn, one per 16 thousand halfedges.  A thread that cannot be started is
-// done without; false: out of memory.
-bool build_lists(const cc_Mesh *const *meshes, std::vector<CageLists> &lists) {
-    std::atomic<size_t> next{0};
-    std::atomic<bool> ok{true};
-    auto work = [&]() {
-        try {
-            for (size_t i = next++; i < lists.size(); i = next++) {
-                build_cage_rings(meshes[i], lists[i].r);
-                if (lists[i].r.ok) build_rare_table(meshes[i], lists[i].r, lists[i].rt);
-            }
-        } catch (const std::bad_alloc &) {
-            ok = false;
-        }
-    };
-    int64_t H = 0;
-    for (size_t i = 0; i < lists.size(); ++i) H += meshes[i]->halfedgeCount;
-    const int64_t threads = std::min<int64_t>({8, (int64_t)lists.size(), (int64_t)std::thread::hardware_concurrency(), H >> 14});
-    std::vector<std::thread> pool;
-    pool.reserve(8);
-    try {
-        for (int64_t i = 1; i < threads; ++i) pool.emplace_back(work);
-    } catch (const std::system_error &) {
-    }
-    work();
-    for (std::thread &t : pool) t.join();
-    return ok;
-}
-
 struct Carve {
     size_t size = 0;
     size_t take(size_t bytes) {
@@ -269,7 +230,7 @@ DCage ccb_Batch::cage_view(int i) const {
     return c;
 }
 
-bool ccb_Batch::create(const cc_Mesh *const *meshes, const int32_t *depths, int32_t count) {
+bool ccb_Batch::create(const cc_Mesh *const *meshes, const int32_t *depths, int32_t count) try {
     N = count;
     cages.resize(count);
     std::vector<CageLists> lists(count);
@@ -404,6 +365,9 @@ bool ccb_Batch::create(const cc_Mesh *const *meshes, const int32_t *depths, int3
                               stream), "upload cage rings");
     CC_TRY(hipStreamSynchronize(stream), "batch upload");
     return build_tables();
+} catch (const std::bad_alloc &) {
+    set_error(2, "out of host memory");
+    return false;
 }
 
 void ccb_Batch::free_all() {
@@ -916,7 +880,11 @@ ccb_Batch *ccb_Create(const cc_Mesh *const *cages, const int32_t *depths, int32_
             }
         }
     }
-    ccb_Batch *b = new ccb_Batch();
+    ccb_Batch *b = new (std::nothrow) ccb_Batch();
+    if (!b) {
+        set_error(2, "out of host memory");
+        return nullptr;
+    }
     if (!b->create(cages, depths, count)) {
         b->free_all();
         delete b;

@@ -10,6 +10,7 @@
 #include <algorithm>
 
 #include <mutex>
+#include <new>
 #include <string>
 #include <unordered_map>
 #include <vector>
@@ -123,7 +124,7 @@ void ccd_Subd::drop_graphs() {
     graphs.clear();
 }
 
-bool ccd_Subd::upload_cage(const cc_Mesh *cage, hipStream_t st) {
+bool ccd_Subd::upload_cage(const cc_Mesh *cage, hipStream_t st) try {
     if (cage->vertexCount != V0 || cage->uvCount != U0 || cage->halfedgeCount != H0 ||
         cage->edgeCount != E0 || cage->faceCount != F0) {
         set_error(10, "cage counts differ from the ones the device mirror was created for");
@@ -217,6 +218,9 @@ bool ccd_Subd::upload_cage(const cc_Mesh *cage, hipStream_t st) {
     CC_TRY(hipMemcpyAsync(cage_arena, cage_host.data(), size, hipMemcpyHostToDevice, st), "upload cage");
     CC_TRY(hipStreamSynchronize(st), "upload cage");   // cage_host may change after return
     return true;
+} catch (const std::bad_alloc &) {
+    set_error(2, "out of host memory");
+    return false;
 }
 
 DCage ccd_Subd::cage_view(const P3 *points) const {

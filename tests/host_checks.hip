@@ -1,6 +1,8 @@
 // Host-side checks of library internals, compiled for the CPU alone by
 // test_host_checks.py.
-#include "../halfedgecatmullclark_amd/csrc/cc_internal.h"
+#include <stdlib.h>
+
+#include "../halfedgecatmullclark_amd/csrc/cc_lists.h"
 
 using namespace cch;
 
@@ -20,4 +22,30 @@ extern "C" uint64_t check_at3(int32_t i, int32_t bytes) {
     const void *p = bytes == 12 ? (const void *)at3(reinterpret_cast<const P3 *>(base), i)
                                 : (const void *)at3(reinterpret_cast<Six *>(base), i);
     return (uint64_t)(static_cast<const char *>(p) - base);
+}
+
+// allocations until one fails (-1: none does), this library's alone
+static std::atomic<int64_t> g_left{-1};
+void *operator new(size_t n) {
+    if (g_left.load() >= 0 && g_left.fetch_sub(1) == 0) throw std::bad_alloc();
+    void *p = malloc(n ? n : 1);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void *p) noexcept { free(p); }
+void operator delete(void *p, size_t) noexcept { free(p); }
+
+// The lists of `count` times the cage with the left-th allocation failing:
+// 1 when they are all there, 0 when memory ran out, 2 when lists are missing
+// without a word.
+extern "C" int32_t check_lists(const cc_Mesh *m, int32_t count, int64_t left) {
+    std::vector<const cc_Mesh *> meshes((size_t)count, m);
+    std::vector<CageLists> lists((size_t)count);
+    g_left = left;
+    const bool ok = build_lists(meshes.data(), lists);
+    g_left = -1;
+    if (!ok) return 0;
+    for (const CageLists &l : lists)
+        if (!l.r.ok || !l.rt.ok) return 2;
+    return 1;
 }

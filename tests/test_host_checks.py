@@ -17,7 +17,8 @@ from tests.test_gpu_rare import bipyramid, cone, prism
 def checks(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("host_checks") / "host_checks.so")
     src = os.path.join(os.path.dirname(os.path.abspath(__file__)), "host_checks.hip")
-    subprocess.run([B.hipcc(), "--offload-host-only", "-O1", "-std=c++17", "-fPIC", "-shared", "-x", "hip", src, "-o", so],
+    subprocess.run([B.hipcc(), "--offload-host-only", "-O1", "-std=c++17", "-fPIC", "-shared", "-Wl,-Bsymbolic",
+                    "-x", "hip", src, "-o", so],
                    check=True, capture_output=True)
     return ctypes.CDLL(so)
 
@@ -46,3 +47,13 @@ def test_record_offsets(checks, i):
     checks.check_at3.restype = ctypes.c_uint64
     for b in (12, 24):
         assert checks.check_at3(i, b) == b * i
+
+
+def test_lists_without_memory(checks):
+    """the threads that build a batch's lists end whichever allocation fails"""
+    checks.check_lists.argtypes = [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64]
+    m = MeshView(C.torus(64, 32).contiguous())
+    p = ctypes.cast(m.pointer, ctypes.c_void_p)
+    assert checks.check_lists(p, 16, -1) == 1
+    got = [checks.check_lists(p, 16, k) for k in range(60)]
+    assert set(got) <= {0, 1} and 0 in got
