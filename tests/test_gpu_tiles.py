@@ -154,3 +154,34 @@ def test_rules_on_two_streams():
         for k, t in enumerate(out[rule]):
             assert torch.equal(t.view(torch.int32), want[rule].view(torch.int32)), (rule, k)
     ds.close()
+
+
+# (level 4 has 256 nu nv quads; the split of a full refinement starts at 655360)
+SPLITS = [("below", 59, 43), ("exact", 64, 40), ("above", 61, 42)]
+
+
+@pytest.mark.parametrize("variant", ["uv", "nouv"])
+@pytest.mark.parametrize("name,nu,nv", SPLITS, ids=[s[0] for s in SPLITS])
+def test_split_edge(name, nu, nv, variant):
+    """full refinements whose largest level has just under, exactly and just
+    over the quads from which its points follow its children (649472, 655360
+    and 655872: 640 tiles of 1024 and half of one), the oracle's bytes"""
+    from halfedgecatmullclark_amd import capi
+    from oracle import oracle as O
+    c, D = C.torus(nu, nv), 5
+    ds = capi.DeviceSubd(c, D, variant)
+    b = capi.Batch([c, C.cube(0)], [D, 3], variant)
+    ds.set_timing(True)
+    for rule, flags in ((0, 0), (16, O.GATHER)):
+        want = O.refine(c, D, O.ALL | flags)
+        ds.refine(15 | rule)
+        ds.synchronize()
+        names = [n for n, _ in ds.timings()]
+        assert ("level_points" in names) == (name != "below")
+        b.refine(15 | rule)
+        for got in (ds.download(), b.download(0)):
+            assert_bytes_equal(got["points"], want["points"], "points")
+            for k in ("twinID", "edgeID", "vertexID"):
+                assert np.array_equal(got["halfedges"][k], want["halfedges"][k]), k
+    ds.close()
+    b.close()
