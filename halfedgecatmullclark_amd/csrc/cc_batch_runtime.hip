@@ -105,7 +105,7 @@ struct ccb_Batch {
     AdjLevelTables t_adj[kMaxDepth + 1];   // levels 1 ..
     BatchTable t_adjc_h, t_adjc_e, t_adjc_f, t_adjc_v;   // cage-step adjoint gathers: per edge, face, vertex
     bool all_rings = true;                     // every cage has its ring lists
-    bool all_simple = true;                    // RareTable::simple of every cage
+    bool all_simple = true;                    // CageRings::simple of every cage
     // the adjoint's finest steps read the caller's gradient (its address in
     // the adjoint arena's first bytes); false when a cage is refined once:
     // its cage step updates the finest gradient in place, so every call
@@ -253,7 +253,7 @@ bool ccb_Batch::create(const cc_Mesh *const *meshes, const int32_t *depths, int3
         g.o_e0 = tot_e0; tot_e0 += g.E0;
         g.o_f0 = tot_f0; tot_f0 += g.F0;
         all_rings = all_rings && r.ok;
-        all_simple = all_simple && rt.simple;
+        all_simple = all_simple && r.simple;
         if (r.ok) {
             auto put = [&](const std::vector<int32_t> &v) {
                 const int64_t o = (int64_t)rings_host.size();

@@ -1,6 +1,10 @@
 // Library-internal helpers shared by the host and runtime translation units.
 #pragma once
 
+#include <atomic>
+#include <exception>
+#include <new>
+#include <thread>
 #include <vector>
 
 #include <hip/hip_runtime.h>
@@ -37,117 +41,223 @@ bool ref_counts_fit_int32(const cc_Mesh *cage, int32_t D, const char **why);
 // The cage's vertex and face rings as the device walks them (kWalkCap
 // steps at most), in CSR form.  `ok` is false when the lists would exceed
 // 4 H + V entries (a cage whose walks do not close): the kernels then walk.
+// The walks also say whether the cage is `simple`: every walk closes, links
+// agree, and every vertex, edge and face has all its halfedges in its one
+// ring.  A tile pass, which finishes a vertex from whichever ring closes
+// inside a tile, takes no other cage (of two rings at a vertex, both might
+// write it).  The tests read nothing that a walk does not read anyway (a pass
+// of their own over 524 thousand halfedges took half as long as the walks).
 struct CageRings {
     std::vector<int32_t> voff, vring, vbnd, foff, fring, ooff, out;
+    // vertices other than closed rings of four, faces other than quads with
+    // consecutive halfedges, boundary halfedges
+    std::vector<int32_t> odd_v, odd_f, bnd;
     std::vector<int32_t> fill;   // scratch
-    bool ok = false;
-    // every listed halfedge leaves its ring's vertex and lies on its ring's face
-    bool own = true;
+    std::vector<uint8_t> seen;
+    bool ok = false, simple = false;
+    int64_t odd_v_entries = 0, odd_f_entries = 0;   // entries the rare-vertex table would have
+    bool part_ok[3] = {};
+    // of each part, any bit: not simple (gathered without branches)
+    int32_t bad[3] = {};
 };
 
-// (into r, whose storage a caller with many cages reuses)
-inline void build_cage_rings(const cc_Mesh *m, CageRings &r) {
-    r.ok = false;
-    r.own = true;
-    r.vring.clear();
-    r.fring.clear();
-    const int32_t V = m->vertexCount, F = m->faceCount, H = m->halfedgeCount;
+inline void ring_vertices(const cc_Mesh *m, CageRings &r) {
+    const int32_t V = m->vertexCount, H = m->halfedgeCount;
+    // (in variables of this thread's own: the lists' headers share cache lines)
+    std::vector<int32_t> voff = std::move(r.voff), vring = std::move(r.vring), vbnd = std::move(r.vbnd), odd_v = std::move(r.odd_v);
     const CageHe *he = reinterpret_cast<const CageHe *>(m->halfedges);
     const size_t cap = 4 * (size_t)H + (size_t)V;
-    r.voff.assign((size_t)V + 1, 0);
-    r.vbnd.assign((size_t)V, 0);
-    r.foff.assign((size_t)F + 1, 0);
-    r.vring.reserve((size_t)H + 1);   // what a cage whose walks close needs
-    r.fring.reserve((size_t)H + 1);
     auto valid = [&](int32_t h) { return h >= 0 && h < H; };
+    int32_t bad = 0;
+    int64_t entries = 0;
+    voff.assign((size_t)V + 1, 0);
+    vbnd.assign((size_t)V, 0);
+    vring.clear();
+    odd_v.clear();
+    vring.reserve((size_t)H + 1);   // what a cage whose walks close needs
+    // twin(prev(h)), -1 without; a ring's step agrees when that twin's twin is
+    // prev(h) again and both have one edge
+    auto step = [&](int32_t h) {
+        const int32_t q = he[h].prev;
+        if (!valid(q)) {
+            bad = 1;
+            return -1;
+        }
+        const int32_t g = he[q].twin;
+        if (valid(g)) bad |= (he[g].twin ^ q) | (he[g].edge ^ he[q].edge);
+        return g;
+    };
     for (int32_t v = 0; v < V; ++v) {
-        r.voff[v] = (int32_t)r.vring.size();
+        voff[v] = (int32_t)vring.size();
         const int32_t p = m->vertexToHalfedgeIDs[v];
         if (!valid(p)) continue;
-        r.vring.push_back(p);
-        r.own = r.own && he[p].vert == v;
+        vring.push_back(p);
+        bad |= he[p].vert ^ v;
         int32_t n = 1;
-        int32_t g = valid(he[p].prev) ? he[he[p].prev].twin : -1;
+        int32_t g = step(p);
         for (; g >= 0 && g != p && n < kWalkCap; ++n) {
-            if (!valid(g) || r.vring.size() >= cap) return;
-            r.vring.push_back(g);
-            r.own = r.own && he[g].vert == v;
-            g = valid(he[g].prev) ? he[he[g].prev].twin : -1;
+            if (!valid(g) || vring.size() >= cap) return;
+            vring.push_back(g);
+            bad |= he[g].vert ^ v;
+            g = step(g);
         }
-        r.vbnd[v] = g < 0 ? 1 : 0;
+        vbnd[v] = g < 0 ? 1 : 0;
+        if (n != 4 || g < 0) {
+            odd_v.push_back(v);
+            entries += n + (g < 0 ? 1 : 0);
+        }
     }
-    r.voff[V] = (int32_t)r.vring.size();
+    voff[V] = (int32_t)vring.size();
+    r.odd_v_entries = entries;
+    r.bad[0] = bad | ((int64_t)vring.size() != H ? 1 : 0);
+    r.voff = std::move(voff);
+    r.vring = std::move(vring);
+    r.vbnd = std::move(vbnd);
+    r.odd_v = std::move(odd_v);
+    r.part_ok[0] = true;
+}
+
+inline void ring_faces(const cc_Mesh *m, CageRings &r) {
+    const int32_t V = m->vertexCount, F = m->faceCount, H = m->halfedgeCount;
+    std::vector<int32_t> foff = std::move(r.foff), fring = std::move(r.fring), odd_f = std::move(r.odd_f);
+    const CageHe *he = reinterpret_cast<const CageHe *>(m->halfedges);
+    const size_t cap = 4 * (size_t)H + (size_t)V;
+    auto valid = [&](int32_t h) { return h >= 0 && h < H; };
+    int32_t bad = 0;
+    int64_t entries = 0;
+    foff.assign((size_t)F + 1, 0);
+    fring.clear();
+    odd_f.clear();
+    fring.reserve((size_t)H + 1);
     for (int32_t f = 0; f < F; ++f) {
-        r.foff[f] = (int32_t)r.fring.size();
+        foff[f] = (int32_t)fring.size();
         const int32_t p = m->faceToHalfedgeIDs[f];
         if (!valid(p)) continue;
-        r.fring.push_back(p);
-        r.own = r.own && he[p].face == f;
-        int32_t n = 1;
+        fring.push_back(p);
+        bad |= he[p].face ^ f;
+        int32_t n = 1, last = p;
         for (int32_t it = he[p].next; it != p && n < kWalkCap; it = he[it].next, ++n) {
-            if (!valid(it) || r.fring.size() >= cap) return;
-            r.fring.push_back(it);
-            r.own = r.own && he[it].face == f;
+            if (!valid(it) || fring.size() >= cap) return;
+            fring.push_back(it);
+            bad |= (he[it].face ^ f) | (he[it].prev ^ last);
+            last = it;
+        }
+        bad |= (he[p].prev ^ last) | (n < 2 ? 1 : 0);
+        if (n != 4 || he[p].next != p + 1 || he[p + 1].next != p + 2 || he[p + 2].next != p + 3) {
+            odd_f.push_back(f);
+            entries += n;
         }
     }
-    r.foff[F] = (int32_t)r.fring.size();
-    // halfedges by vertex, ascending (a counting sort)
-    r.ooff.assign((size_t)V + 1, 0);
+    foff[F] = (int32_t)fring.size();
+    r.odd_f_entries = entries;
+    r.bad[1] = bad | ((int64_t)fring.size() != H ? 1 : 0);
+    r.foff = std::move(foff);
+    r.fring = std::move(fring);
+    r.odd_f = std::move(odd_f);
+    r.part_ok[1] = true;
+}
+
+// halfedges by vertex, ascending (a counting sort); an edge has one pair of
+// halfedges or one boundary halfedge
+inline void ring_out(const cc_Mesh *m, CageRings &r) {
+    const int32_t V = m->vertexCount, H = m->halfedgeCount, E = m->edgeCount;
+    std::vector<int32_t> ooff = std::move(r.ooff), out = std::move(r.out), fill = std::move(r.fill), bnd = std::move(r.bnd);
+    std::vector<uint8_t> seen = std::move(r.seen);
+    const CageHe *he = reinterpret_cast<const CageHe *>(m->halfedges);
+    ooff.assign((size_t)V + 1, 0);
+    seen.assign((size_t)(E > 0 ? E : 0), 0);
+    bnd.clear();
+    int32_t bad = 0, pairs = 0;
     for (int32_t h = 0; h < H; ++h) {
-        const int32_t v = he[h].vert;
-        if (v < 0 || v >= V) return;
-        ++r.ooff[(size_t)v + 1];
+        const CageHe &x = he[h];
+        if (x.vert < 0 || x.vert >= V) return;
+        ++ooff[(size_t)x.vert + 1];
+        if (x.edge < 0 || x.edge >= E) bad = 1;
+        else seen[x.edge] += h > x.twin ? 1 : 0;
+        pairs += h > x.twin ? 1 : 0;
+        if (x.twin < 0) bnd.push_back(h);
     }
-    for (int32_t v = 0; v < V; ++v) r.ooff[(size_t)v + 1] += r.ooff[v];
-    r.out.assign((size_t)H, 0);
-    r.fill.assign(r.ooff.begin(), r.ooff.end() - 1);
-    for (int32_t h = 0; h < H; ++h) r.out[(size_t)r.fill[he[h].vert]++] = h;
-    r.ok = true;
+    for (const uint8_t n : seen) bad |= n ^ 1;   // (modulo 256; with E pairs in all, one each)
+    for (int32_t v = 0; v < V; ++v) ooff[(size_t)v + 1] += ooff[v];
+    out.assign((size_t)H, 0);
+    fill.assign(ooff.begin(), ooff.end() - 1);
+    for (int32_t h = 0; h < H; ++h) out[(size_t)fill[he[h].vert]++] = h;
+    r.bad[2] = bad | (pairs ^ E);
+    r.ooff = std::move(ooff);
+    r.out = std::move(out);
+    r.fill = std::move(fill);
+    r.bnd = std::move(bnd);
+    r.seen = std::move(seen);
+    r.part_ok[2] = true;
+}
+
+// (into r, whose storage a caller with many cages reuses)
+// threads: a second one for the faces and the outgoing halfedges of a cage of
+// at least kRingThreadsFrom halfedges (whole host calls, depth 1: 524 thousand
+// halfedges 5.6 ms alone and 4.6 with it, 45 thousand 0.74 and 0.60; at 16
+// thousand 0.27 and 0.30)
+constexpr int32_t kRingThreadsFrom = 1 << 15;
+inline void build_cage_rings(const cc_Mesh *m, CageRings &r, bool threads = false) {
+    for (bool &x : r.part_ok) x = false;
+    r.ok = r.simple = false;
+    std::atomic<bool> memory{true};
+    auto rest = [&]() {   // no exception leaves a thread
+        try {
+            ring_faces(m, r);
+            ring_out(m, r);
+        } catch (const std::bad_alloc &) {
+            memory = false;
+        }
+    };
+    std::thread other;
+    if (threads && m->halfedgeCount >= kRingThreadsFrom) {
+        try {
+            other = std::thread(rest);
+        } catch (const std::exception &) {   // no thread to be had: done below
+        }
+    }
+    try {
+        ring_vertices(m, r);
+    } catch (const std::bad_alloc &) {
+        memory = false;
+    }
+    if (other.joinable()) other.join();
+    else rest();
+    if (!memory) throw std::bad_alloc();
+    r.ok = r.part_ok[0] && r.part_ok[1] && r.part_ok[2];
+    if (!r.ok) return;
+    // (rings of as many halfedges as the cage has, none of them twice: all)
+    int32_t bad = r.bad[0] | r.bad[1] | r.bad[2];
+    for (int32_t v = 0; v < m->vertexCount; ++v)   // all of v's in its ring
+        bad |= (r.voff[v + 1] - r.voff[v]) ^ (r.ooff[v + 1] - r.ooff[v]);
+    r.simple = bad == 0;
 }
 
 // The rare-vertex table of a cage (RareView) as one run of int32s: items |
 // entries | boundary halfedges, item and boundary records of four ints,
-// entries of two.  `simple`: every walk closes, links agree, and every vertex,
-// edge and face has all its halfedges in its one ring; a tile pass, which
-// finishes a vertex from whichever ring closes inside a tile, takes no other
-// cage (of two rings at a vertex, both might write it).  `ok` is false when
-// the cage does not fit the table (not simple, or a fan of more than 64
-// entries): its rare vertices then go through the rare list.
+// entries of two.  `ok` is false when the cage does not fit it (not simple, or
+// a fan of more than 64 entries): its rare vertices then go through the rare
+// list.
 struct RareTable {
     std::vector<int32_t> item, ent, bnd;
     int32_t n4 = 0, n8 = 0, n64 = 0, nb = 0;
-    bool ok = false, simple = false;
+    bool ok = false;
     bool empty() const { return n4 + n8 + n64 + nb == 0; }
+    void clear() {
+        ok = false;
+        n4 = n8 = n64 = nb = 0;
+        for (std::vector<int32_t> *x : {&item, &ent, &bnd}) x->clear();
+        for (auto &x : items) x.clear();
+    }
     struct Item { int32_t v, first, n, boundary; };
     std::vector<Item> items[3];   // scratch
-    std::vector<char> seen;
 };
 
 inline void build_rare_table(const cc_Mesh *m, const CageRings &r, RareTable &t) {
-    t.ok = t.simple = false;
-    t.n4 = t.n8 = t.n64 = t.nb = 0;
-    for (std::vector<int32_t> *x : {&t.item, &t.ent, &t.bnd}) x->clear();
-    for (auto &x : t.items) x.clear();
-    const int32_t V = m->vertexCount, F = m->faceCount, H = m->halfedgeCount, E = m->edgeCount;
-    if (!r.ok || !r.own || (int64_t)r.vring.size() != H || (int64_t)r.fring.size() != H) return;
+    t.clear();
+    if (!r.ok || !r.simple) return;
+    const int32_t V = m->vertexCount, E = m->edgeCount;
     const CageHe *he = reinterpret_cast<const CageHe *>(m->halfedges);
-    auto valid = [&](int32_t h) { return h >= 0 && h < H; };
-    t.seen.assign((size_t)E, 0);
-    int32_t pairs = 0;
-    for (int32_t h = 0; h < H; ++h) {
-        const CageHe &x = he[h];
-        if (!valid(x.next) || !valid(x.prev) || x.prev == h || x.next == h || he[x.next].prev != h ||
-            x.twin >= H || x.edge < 0 || x.edge >= E || x.face < 0 || x.face >= F)
-            return;
-        if (x.twin >= 0 && (he[x.twin].twin != h || he[x.twin].edge != x.edge)) return;
-        if (h > x.twin) {   // one pair of halfedges, or one boundary halfedge, per edge
-            if (t.seen[x.edge]) return;
-            t.seen[x.edge] = 1;
-            ++pairs;
-            if (x.twin < 0) t.bnd.insert(t.bnd.end(), {h, x.next, x.edge, 0});
-        }
-    }
-    if (pairs != E) return;
     bool fits = true;
     auto add_item = [&](int32_t v, int32_t n, int32_t boundary, size_t first) {
         const int32_t entries = n + boundary;
@@ -155,46 +265,43 @@ inline void build_rare_table(const cc_Mesh *m, const CageRings &r, RareTable &t)
         t.items[k].push_back({v, (int32_t)(first / 2), n, boundary});
         fits = fits && entries <= 64;
     };
+    std::vector<int32_t> ent = std::move(t.ent);
+    ent.reserve(2 * (size_t)(r.odd_v_entries + r.odd_f_entries));
     auto add_ent = [&](int32_t h, int32_t e, bool odd) {
-        t.ent.push_back(h);
-        t.ent.push_back(odd ? (int32_t)((uint32_t)e | 0x80000000u) : e);
+        ent.push_back(h);
+        ent.push_back(odd ? (int32_t)((uint32_t)e | 0x80000000u) : e);
     };
-    for (int32_t v = 0; v < V; ++v) {
+    // (a closed ring of four marked_ring_fan and structural_ring take: every
+    // entry R has a twin w, and next(w) is the entry before it)
+    for (const int32_t v : r.odd_v) {
         const int32_t o = r.voff[v], n = r.voff[v + 1] - o;
-        if (n != r.ooff[v + 1] - r.ooff[v]) return;
-        if (n == 0) continue;   // no halfedge leaves v
         const bool boundary = r.vbnd[v] != 0;
-        // A closed ring of four: marked_ring_fan and structural_ring take it
-        // (every entry has a twin w, and next(w) is the entry before it).
-        if (n == 4 && !boundary) continue;
-        const size_t first = t.ent.size();
+        const size_t first = ent.size();
+        int32_t before = boundary ? -1 : r.vring[o + n - 1];
         for (int32_t i = 0; i < n; ++i) {   // the ring's previous edge is the next entry's edge
-            const int32_t R = r.vring[o + i], w = he[R].twin;
-            const int32_t tw = w >= 0 ? 4 * he[w].next + 3 : -1;
-            add_ent(4 * R, 2 * he[R].edge + (R > w ? 0 : 1), 4 * R < tw);
+            const int32_t R = r.vring[o + i];
+            const CageHe &x = he[R];
+            add_ent(4 * R, 2 * x.edge + (R > x.twin ? 0 : 1), R <= before);   // child 0's twin is 4 before + 3
+            before = R;
         }
-        if (boundary) {
-            const int32_t R = r.vring[o + n - 1], p = he[R].prev;
-            add_ent(4 * R, 2 * he[p].edge + 1, true);
-        }
+        if (boundary) add_ent(4 * before, 2 * he[he[before].prev].edge + 1, true);
         add_item(v, n, boundary ? 1 : 0, first);
+        if (!fits) return;
     }
-    for (int32_t f = 0; f < F; ++f) {
+    for (const int32_t f : r.odd_f) {
         const int32_t o = r.foff[f], n = r.foff[f + 1] - o;
-        if (n == 0) continue;
-        const int32_t p = r.fring[o];
-        if (p + 3 < H && he[p].next == p + 1 && he[p + 1].next == p + 2 && he[p + 2].next == p + 3 &&
-            he[p + 3].next == p)
-            continue;
-        const size_t first = t.ent.size();
+        const size_t first = ent.size();
+        int32_t pr = r.fring[o + n - 1];
         for (int32_t i = 0; i < n; ++i) {
-            const int32_t q = r.fring[o + i], pr = he[q].prev;
-            add_ent(4 * q + 2, 2 * E + pr, 4 * q + 2 < 4 * pr + 1);
+            const int32_t q = r.fring[o + i];
+            add_ent(4 * q + 2, 2 * E + pr, q < pr);   // 4 q + 2 < 4 pr + 1
+            pr = q;
         }
         add_item(V + f, n, 0, first);
+        if (!fits) return;
     }
-    t.simple = true;
-    if (!fits) return;
+    t.ent = std::move(ent);
+    for (const int32_t h : r.bnd) t.bnd.insert(t.bnd.end(), {h, he[h].next, he[h].edge, 0});
     for (const auto &group : t.items) {
         const int32_t *p = reinterpret_cast<const int32_t *>(group.data());
         t.item.insert(t.item.end(), p, p + 4 * group.size());
@@ -202,7 +309,7 @@ inline void build_rare_table(const cc_Mesh *m, const CageRings &r, RareTable &t)
     t.n4 = (int32_t)t.items[0].size();
     t.n8 = (int32_t)t.items[1].size();
     t.n64 = (int32_t)t.items[2].size();
-    t.nb = (int32_t)(t.bnd.size() / 4);
+    t.nb = (int32_t)r.bnd.size();
     t.ok = true;
 }
 

@@ -50,7 +50,7 @@ struct ccd_Subd {
     // the rare-vertex table (cch::RareView) in `rings`, rare_on when the cage
     // fits it; offsets in ints
     bool rare_on = false;
-    bool simple = false;   // cch::RareTable::simple
+    bool simple = false;   // cch::CageRings::simple
     size_t o_ritem = 0, o_rent = 0, o_rbnd = 0;
     int32_t rare_n4 = 0, rare_n8 = 0, rare_n64 = 0, rare_nb = 0;
     // levels 1..D, cumulative, laid out as cc_Subd's arrays
@@ -116,7 +116,7 @@ struct ccd_Subd {
     bool alloc(const cc_Mesh *cage, int32_t depth);
     int32_t autotune(int32_t steps, hipStream_t st);
     void free_all();
-    bool upload_cage(const cc_Mesh *cage, hipStream_t st);
+    bool upload_cage(const cc_Mesh *cage, hipStream_t st, bool kept);
     cch::DCage cage_view(const cch::P3 *points) const;
     cch::Lvl level_view(int d, const cch::P3 *levelPts, cch::P3 *nextPts) const;
     cch::FusedArgs fused_args(int d, const cch::P3 *points) const;

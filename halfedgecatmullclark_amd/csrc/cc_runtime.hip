@@ -124,7 +124,9 @@ void ccd_Subd::drop_graphs() {
     graphs.clear();
 }
 
-bool ccd_Subd::upload_cage(const cc_Mesh *cage, hipStream_t st) try {
+// kept: for many calls, with the rare-vertex table whenever the cage fits it;
+// else for one forward call, with it where it pays
+bool ccd_Subd::upload_cage(const cc_Mesh *cage, hipStream_t st, bool kept) try {
     if (cage->vertexCount != V0 || cage->uvCount != U0 || cage->halfedgeCount != H0 ||
         cage->edgeCount != E0 || cage->faceCount != F0) {
         set_error(10, "cage counts differ from the ones the device mirror was created for");
@@ -134,33 +136,17 @@ bool ccd_Subd::upload_cage(const cc_Mesh *cage, hipStream_t st) try {
     for (bool &v : own_valid) v = false;
     adj_vp_key = -1;
     drop_graphs();
-    CageRings &r = cage_rings;
-    RareTable &rt = cage_rare;
-    build_cage_rings(cage, r);
-    rings_ok = r.ok;
-    build_rare_table(cage, r, rt);
-    rare_free = rt.ok && rt.empty();
-    rare_on = rt.ok;
-    simple = rt.simple;
-    rare_n4 = rt.n4; rare_n8 = rt.n8; rare_n64 = rt.n64; rare_nb = rt.nb;
-    if (!rt.ok) {   // the rare-vertex list: cage vertices, cage faces and boundary vertices
-        int64_t b0 = 0;
-        const CageHe *ch = reinterpret_cast<const CageHe *>(cage->halfedges);
-        for (int32_t h = 0; h < H0; ++h) b0 += ch[h].twin < 0 ? 1 : 0;
-        const int64_t cap = std::min<int64_t>((int64_t)V0 + F0 + (b0 << (D >= 1 ? D - 1 : 0)), INT32_MAX - 1);
-        if (cap > rare_cap || !rare) {
-            if (rare) (void)hipFree(rare);
-            rare = nullptr;
-            rare_cap = 0;
-            CC_TRY(hipMalloc(&rare, sizeof(int32_t) * (size_t)(cap + 1)), "hipMalloc(rare vertices)");
-            rare_cap = (int32_t)cap;
-        }
-    }
     // The cage's arrays, then its ring lists (vertex offsets | boundary flags |
     // face offsets | vertex rings | face rings | outgoing halfedges), each
-    // padded by one entry, and its rare-vertex table: packed on the host and
-    // copied at once (a host refinement of a 512-face torus to depth 6: 4044
-    // us with nine copies from pageable memory, 3997 us with one).
+    // padded by one entry, and its rare-vertex table, in one allocation.  A
+    // small cage is packed on the host and copied at once (a host refinement
+    // of a 512-face torus to depth 6: 4044 us with nine copies from pageable
+    // memory, 3997 us with one).  From kDirectFrom bytes of arrays on, a copy
+    // costs less than packing: they go first and the lists are built meanwhile
+    // (131 thousand quads to depth 1: 6.5 ms packed, 4.6 so, the lists' second
+    // thread included; 4 thousand the same, 2 thousand to depth 3 0.63 and
+    // 0.67).
+    constexpr size_t kDirectFrom = 1 << 20;
     struct Part {
         const void *src;
         size_t bytes, off;
@@ -174,6 +160,22 @@ bool ccd_Subd::upload_cage(const cc_Mesh *cage, hipStream_t st) try {
         return off;
     };
     auto list = [&](const std::vector<int32_t> &v) { return add(v.data(), sizeof(int32_t) * v.size()) / sizeof(int32_t); };
+    auto grow = [&](size_t bytes) {
+        if (bytes <= cage_cap) return true;
+        if (cage_arena) (void)hipFree(cage_arena);
+        cage_arena = nullptr;
+        cage_cap = 0;
+        if (hip_failed(hipMalloc(&cage_arena, bytes), "hipMalloc(cage)")) return false;
+        cage_cap = bytes;
+        return true;
+    };
+    auto copy_arrays = [&]() {
+        for (size_t i = 0; i < 7; ++i)
+            if (parts[i].bytes && hip_failed(hipMemcpyAsync(cage_arena + parts[i].off, parts[i].src, parts[i].bytes,
+                                                            hipMemcpyHostToDevice, st), "upload cage"))
+                return false;
+        return true;
+    };
     const size_t p_he = add(cage->halfedges, sizeof(CageHe) * (size_t)H0);
     const size_t p_v2h = add(cage->vertexToHalfedgeIDs, sizeof(int32_t) * (size_t)V0);
     const size_t p_e2h = add(cage->edgeToHalfedgeIDs, sizeof(int32_t) * (size_t)E0);
@@ -181,6 +183,45 @@ bool ccd_Subd::upload_cage(const cc_Mesh *cage, hipStream_t st) try {
     const size_t p_pts = add(cage->vertexPoints, sizeof(P3) * (size_t)V0);
     const size_t p_uvs = add(cage->uvs, U0 > 0 ? sizeof(UV) * (size_t)U0 : 0);
     const size_t p_cr = add(cage->creases, sizeof(Crease) * (size_t)E0);
+    const bool direct = size >= kDirectFrom;
+    if (direct) {   // with room for the lists of a cage whose walks close, and a table
+        size_t room = sizeof(int32_t) * (3 * (size_t)H0 + 3 * (size_t)V0 + (size_t)F0 + 3) + 12 * 272;
+        if ((int64_t)H0 != 4 * (int64_t)F0 || (int64_t)H0 != 2 * (int64_t)E0)
+            room += 16 * ((size_t)V0 + F0 + H0) + 24 * (size_t)V0;
+        if (!grow(size + room) || !copy_arrays()) return false;
+    }
+    CageRings &r = cage_rings;
+    RareTable &rt = cage_rare;
+    build_cage_rings(cage, r, true);
+    rings_ok = r.ok;
+    simple = r.simple;
+    // The table costs about 2.7 ns an entry to build and upload, and saves a
+    // launch of about 15 us on each of the D - 1 levels that read it: a mesh
+    // of 45 thousand halfedges and 70 thousand entries to depth 2 takes 0.92
+    // ms without it and 1.00 with it.
+    constexpr int64_t kEntriesPerLevel = 5000;
+    if (D >= 2 && (kept || r.odd_v_entries + r.odd_f_entries <= kEntriesPerLevel * (D - 1))) build_rare_table(cage, r, rt);
+    else rt.clear();
+    rare_free = rt.ok && rt.empty();
+    rare_on = rt.ok;
+    rare_n4 = rt.n4; rare_n8 = rt.n8; rare_n64 = rt.n64; rare_nb = rt.nb;
+    if (!rt.ok && D >= 2) {   // the rare-vertex list: cage vertices, cage faces and boundary vertices
+        int64_t b0 = (int64_t)r.bnd.size();
+        if (!r.ok) {
+            b0 = 0;
+            const CageHe *ch = reinterpret_cast<const CageHe *>(cage->halfedges);
+            for (int32_t h = 0; h < H0; ++h) b0 += ch[h].twin < 0 ? 1 : 0;
+        }
+        const int64_t cap = std::min<int64_t>((int64_t)V0 + F0 + (b0 << (D - 1)), INT32_MAX - 1);
+        if (cap > rare_cap || !rare) {
+            if (rare) (void)hipFree(rare);
+            rare = nullptr;
+            rare_cap = 0;
+            CC_TRY(hipMalloc(&rare, sizeof(int32_t) * (size_t)(cap + 1)), "hipMalloc(rare vertices)");
+            rare_cap = (int32_t)cap;
+        }
+    }
+    const size_t lists = size;
     if (r.ok) {
         o_vro = list(r.voff);
         o_vb = list(r.vbnd);
@@ -195,17 +236,13 @@ bool ccd_Subd::upload_cage(const cc_Mesh *cage, hipStream_t st) try {
         o_rent = list(rt.ent);
         o_rbnd = list(rt.bnd);
     }
-    if (size > cage_cap) {
-        if (cage_arena) (void)hipFree(cage_arena);
-        cage_arena = nullptr;
-        cage_cap = 0;
-        CC_TRY(hipMalloc(&cage_arena, size), "hipMalloc(cage)");
-        cage_cap = size;
-    }
-    if (cage_host.size() < size) cage_host.resize(size);
-    for (const Part &x : parts) {
-        if (x.bytes) memcpy(cage_host.data() + x.off, x.src, x.bytes);
-        memset(cage_host.data() + x.off + x.bytes, 0, 16);
+    if (size > cage_cap && (!grow(size) || (direct && !copy_arrays()))) return false;
+    const size_t from = direct ? lists : 0;
+    if (cage_host.size() < size - from) cage_host.resize(size - from);
+    for (size_t i = direct ? 7 : 0; i < parts.size(); ++i) {
+        char *dst = cage_host.data() + (parts[i].off - from);
+        if (parts[i].bytes) memcpy(dst, parts[i].src, parts[i].bytes);
+        memset(dst + parts[i].bytes, 0, 16);
     }
     c_he = reinterpret_cast<CageHe *>(cage_arena + p_he);
     c_v2h = reinterpret_cast<int32_t *>(cage_arena + p_v2h);
@@ -215,8 +252,9 @@ bool ccd_Subd::upload_cage(const cc_Mesh *cage, hipStream_t st) try {
     c_uvs = reinterpret_cast<UV *>(cage_arena + p_uvs);
     c_cr = reinterpret_cast<Crease *>(cage_arena + p_cr);
     rings = reinterpret_cast<int32_t *>(cage_arena);
-    CC_TRY(hipMemcpyAsync(cage_arena, cage_host.data(), size, hipMemcpyHostToDevice, st), "upload cage");
-    CC_TRY(hipStreamSynchronize(st), "upload cage");   // cage_host may change after return
+    if (size > from)
+        CC_TRY(hipMemcpyAsync(cage_arena + from, cage_host.data(), size - from, hipMemcpyHostToDevice, st), "upload cage");
+    CC_TRY(hipStreamSynchronize(st), "upload cage");   // cage_host and the cage may change after return
     return true;
 } catch (const std::bad_alloc &) {
     set_error(2, "out of host memory");
@@ -701,7 +739,7 @@ bool host_refine(cc_Subd *subd, int32_t steps, int dmax, const char *fname) {
     DeviceGuard g(s->device);
     hipStream_t st = s->stream;
     const cc_Mesh *cage = subd->cage;
-    if (!s->upload_cage(cage, st)) return false;
+    if (!s->upload_cage(cage, st, false)) return false;
     const Counts &n = s->n;
     const bool uvActive = kHasUv && (steps & CCD_UVS) && s->U0 > 0;
     const bool writesHe = (steps & CCD_HALFEDGES) || uvActive;
@@ -822,7 +860,7 @@ static void host_adjoint(const cc_Subd *subd, const void *dL_dFinest, void *dL_d
     hipStream_t st = s->stream;
     const Counts &n = s->n;
     const int D = s->D;
-    if (!s->upload_cage(subd->cage, st)) return;
+    if (!s->upload_cage(subd->cage, st, true)) return;
     // gradient staging, sized for doubles so both precisions fit
     if (!s->adj_in && hip_failed(hipMalloc(&s->adj_in, 3 * sizeof(double) * (size_t)n.V[D]), "hipMalloc(adjoint input)")) return;
     if (!s->adj_out && hip_failed(hipMalloc(&s->adj_out, 3 * sizeof(double) * (size_t)n.V[0]), "hipMalloc(adjoint output)")) return;
@@ -872,7 +910,7 @@ ccd_Subd *ccd_Create(const cc_Mesh *cage, int32_t maxDepth) {
     ccd_Subd *s = create_mirror(cage, maxDepth);
     if (!s) return nullptr;
     DeviceGuard g(s->device);
-    if (!s->upload_cage(cage, s->stream) || hip_failed(hipStreamSynchronize(s->stream), "ccd_Create")) {
+    if (!s->upload_cage(cage, s->stream, true) || hip_failed(hipStreamSynchronize(s->stream), "ccd_Create")) {
         s->free_all();
         delete s;
         return nullptr;

@@ -6,13 +6,13 @@
 
 using namespace cch;
 
-// bit 0: the cage has ring lists, 1: RareTable::simple, 2: RareTable::ok
+// bit 0: the cage has ring lists, 1: CageRings::simple, 2: RareTable::ok
 extern "C" int32_t check_rare_table(const cc_Mesh *m) {
     CageRings r;
     RareTable t;
     build_cage_rings(m, r);
     build_rare_table(m, r, t);
-    return (r.ok ? 1 : 0) | (t.simple ? 2 : 0) | (t.ok ? 4 : 0);
+    return (r.ok ? 1 : 0) | (r.simple ? 2 : 0) | (t.ok ? 4 : 0);
 }
 
 // the byte offset at3 gives element i of 12- and 24-byte records
@@ -48,4 +48,15 @@ extern "C" int32_t check_lists(const cc_Mesh *m, int32_t count, int64_t left) {
     for (const CageLists &l : lists)
         if (!l.r.ok || !l.rt.ok) return 2;
     return 1;
+}
+
+// do the lists agree whether one thread or two build them?
+extern "C" int32_t check_threads(const cc_Mesh *m) {
+    CageRings a, b;
+    build_cage_rings(m, a, false);
+    build_cage_rings(m, b, true);
+    return a.ok == b.ok && a.simple == b.simple && a.voff == b.voff && a.vring == b.vring && a.vbnd == b.vbnd &&
+           a.foff == b.foff && a.fring == b.fring && a.ooff == b.ooff && a.out == b.out && a.odd_v == b.odd_v &&
+           a.odd_f == b.odd_f && a.bnd == b.bnd && a.odd_v_entries == b.odd_v_entries &&
+           a.odd_f_entries == b.odd_f_entries;
 }

@@ -57,3 +57,10 @@ def test_lists_without_memory(checks):
     assert checks.check_lists(p, 16, -1) == 1
     got = [checks.check_lists(p, 16, k) for k in range(60)]
     assert set(got) <= {0, 1} and 0 in got
+
+
+@pytest.mark.parametrize("name,cage", [("irregular", C.irregular(5)), ("torus", C.torus(128, 66))],
+                         ids=lambda x: x if isinstance(x, str) else "")
+def test_lists_on_two_threads(checks, name, cage):
+    assert cage.H >= 1 << 15
+    assert checks.check_threads(MeshView(cage.contiguous()).pointer)
