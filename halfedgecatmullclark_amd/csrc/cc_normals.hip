@@ -11,7 +11,9 @@
 // Two kernels: tile by tile, one thread per quad, the corner normals and the
 // vertex normals of rings that close inside the tile; then the other vertices
 // from the corner normals the first stored.  Corner normals alone, and cages
-// without ring lists, take one thread per halfedge.
+// where a vertex may have several rings (CageRings::simple), take one thread
+// per halfedge: vertex by vertex, only the representative's ring would be
+// written.
 #include <stdio.h>
 
 #include "cc_fan.h"
@@ -263,7 +265,7 @@ bool ccd_Subd::normals(P3 *out, bool smooth, hipStream_t st) {
             return false;
         corner = nrm_tmp;
     }
-    if (smooth && D >= 1 && rings_ok) {
+    if (smooth && D >= 1 && simple) {
         uint64_t *mask = reinterpret_cast<uint64_t *>(nrm_tmp + H);   // H is a multiple of 4: 8-byte aligned
         const int32_t F = (int32_t)(H / 4);
         const bool big = F >= kTileBigFrom;

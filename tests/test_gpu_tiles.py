@@ -185,3 +185,22 @@ def test_split_edge(name, nu, nv, variant):
                 assert np.array_equal(got["halfedges"][k], want["halfedges"][k]), k
     ds.close()
     b.close()
+
+
+def test_normals_of_two_rings_at_a_vertex():
+    """the halfedges of both rings of a shared vertex get their own ring's
+    normal"""
+    import torch
+    from halfedgecatmullclark_amd import capi
+    from oracle import oracle as O
+    from tests.helpers import welded_tori
+    st = torch.cuda.current_stream().cuda_stream
+    for c, depth in ((welded_tori(3, 3, 0, 4), 1), (welded_tori(3, 3, 0, 4), 2), (welded_tori(5, 4, 7, 2), 4)):
+        ds = capi.DeviceSubd(c, depth)
+        ds.refine(15, st)
+        out = torch.full((ds.n["H"][depth], 3), 7.0, device="cuda")
+        ds.halfedge_normals(out.data_ptr(), True, st)
+        got = out.cpu().numpy()
+        want = O.halfedge_normals(ds.download(), depth, True)
+        ds.close()
+        assert_bytes_equal(got, np.ascontiguousarray(want).reshape(got.shape), f"welded {c.H} {depth}")
