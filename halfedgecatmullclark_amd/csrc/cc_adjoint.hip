@@ -5,14 +5,20 @@
 // CatmullClark.h:1437-1991 and :2032-2615, depend only on valence, crease
 // count, boundary and sharpness).  The adjoint applies the transposes level
 // by level, finest first.  For a level step d -> d+1 (d >= 1) it runs in
-// gather form, without atomics, in three passes:
+// gather form, without atomics:
 //   P. parameters: the owner of each level-d vertex packs its vertex rule's
 //      parameters (valence, boundary, rule, the first two sharp ring edges:
-//      16 bytes, VParam) from its ring;
-//   Q. quads: the four lanes of each quad form, from their corners'
-//      parameters, the vertex rule's shares of each of the quad's edges and
-//      the updated edge gradients (the larger halfedge of a pair stores its
-//      edge's), then the updated face gradient;
+//      16 bytes, VParam) from its ring; kept across calls;
+//   tiles: the four lanes of each quad form, from their corners' parameters,
+//      the vertex rule's shares of each of the quad's edges and the updated
+//      edge and face gradients, then each halfedge its share of its vertex's
+//      gradient, summed for the rings of four that close inside the tile;
+//   border: the vertices whose rings leave their tile, from the shares that
+//      the tiles stored for them, and those of the cage's rare-vertex table.
+// A cage without that table takes two passes instead of the tiles and the
+// border:
+//   Q. quads: the updated edge gradients (the larger halfedge of a pair stores
+//      its edge's) and face gradients;
 //   R. vertices: the owner of each vertex gathers its level-d gradient from
 //      the vertex rule (its own weight), its edges' and its faces' updated
 //      gradients.

@@ -107,15 +107,6 @@ __device__ __forceinline__ P3 face_rule(P3 p0, P3 p1, P3 p2, P3 p3, bool gather)
     return a;
 }
 
-// The same from each lane's own corner, by DPP; the quarters are taken before
-// the exchange, which then folds into the additions.
-template <int GATHER>
-__device__ __forceinline__ P3 quad_face_rule(P3 P) {
-    if (GATHER) return face_rule(quad_bcast3<0>(P), quad_bcast3<1>(P), quad_bcast3<2>(P), quad_bcast3<3>(P), true);
-    const P3 q = P3{P.x / 4.0f, P.y / 4.0f, P.z / 4.0f};
-    return add(add(add(add(zero3(), quad_bcast3<0>(q)), quad_bcast3<1>(q)), quad_bcast3<2>(q)), quad_bcast3<3>(q));
-}
-
 __device__ __forceinline__ P3 quad_face(const He *he, const P3 *old, int32_t quad_base, bool gather) {
     const HeView q4{he + quad_base};
     return face_rule(old[q4[0].z], old[q4[1].z], old[q4[2].z], old[q4[3].z], gather);

@@ -395,8 +395,8 @@ struct RingVertexFn {
 };
 
 // vertex points of the owners the fused kernel marked, or of the far ones the
-// tile kernel left; `wave` is the
-// index of this wave among the level's waves (WORDS words each)
+// tile kernel left; `wave` is the index of this wave among the level's waves
+// (WORDS words each)
 template <int GATHER, int CREASED, int WORDS, class LP>
 __device__ __forceinline__ void level_vertices_masked(const FusedArgs &a, const DCage &c, const LevelTab &t,
                                                       const LP &lp, int d, int32_t wave) {
