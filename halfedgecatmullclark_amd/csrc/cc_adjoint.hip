@@ -338,7 +338,7 @@ template <typename T, int CREASED, bool DERIVE>
 __device__ __forceinline__ void adj_quad_gather(const AdjArgs<T> &a, int32_t h, QuadIn<T> &q) {
     const int32_t g = q.live ? h : h & 3;
     if (DERIVE) q.x = derived_record(q.x, g, a.pV, a.pF, a.pE);
-    q.gv = *at3(reinterpret_cast<const V3<T> *>(a.gV), q.x.z);
+    q.gv = *at3v(reinterpret_cast<const V3<T> *>(a.gV), q.x.z);
     q.ge = *at3(reinterpret_cast<const V3<T> *>(a.gE), q.x.y);
     q.gf = *at3(reinterpret_cast<const V3<T> *>(a.gF), g >> 2);
     q.ts = CREASED ? sharp_at(a, q.x.y) : (T)0;
@@ -450,7 +450,7 @@ __device__ __forceinline__ int32_t border_slot(const AdjArgs<T> &a, int32_t h) {
 template <typename T>
 __device__ __forceinline__ void adj_vertex_store(const AdjArgs<T> &a, int32_t v, const V3<T> &gv, T alpha,
                                                  const V3<T> &acc) {
-    *at3(reinterpret_cast<V3<T> *>(a.gP), v) = {alpha * gv.x + acc.x, alpha * gv.y + acc.y, alpha * gv.z + acc.z};
+    *at3v(reinterpret_cast<V3<T> *>(a.gP), v) = {alpha * gv.x + acc.x, alpha * gv.y + acc.y, alpha * gv.z + acc.z};
 }
 
 template <typename T, int CREASED, bool DERIVE>
@@ -554,7 +554,7 @@ struct BorderFn {
         // other fans are the rare-vertex table's
         if (!marked_ring_fan(h, d, c, t, lp.he, f, v) || !structural_ring(f, t, d, v, r, e, c)) return;
         sort4(r);
-        const V3<T> gv = *at3(reinterpret_cast<const V3<T> *>(a.gV), v);
+        const V3<T> gv = *at3v(reinterpret_cast<const V3<T> *>(a.gV), v);
         W4<T> s[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) s[k] = reinterpret_cast<const W4<T> *>(a.Cs)[border_slot(a, r[k])];

@@ -62,15 +62,16 @@ __host__ __device__ __forceinline__ T *at32(T *p, uint32_t i) {
     return reinterpret_cast<T *>(reinterpret_cast<char *>(p) + i * (uint32_t)sizeof(T));
 }
 // Element i >= 0 of an array of 12- or 24-byte records (points, creases,
-// gradients, normals) gathered at a per-lane index: 3 i as one 64-bit
-// shift-add, the address as another.  Left to itself the compiler takes a
-// 64-bit multiply-add (quarter rate) for each.  (3 i in 32 bits does for the
-// edges, faces and halfedges of a level, below 2^30 by the limits on IDs, but
-// not for its vertices, which halfedges need not use; it is no faster: 2866
-// and 2884 us for a fit of the 64 x 32 torus at depth 8.)  For the adjoint,
-// the tile kernel and the normals, which are short of issue slots; in the
-// fused level kernel the same change moves the loads behind the child stores:
-// 2433 -> 2671 us at level 7 of that torus.
+// gradients, normals) gathered at a per-lane index: 3 i as a shift-add, the
+// address as a 64-bit shift-add.  Left to itself the compiler takes a 64-bit
+// multiply-add (quarter rate) for each.  at3: edges, faces and halfedges of a
+// level, which the limits on IDs keep below 2^30, so that 3 i fits 32 bits.
+// at3v: vertices, of which a cage may have up to 2^31 (halfedges need not use
+// them all), with 3 i in 64 bits; everywhere, it would spill two more
+// registers in the creased gather form of the tile kernel.
+// For the adjoint, the tile kernel and the normals, which are short of issue
+// slots; in the fused level kernel the same change moves the loads behind the
+// child stores: 2433 -> 2671 us at level 7 of the 64 x 32 torus.
 __host__ __device__ __forceinline__ uint64_t times3(uint32_t i) {
 #ifdef __HIP_DEVICE_COMPILE__
     uint64_t r;
@@ -84,7 +85,13 @@ template <class T>
 __host__ __device__ __forceinline__ T *at3(T *p, int32_t i) {
     static_assert(sizeof(T) == 12 || sizeof(T) == 24, "three words or three double words");
     using C = std::conditional_t<std::is_const_v<T>, const char, char>;
-    return reinterpret_cast<T *>(reinterpret_cast<C *>(p) + (times3((uint32_t)i) << (sizeof(T) == 12 ? 2 : 3)));
+    return reinterpret_cast<T *>(reinterpret_cast<C *>(p) + ((uint64_t)(3u * (uint32_t)i) << (sizeof(T) == 12 ? 2 : 3)));
+}
+template <class T>
+__host__ __device__ __forceinline__ T *at3v(T *p, int32_t v) {
+    static_assert(sizeof(T) == 12 || sizeof(T) == 24, "three words or three double words");
+    using C = std::conditional_t<std::is_const_v<T>, const char, char>;
+    return reinterpret_cast<T *>(reinterpret_cast<C *>(p) + (times3((uint32_t)v) << (sizeof(T) == 12 ? 2 : 3)));
 }
 __host__ __device__ __forceinline__ int4 he_load(const HeRec<12> *p, int64_t i) {
     const int32_t *q = reinterpret_cast<const int32_t *>(p) + 3 * i;

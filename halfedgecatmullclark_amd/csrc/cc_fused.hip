@@ -44,8 +44,8 @@ __global__ __launch_bounds__(NT) void k_level_fused(FusedArgs a, DCage c, LevelT
     }
 }
 
-// (eight waves per SIMD: 56 registers, 64 by the gather rules, whose creased
-// form spills 4)
+// (eight waves per SIMD: 55 registers, 64 by the gather rules, whose creased
+// form spills 2)
 template <int GATHER, int CREASED, int N>
 __global__ __launch_bounds__(N, 8) void k_level_points(FusedArgs a) {
     point_tile<GATHER, CREASED, N>(a, xcd_block(blockIdx.x, gridDim.x, a.xcd_remap));

@@ -150,7 +150,7 @@ __global__ __launch_bounds__(N, 8) void k_normal_tiles(const He *__restrict__ he
 #pragma unroll
         for (int k = 0; k < 4; ++k) x[k] = he_gld(he, 4 * g + k);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) P[k] = gld(at3(pts, x[k].z));
+        for (int k = 0; k < 4; ++k) P[k] = gld(at3v(pts, x[k].z));
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             nx[k] = x[(k + 3) & 3].x;

@@ -92,7 +92,7 @@ __device__ __forceinline__ void point_tile(const FusedArgs &a, uint32_t tile) {
     const int32_t w = r.x, wp = quad_rel<kQuadPrev>(w), gp = qprev(g);
     const int32_t e0 = 2 * r.y + (g > w ? 0 : 1), e3 = 2 * quad_rel<kQuadPrev>(r.y) + (gp > wp ? 1 : 0);
     const int32_t v1 = a.pV + a.pF + r.y, v2 = a.pV + (g >> 2);
-    const P3 P0 = gld(at3(a.old, r.z)), P1 = gld(at3(a.old, v1)), P2 = gld(at3(a.old, v2));
+    const P3 P0 = gld(at3v(a.old, r.z)), P1 = gld(at3v(a.old, v1)), P2 = gld(at3v(a.old, v2));
     float s0 = 0.0f, s3 = 0.0f;          // (edges inside p's quad have no sharpness)
     if (CREASED && __any(e0 < a.C || e3 < a.C)) {
         s0 = sharp(e0);
@@ -172,14 +172,14 @@ __device__ __forceinline__ void point_tile(const FusedArgs &a, uint32_t tile) {
         const P3 c2 = share(P2, E2, F);
         const P3 v = add(add(add(add(zero3(), quad_bcast3<0>(c2)), quad_bcast3<1>(c2)), quad_bcast3<2>(c2)),
                          quad_bcast3<3>(c2));
-        if (live && (g & 3) == 0) *at3(a.vp, v2) = v;
+        if (live && (g & 3) == 0) *at3v(a.vp, v2) = v;
     }
     if (GATHER) {
         const P3 E2 = quad_rel3<kQuadPrev>(E1);
         const P3 Fq[4] = {quad_bcast3<0>(F), quad_bcast3<1>(F), quad_bcast3<2>(F), quad_bcast3<3>(F)};
         const P3 Eq[4] = {quad_bcast3<0>(E2), quad_bcast3<1>(E2), quad_bcast3<2>(E2), quad_bcast3<3>(E2)};
         const P3 v = smooth_gather4<CREASED>(Fq, Eq, P2);
-        if (live && (g & 3) == 0) *at3(a.vp, v2) = v;
+        if (live && (g & 3) == 0) *at3v(a.vp, v2) = v;
     }
     // the level's owner bits, four of each lane
     uint32_t own = 0;
@@ -193,10 +193,10 @@ __device__ __forceinline__ void point_tile(const FusedArgs &a, uint32_t tile) {
         if (done1 && (own & 2u) != 0u) {
             const P3 Fq[4] = {F, tile_get(sA, qnext(w) - base), tile_get(sA, w - base), Fn};
             const P3 Eq[4] = {E1, E0, tile_get(sD, w - base), E3n};
-            *at3(a.vp, v1) = smooth_gather4<CREASED>(Fq, Eq, P1);
+            *at3v(a.vp, v1) = smooth_gather4<CREASED>(Fq, Eq, P1);
         }
     } else if (live && done1 && g > w) {
-        *at3(a.vp, v1) = add(add(tile_get(sD, w - base), a1), a2);
+        *at3v(a.vp, v1) = add(add(tile_get(sD, w - base), a1), a2);
     }
     // p's vertex: p's ring, four times x -> twin(prev(x))
     const int32_t r1 = sring[q];
@@ -219,13 +219,13 @@ __device__ __forceinline__ void point_tile(const FusedArgs &a, uint32_t tile) {
             const int32_t x1 = r1 - base, x2 = r2 - base, x3 = r3 - base;
             const P3 Fq[4] = {F, tile_get(sA, x1), tile_get(sA, x2), tile_get(sA, x3)};
             const P3 Eq[4] = {E0, tile_get(sC, x1), tile_get(sC, x2), tile_get(sC, x3)};
-            *at3(a.vp, r.z) = smooth_gather4<CREASED>(Fq, Eq, P0);
+            *at3v(a.vp, r.z) = smooth_gather4<CREASED>(Fq, Eq, P0);
         }
     } else if (ring && g < r1 && g < r2 && g < r3) {   // shares in ascending halfedge order
         const int32_t lo = r1 < r2 ? r1 : r2, hi = r1 < r2 ? r2 : r1;
         const int32_t x3 = hi > r3 ? hi : r3, m = hi > r3 ? r3 : hi;
         const int32_t x1 = lo < m ? lo : m, x2 = lo < m ? m : lo;
-        *at3(a.vp, r.z) = add(add(add(add(zero3(), c0), tile_get(sC, x1 - base)), tile_get(sC, x2 - base)),
+        *at3v(a.vp, r.z) = add(add(add(add(zero3(), c0), tile_get(sC, x1 - base)), tile_get(sC, x2 - base)),
                               tile_get(sC, x3 - base));
     }
     // Outer edges whose twin lies in another tile, one lane each (every wave
@@ -240,8 +240,8 @@ __device__ __forceinline__ void point_tile(const FusedArgs &a, uint32_t tile) {
         const int32_t t = last ? y.x : qnext(y.x);
         const int32_t e = 2 * y.y + ((last ? qprev(f) : f) > y.x ? 0 : 1);
         const int4 y0 = he_gld(a.par, t), y3 = he_gld(a.par, qprev(t));
-        const P3 Q0 = gld(at3(a.old, y0.z)), Q1 = gld(at3(a.old, a.pV + a.pF + y0.y));
-        const P3 Q2 = gld(at3(a.old, a.pV + (t >> 2))), Q3 = gld(at3(a.old, a.pV + a.pF + y3.y));
+        const P3 Q0 = gld(at3v(a.old, y0.z)), Q1 = gld(at3v(a.old, a.pV + a.pF + y0.y));
+        const P3 Q2 = gld(at3v(a.old, a.pV + (t >> 2))), Q3 = gld(at3v(a.old, a.pV + a.pF + y3.y));
         const int32_t ee = last ? (e ^ 1) : e;
         const float ts = CREASED ? sharp(ee) : 0.0f;
         const P3 Ft = face_rule(Q0, Q1, Q2, Q3, GATHER);

@@ -15,13 +15,15 @@ extern "C" int32_t check_rare_table(const cc_Mesh *m) {
     return (r.ok ? 1 : 0) | (r.simple ? 2 : 0) | (t.ok ? 4 : 0);
 }
 
-// the byte offset at3 gives element i of 12- and 24-byte records
+// the byte offset at3 (at3v: vertices) gives element i of 12- and 24-byte records
 struct Six { int32_t w[6]; };
-extern "C" uint64_t check_at3(int32_t i, int32_t bytes) {
+extern "C" uint64_t check_at3(int32_t i, int32_t bytes, int32_t vertices) {
     char *base = reinterpret_cast<char *>(uintptr_t(1) << 40);
-    const void *p = bytes == 12 ? (const void *)at3(reinterpret_cast<const P3 *>(base), i)
-                                : (const void *)at3(reinterpret_cast<Six *>(base), i);
-    return (uint64_t)(static_cast<const char *>(p) - base);
+    const P3 *p = reinterpret_cast<const P3 *>(base);
+    Six *q = reinterpret_cast<Six *>(base);
+    const void *r = bytes == 12 ? (const void *)(vertices ? at3v(p, i) : at3(p, i))
+                                : (const void *)(vertices ? at3v(q, i) : at3(q, i));
+    return (uint64_t)(static_cast<const char *>(r) - base);
 }
 
 // allocations until one fails (-1: none does), this library's alone

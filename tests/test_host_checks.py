@@ -42,11 +42,13 @@ def test_which_cages_take_the_table_and_the_tiles(checks, name, cage, want):
     assert checks.check_rare_table(m.pointer) == want
 
 
-@pytest.mark.parametrize("i", [0, 1, 2 ** 30, 1431655765, 1431655766, 2 ** 31 - 1])
+@pytest.mark.parametrize("i", [0, 1, 2 ** 30 - 1, 1431655765, 1431655766, 2 ** 31 - 1])
 def test_record_offsets(checks, i):
     checks.check_at3.restype = ctypes.c_uint64
     for b in (12, 24):
-        assert checks.check_at3(i, b) == b * i
+        assert checks.check_at3(i, b, 1) == b * i
+        if i < 2 ** 30:
+            assert checks.check_at3(i, b, 0) == b * i
 
 
 def test_lists_without_memory(checks):
