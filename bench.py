@@ -113,14 +113,15 @@ def refinement_bytes(n, D, rec_bytes=16):
 
 def adjoint_bytes(n, D):
     """Compulsory bytes of the adjoint of the points (all steps d+1 -> d,
-    d = D-1 .. 0): per step the level-d topology (16 B per halfedge; 28 B per
-    cage halfedge at d = 0) and creases (12 B) read once, the level-(d+1)
-    gradient (12 B per point) read once and the level-d gradient written
-    once."""
+    d = D-1 .. 0): per step the topology and creases (12 B) read once, the
+    level-(d+1) gradient (12 B per point) read once and the level-d gradient
+    written once.  A step's topology is the cage's (28 B per halfedge) at
+    d = 0 and level 1's (16 B) at d = 1; from d = 2 on level d's records
+    follow from level d-1's."""
     total = 0
     for d in range(D):
-        rec = 28 if d == 0 else 16
-        total += rec * n["H"][d] + 12 * n["V"][d + 1] + 12 * n["V"][d] + 12 * n["C"][d]
+        topology = 28 * n["H"][0] if d == 0 else 16 * n["H"][max(1, d - 1)]
+        total += topology + 12 * n["V"][d + 1] + 12 * n["V"][d] + 12 * n["C"][d]
     return total
 
 
@@ -315,17 +316,18 @@ def main():
         ds.set_timing(per_kernel)
         torch.cuda.synchronize()
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        kern = {}
+        kern, levels = {}, []
         e0.record(stream)
         for _ in range(k):
             ds.refine(steps_flags, sptr)
             if per_kernel:
                 for i, (name, ms) in enumerate(ds.timings()):
                     kern.setdefault((i, name), []).append(ms)
+                levels = ds.timing_levels()
         e1.record(stream)
         torch.cuda.synchronize()
         ds.set_timing(False)
-        return e0.elapsed_time(e1) / k, kern
+        return e0.elapsed_time(e1) / k, kern, levels
 
     ds.refine(capi.ALL, sptr)
     ds.autotune(capi.ALL, sptr)
@@ -333,9 +335,9 @@ def main():
     # the step time with nothing between the launches; then the same steps
     # again with a HIP event pair around every launch (read back after each
     # step) for the per-kernel durations
-    ms_scatter, _ = timed(capi.ALL, args.steps, args.warmup)
-    ms_events, kern = timed(capi.ALL, args.steps, 1, per_kernel=True)
-    ms_gather, _ = timed(capi.ALL | capi.GATHER, max(3, args.steps // 2), 1)
+    ms_scatter, _, _ = timed(capi.ALL, args.steps, args.warmup)
+    ms_events, kern, levels = timed(capi.ALL, args.steps, 1, per_kernel=True)
+    ms_gather, _, _ = timed(capi.ALL | capi.GATHER, max(3, args.steps // 2), 1)
 
     # the adjoint on the same workload: points-only forward (the topology
     # stays), the adjoint of the points, and the two in a row
@@ -375,11 +377,11 @@ def main():
     nrm_ms = {s_: ev_time(lambda: ds.halfedge_normals(nrm.data_ptr(), s_, sptr), 5) for s_ in (False, True)}
     del nrm
     HD, VD = n["H"][D], n["V"][D]
-    nrm_bytes = {False: 16 * HD + 12 * VD + 12 * HD, True: 16 * HD + 12 * VD + 12 * HD + 16 * HD + 24 * HD}
+    nrm_bytes = 16 * HD + 12 * VD + 12 * HD   # either kind: records and points read, normals written
     normals = {"workload": "halfedge normals of the torus 64x32 at depth 8 (ccd_HalfedgeNormals)",
                "corner_ms": nrm_ms[False], "vertex_ms": nrm_ms[True],
-               "corner_gbs": nrm_bytes[False] / (nrm_ms[False] * 1e-3) / 1e9,
-               "vertex_gbs": nrm_bytes[True] / (nrm_ms[True] * 1e-3) / 1e9}
+               "corner_gbs": nrm_bytes / (nrm_ms[False] * 1e-3) / 1e9,
+               "vertex_gbs": nrm_bytes / (nrm_ms[True] * 1e-3) / 1e9}
 
     # the cage builder on a 512 x 256 quad torus with uvs and two crease
     # rings (131,072 faces, 524,288 halfedges): its OBJ text through
@@ -424,20 +426,13 @@ def main():
             "ms_per_step": ms12, "value": hcum / (ms12 * 1e-3),
             "hbm_gbs_algorithmic": refinement_bytes(n, D, 12) / (ms12 * 1e-3) / 1e9}
 
-    # dominant kernel: largest mean duration among the launches of one step;
-    # the per-level kernels run in level order, each level starting with its
-    # fused or patch-local kernel (a level's points may follow its children)
-    labelled, d, split, prev = [], 0, set(), None
-    for (i, nm) in sorted(kern):
-        if nm == "level_points" and prev == "level_fused":
-            split.add(d)
-        elif nm in ("level_fused", "level_points", "level_patch"):
-            d += 1
-        labelled.append(((i, nm), d))
-        prev = nm
+    # dominant kernel: largest mean duration among the launches of one step
+    # (split: the levels whose points follow their children)
+    labelled = [((i, nm), levels[i]) for (i, nm) in sorted(kern)]
+    split = {lv for (_, nm), lv in labelled if nm == "level_points"}
     ((idx, name), level) = max(labelled, key=lambda kv: sum(kern[kv[0]]) / len(kern[kv[0]]))
     # every launch of one step: (name, level, mean ms), the level a kernel
-    # reads (0: cage step and creases)
+    # reads (0: the cage)
     step_kernels = [(nm, lv, round(sum(kern[(i, nm)]) / len(kern[(i, nm)]), 4)) for (i, nm), lv in labelled]
     durs = kern[(idx, name)]
     mean_ms = sum(durs) / len(durs)
