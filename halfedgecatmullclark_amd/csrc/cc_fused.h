@@ -33,7 +33,7 @@ constexpr int64_t kTileBigFrom = 512 * kTileBig;
 // Quads from which a full refinement writes a level's children and owner bits
 // first and its points by tiles, instead of the fused kernel and a vertex
 // kernel that reads every point back: level 7 of the torus 2425 + 646 us
-// against 1775 + 620 + 276; 0.72 M quads 61 + 38 against 49 + 21 + 15; 0.52 M
+// against 1805 + 625 + 280; 0.72 M quads 61 + 38 against 49 + 21 + 15; 0.52 M
 // 46 + 14 against 36 + 12 + 10; 0.58 M of 12-byte records 38 + 15 against 29 +
 // 14 + 10, and one launch more.
 constexpr int64_t kSplitFrom = 640 * 1024;

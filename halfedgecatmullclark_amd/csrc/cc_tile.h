@@ -20,7 +20,9 @@
 // (20 spilled registers: 1450 us).  Level 7 of the torus, tile kernel and far
 // vertices: 1059 + 642 us with the fused kernel and every vertex read back,
 // 1036 + 372 one halfedge at a time, 612 + 345 with tiles of 512 quads, 596 +
-// 277 with 1024 (half as many vertices lie on an edge).
+// 277 with 1024 (half as many vertices lie on an edge); over runs and boxes
+// 596-650 + 276-282.  Only cages whose vertices have one ring each come here
+// (CageRings::simple): whichever ring closes in a tile writes its vertex.
 #pragma once
 
 #include "cc_level.h"
