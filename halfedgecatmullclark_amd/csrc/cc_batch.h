@@ -39,7 +39,7 @@ struct LevelJob {
     int64_t c_he, c_v2h, c_e2h, c_f2h, c_pts, c_uvs, c_cr, c_vro, c_vr, c_vb, c_fro, c_fr, c_voo, c_vo;
     int64_t lp[kMaxDepth + 1];
     int32_t H, V, F, E, C;
-    int32_t cV, cU, cH, cE, cF;
+    int32_t cV, cU, cH, cE, cF, by_pair;
     int32_t xcd_remap, uv_refine, rare_cap, erep_read, erep_write;
     // the rare-vertex table (RareView): offsets and counts, and the
     // workgroups its vertices take in front of the job's in the masked
@@ -77,7 +77,7 @@ struct AdjJob {
     int64_t c_he, c_v2h, c_e2h, c_f2h, c_pts, c_uvs, c_cr, c_vro, c_vr, c_vb, c_fro, c_fr, c_voo, c_vo;
     int64_t lp[kMaxDepth + 1];
     int32_t H, C, V;
-    int32_t cV, cU, cH, cE, cF;
+    int32_t cV, cU, cH, cE, cF, by_pair;
     LevelTab t;
 };
 
@@ -115,6 +115,7 @@ __host__ __device__ __forceinline__ DCage arena_cage(char *base, const J &j) {
     c.vout_off = arena_ptr<const int32_t>(base, j.c_voo);
     c.vout = arena_ptr<const int32_t>(base, j.c_vo);
     c.V = j.cV; c.U = j.cU; c.H = j.cH; c.E = j.cE; c.F = j.cF;
+    c.by_pair = j.by_pair;
     return c;
 }
 

@@ -36,6 +36,7 @@ struct ccb_Batch {
         // through the rare list)
         int64_t o_ritem = -1, o_rent = -1, o_rbnd = -1;
         RareView rv;   // its counts
+        bool by_pair = true;   // DCage::by_pair
         int64_t o_adjVP = 0;   // VParam offset of levels 1..D-1's vertex-rule parameters
         int32_t rare_cap = 0;   // rare-vertex list entries (FusedArgs::rare), the count first
         int64_t o_own[kMaxDepth + 1] = {};   // word offsets of the levels' owner bits
@@ -227,6 +228,7 @@ DCage ccb_Batch::cage_view(int i) const {
     c.fring_off = ring(g.o_fro); c.fring = ring(g.o_fr);
     c.vout_off = ring(g.o_voo); c.vout = ring(g.o_vo);
     c.V = g.V0; c.U = g.U0; c.H = g.H0; c.E = g.E0; c.F = g.F0;
+    c.by_pair = g.by_pair ? 1 : 0;
     return c;
 }
 
@@ -254,6 +256,7 @@ bool ccb_Batch::create(const cc_Mesh *const *meshes, const int32_t *depths, int3
         g.o_f0 = tot_f0; tot_f0 += g.F0;
         all_rings = all_rings && r.ok;
         all_simple = all_simple && r.simple;
+        g.by_pair = r.by_pair;
         if (r.ok) {
             auto put = [&](const std::vector<int32_t> &v) {
                 const int64_t o = (int64_t)rings_host.size();
@@ -434,6 +437,7 @@ bool ccb_Batch::build_tables() {
         j.c_fro = roff(g.o_fro); j.c_fr = roff(g.o_fr);
         j.c_voo = roff(g.o_voo); j.c_vo = roff(g.o_vo);
         j.cV = g.V0; j.cU = g.U0; j.cH = g.H0; j.cE = g.E0; j.cF = g.F0;
+        j.by_pair = g.by_pair ? 1 : 0;
     };
     {   // cage step
         std::vector<CageJob> jobs(N);

@@ -178,6 +178,9 @@ struct DCage {
     // vout_off[v + 1]) (null when the rings are)
     const int32_t *vout_off, *vout;
     int32_t V, U, H, E, F;
+    // 0: the larger halfedge of every level-1 pair represents its edge
+    // (edge_owner_first)
+    int32_t by_pair = 1;
 };
 
 // Loads through explicit address spaces.  A pointer that may point to LDS
@@ -306,6 +309,27 @@ __host__ __device__ inline int32_t edge_rep_first(const DCage &c, int32_t e) {
     return 4 * c.e2h[e >> 1] + 0;
 }
 
+// The halfedge that owns level-1 edge e where kernels give every edge and
+// edge vertex one owner: the larger of its pair.  That is the representative
+// as long as the larger halfedge g of a cage edge represents it and lies, with
+// next(g), beyond next(u) and u, u its twin.  An edge that one face uses twice
+// breaks this (at a tip of it child 0 of g has its twin 4 g + 3 in its own
+// quad), and so do face loops that are not consecutive: from level 2 on the
+// representatives of such an edge's children each have the other child's edge,
+// and both would be without an owner.
+__host__ __device__ inline int32_t edge_owner_first(const DCage &c, int32_t e) {
+    if (c.by_pair && e < 2 * c.E) {
+        const int32_t r = c.e2h[e >> 1], w = c.he[r].twin;
+        if (w >= 0) {
+            const int32_t g = imax(r, w), u = r < w ? r : w;
+            return (e & 1) ? imax(4 * c.he[g].next + 3, 4 * u) : imax(4 * g, 4 * c.he[u].next + 3);
+        }
+    }
+    return edge_rep_first(c, e);
+}
+
+// (OWNER: edge_owner_first's halfedge brought down the levels instead)
+template <bool OWNER = false>
 __host__ __device__ inline int32_t edge_rep(const DCage &c, const LevelTab &t, int32_t e, int d) {
     uint32_t path = 1u;
     int32_t rep = 0;
@@ -320,13 +344,13 @@ __host__ __device__ inline int32_t edge_rep(const DCage &c, const LevelTab &t, i
         path = (path << 1) | (uint32_t)(e & 1);
         e >>= 1;
     }
-    if (k == 1) rep = edge_rep_first(c, e);
+    if (k == 1) rep = OWNER ? edge_owner_first(c, e) : edge_rep_first(c, e);
     for (; path > 1u; path >>= 1) rep = (path & 1u) ? 4 * qnext(rep) + 3 : 4 * rep + 0;
     return rep;
 }
 
-// Is level-d halfedge p (d >= 1) the representative edge_rep(e, d) of its
-// edge e?  Compares level by level from fine to coarse and stops at the
+// Is level-d halfedge p (d >= 1) the owner edge_rep<true>(e, d) of its edge
+// e?  Compares level by level from fine to coarse and stops at the
 // first mismatch, so most calls end after a few integer steps: child 0 of
 // rep(e') represents the even child edge 2e', child 3 of next(rep(e')) the
 // odd one 2e' + 1.
@@ -347,7 +371,7 @@ __host__ __device__ inline bool is_edge_rep(const DCage &c, const LevelTab &t, i
         }
         e >>= 1;
     }
-    return edge_rep_first(c, e) == p;
+    return edge_owner_first(c, e) == p;
 }
 
 __host__ __device__ inline int32_t vertex_rep(const DCage &c, const LevelTab &t, int32_t v, int d) {

@@ -681,7 +681,7 @@ __device__ __forceinline__ void vertex_fan(int32_t v, int d, const DCage &c, con
     const int32_t e = v - Vp - Fp;   // an edge vertex
     int32_t p, tw, np, nt;
     if (b - 1 >= 1) {
-        p = edge_rep(c, t, e, b - 1);
+        p = edge_rep<true>(c, t, e, b - 1);
         tw = levels[b - 1][p].twin;
         np = qnext(p);
         nt = qnext(tw);

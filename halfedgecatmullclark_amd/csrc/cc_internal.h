@@ -55,6 +55,8 @@ struct CageRings {
     std::vector<int32_t> fill;   // scratch
     std::vector<uint8_t> seen;
     bool ok = false, simple = false;
+    bool by_pair = true;   // DCage::by_pair
+    bool pairs[2] = {};    // as the vertices' and the edges' part find it
     int64_t odd_v_entries = 0, odd_f_entries = 0;   // entries the rare-vertex table would have
     bool part_ok[3] = {};
     // of each part, any bit: not simple (gathered without branches)
@@ -70,6 +72,7 @@ inline void ring_vertices(const cc_Mesh *m, CageRings &r) {
     auto valid = [&](int32_t h) { return h >= 0 && h < H; };
     int32_t bad = 0;
     int64_t entries = 0;
+    bool by_pair = false;
     voff.assign((size_t)V + 1, 0);
     vbnd.assign((size_t)V, 0);
     vring.clear();
@@ -84,7 +87,10 @@ inline void ring_vertices(const cc_Mesh *m, CageRings &r) {
             return -1;
         }
         const int32_t g = he[q].twin;
-        if (valid(g)) bad |= (he[g].twin ^ q) | (he[g].edge ^ he[q].edge);
+        if (valid(g)) {
+            bad |= (he[g].twin ^ q) | (he[g].edge ^ he[q].edge);
+            by_pair |= q > g && (q <= he[g].next || h < g);   // (h is next(q))
+        }
         return g;
     };
     for (int32_t v = 0; v < V; ++v) {
@@ -109,6 +115,7 @@ inline void ring_vertices(const cc_Mesh *m, CageRings &r) {
     }
     voff[V] = (int32_t)vring.size();
     r.odd_v_entries = entries;
+    r.pairs[0] = by_pair;
     r.bad[0] = bad | ((int64_t)vring.size() != H ? 1 : 0);
     r.voff = std::move(voff);
     r.vring = std::move(vring);
@@ -168,12 +175,17 @@ inline void ring_out(const cc_Mesh *m, CageRings &r) {
     seen.assign((size_t)(E > 0 ? E : 0), 0);
     bnd.clear();
     int32_t bad = 0, pairs = 0;
+    bool by_pair = false;
     for (int32_t h = 0; h < H; ++h) {
         const CageHe &x = he[h];
         if (x.vert < 0 || x.vert >= V) return;
         ++ooff[(size_t)x.vert + 1];
-        if (x.edge < 0 || x.edge >= E) bad = 1;
-        else seen[x.edge] += h > x.twin ? 1 : 0;
+        if (x.edge < 0 || x.edge >= E) {
+            bad = 1;
+        } else {
+            seen[x.edge] += h > x.twin ? 1 : 0;
+            by_pair |= h > x.twin && m->edgeToHalfedgeIDs[x.edge] != h;
+        }
         pairs += h > x.twin ? 1 : 0;
         if (x.twin < 0) bnd.push_back(h);
     }
@@ -182,6 +194,7 @@ inline void ring_out(const cc_Mesh *m, CageRings &r) {
     out.assign((size_t)H, 0);
     fill.assign(ooff.begin(), ooff.end() - 1);
     for (int32_t h = 0; h < H; ++h) out[(size_t)fill[he[h].vert]++] = h;
+    r.pairs[1] = by_pair;
     r.bad[2] = bad | (pairs ^ E);
     r.ooff = std::move(ooff);
     r.out = std::move(out);
@@ -200,6 +213,7 @@ constexpr int32_t kRingThreadsFrom = 1 << 15;
 inline void build_cage_rings(const cc_Mesh *m, CageRings &r, bool threads = false) {
     for (bool &x : r.part_ok) x = false;
     r.ok = r.simple = false;
+    r.by_pair = true;
     std::atomic<bool> memory{true};
     auto rest = [&]() {   // no exception leaves a thread
         try {
@@ -231,6 +245,7 @@ inline void build_cage_rings(const cc_Mesh *m, CageRings &r, bool threads = fals
     for (int32_t v = 0; v < m->vertexCount; ++v)   // all of v's in its ring
         bad |= (r.voff[v + 1] - r.voff[v]) ^ (r.ooff[v + 1] - r.ooff[v]);
     r.simple = bad == 0;
+    r.by_pair = !r.simple || r.pairs[0] || r.pairs[1];
 }
 
 // The rare-vertex table of a cage (RareView) as one run of int32s: items |

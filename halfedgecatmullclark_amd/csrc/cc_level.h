@@ -274,11 +274,11 @@ __device__ __forceinline__ void level_fused_block(const FusedArgs &a, const DCag
         // through the child numbering): child 0 when h > twin(h) and h
         // represents its edge, child 1 when h is the quad's last halfedge,
         // child 2 unless it is the first, child 3 when prev(h) > twin(prev(h))
-        // and prev(h) represents its edge.  Level 1 takes its own bits from
-        // the cage maps.
+        // and prev(h) represents its edge.  At level 1 the larger halfedge of
+        // a pair does.
         bool rh, rp;
         if (d == 1) {
-            rh = live && edge_rep_first(cg, x.y) == h;
+            rh = live && h > x.x;   // edge_owner_first
             rp = quad_rel<kQuadPrev>(rh ? 1 : 0) != 0;
             const uint64_t m1 = __ballot(rh);
             if ((threadIdx.x & 63u) == 0 && live) *at32(a.erep + (tb.R[1] + (base >> 6)), threadIdx.x >> 6) = m1;

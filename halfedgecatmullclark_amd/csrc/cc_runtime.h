@@ -51,6 +51,7 @@ struct ccd_Subd {
     // fits it; offsets in ints
     bool rare_on = false;
     bool simple = false;   // cch::CageRings::simple
+    bool by_pair = true;    // cch::DCage::by_pair
     size_t o_ritem = 0, o_rent = 0, o_rbnd = 0;
     int32_t rare_n4 = 0, rare_n8 = 0, rare_n64 = 0, rare_nb = 0;
     // levels 1..D, cumulative, laid out as cc_Subd's arrays

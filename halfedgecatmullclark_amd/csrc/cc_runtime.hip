@@ -195,6 +195,7 @@ bool ccd_Subd::upload_cage(const cc_Mesh *cage, hipStream_t st, bool kept) try {
     build_cage_rings(cage, r, true);
     rings_ok = r.ok;
     simple = r.simple;
+    by_pair = r.by_pair;
     // The table costs about 2.7 ns an entry to build and upload, and saves a
     // launch of about 15 us on each of the D - 1 levels that read it: a mesh
     // of 45 thousand halfedges and 70 thousand entries to depth 2 takes 0.92
@@ -274,6 +275,7 @@ DCage ccd_Subd::cage_view(const P3 *points) const {
         c.vring_off = c.vring = c.vring_bnd = c.fring_off = c.fring = c.vout_off = c.vout = nullptr;
     }
     c.V = V0; c.U = U0; c.H = H0; c.E = E0; c.F = F0;
+    c.by_pair = by_pair ? 1 : 0;
     return c;
 }
 

@@ -70,3 +70,38 @@ def welded_tori(nu: int, nv: int, v: int = 0, w: int = 0):
     keep = np.delete(np.arange(2 * n), n + w)
     remap = {int(x): i for i, x in enumerate(keep)}
     return C.from_faces(pts[keep], [[remap[x] for x in f] for f in faces], creases=a[4])
+
+
+def permuted(c, seed: int):
+    """the same cage with its halfedges numbered at random: faces that are not
+    runs of consecutive halfedges, edges represented by either halfedge"""
+    p = np.random.default_rng(seed).permutation(c.H).astype(np.int32)   # old -> new
+    q = c.copy()
+    he = c.halfedges.copy()
+    for k in (0, 1, 2):   # twin, next, prev
+        he[:, k] = np.where(c.halfedges[:, k] >= 0, p[np.maximum(c.halfedges[:, k], 0)], c.halfedges[:, k])
+    q.halfedges[p] = he
+    for a, b in ((q.v2h, c.v2h), (q.e2h, c.e2h), (q.f2h, c.f2h)):
+        a[:] = np.where(b >= 0, p[np.maximum(b, 0)], b)
+    return q
+
+
+def tip_cages():
+    """cages with faces that use an edge twice: an edge that ends inside a
+    face, from its first, a middle and its last corner, a path of two such
+    edges, and a face that is a strip around another one"""
+    out = []
+    pts, faces = C.cube_mesh(3)[:2]
+    pts = [np.asarray(p, np.float32) for p in pts]
+    for name, at, n in (("tip_first", 0, 1), ("tip_middle", 2, 1), ("tip_last", 3, 1), ("tip_path", 1, 2)):
+        f = [list(x) for x in faces]
+        g, v = f[4], f[4][at]
+        new = list(range(len(pts), len(pts) + n))
+        g[at + 1:at + 1] = new + new[:-1][::-1] + [v]
+        mid = sum(pts[x] for x in faces[4]) / 4
+        ps = pts + [pts[v] + (mid - pts[v]) * np.float32(0.3 + 0.2 * k) for k in range(n)]
+        out.append((name, C.from_faces(np.stack(ps), f, creases=[(v, new[0], 1.3), (0, 1, 2.0)])))
+    ring = [[0, 0], [3, 0], [3, 3], [0, 3], [1, 1], [2, 1], [2, 2], [1, 2]]
+    ps = np.array([[x, y, 0.1 * x * y] for x, y in ring], np.float32)
+    out.append(("strip", C.from_faces(ps, [[0, 1, 2, 3, 0, 4, 7, 6, 5, 4], [4, 5, 6, 7]], creases=[(0, 4, 0.6)])))
+    return out

@@ -62,3 +62,19 @@ extern "C" int32_t check_threads(const cc_Mesh *m) {
            a.odd_f == b.odd_f && a.bnd == b.bnd && a.odd_v_entries == b.odd_v_entries &&
            a.odd_f_entries == b.odd_f_entries;
 }
+
+// owners of the edges of level d, out[e]; returns DCage::by_pair
+extern "C" int32_t check_edge_owners(const cc_Mesh *m, int32_t d, int32_t *out) {
+    CageRings r;
+    build_cage_rings(m, r);
+    DCage c = host_cage_view(m);
+    c.by_pair = r.by_pair ? 1 : 0;
+    Counts n;
+    n.init(m->vertexCount, m->halfedgeCount, m->edgeCount, m->faceCount);
+    const LevelTab t = level_tab(n);
+    for (int32_t e = 0; e < (int32_t)n.E[d]; ++e) {
+        out[e] = edge_rep<true>(c, t, e, d);
+        if (!is_edge_rep(c, t, e, d, out[e])) return -1;
+    }
+    return c.by_pair;
+}

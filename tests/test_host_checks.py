@@ -9,7 +9,8 @@ import pytest
 from halfedgecatmullclark_amd import build as B
 from halfedgecatmullclark_amd import cage as C
 from halfedgecatmullclark_amd.abi import MeshView
-from tests.helpers import welded_tori
+from oracle import oracle as O
+from tests.helpers import permuted, tip_cages, welded_tori
 from tests.test_gpu_rare import bipyramid, cone, prism
 
 
@@ -66,3 +67,27 @@ def test_lists_without_memory(checks):
 def test_lists_on_two_threads(checks, name, cage):
     assert cage.H >= 1 << 15
     assert checks.check_threads(MeshView(cage.contiguous()).pointer)
+
+
+OWNERS = [("torus", C.torus(5, 3), 0), ("irregular", C.irregular(1, seed=3), 0), ("cone", cone(5), 0),
+          ("welded", welded_tori(3, 3), 1), ("permuted_torus", permuted(C.torus(4, 3), 1), 1),
+          ("permuted_cone", permuted(cone(7), 2), 1)] + [(n, c, 1) for n, c in tip_cages()]
+
+
+@pytest.mark.parametrize("name,cage,by_pair", OWNERS, ids=[o[0] for o in OWNERS])
+def test_edge_owners(checks, name, cage, by_pair):
+    """every edge of every level has one owner, the larger halfedge of its
+    pair; the reference's representative where it is that halfedge on every
+    level (by_pair 0)"""
+    m = MeshView(cage.contiguous())
+    out = O.refine(cage, 4, O.HALFEDGES)
+    for d in range(1, 5):
+        lv = O.level(out, "halfedges", d)
+        got = np.full(out["counts"]["E"][d], -1, np.int32)
+        assert checks.check_edge_owners(m.pointer, d, ctypes.c_void_p(got.ctypes.data)) == by_pair
+        larger = np.flatnonzero(np.arange(len(lv)) > lv["twinID"])
+        want = np.full_like(got, -1)
+        want[lv["edgeID"][larger]] = larger
+        assert np.array_equal(got, want), (d, np.flatnonzero(got != want)[:5])
+        if not by_pair:
+            assert all(O.edge_to_halfedge(cage, e, d) == got[e] for e in range(0, len(got), 7))
