@@ -5,6 +5,7 @@
 #include <exception>
 #include <new>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include <hip/hip_runtime.h>
@@ -206,9 +207,9 @@ inline void ring_out(const cc_Mesh *m, CageRings &r) {
 
 // (into r, whose storage a caller with many cages reuses)
 // threads: a second one for the faces and the outgoing halfedges of a cage of
-// at least kRingThreadsFrom halfedges (whole host calls, depth 1: 524 thousand
-// halfedges 5.6 ms alone and 4.6 with it, 45 thousand 0.74 and 0.60; at 16
-// thousand 0.27 and 0.30)
+// at least kRingThreadsFrom halfedges (the lists of 524 thousand halfedges 3.33
+// ms on one and 1.85 on two, of 45 thousand 0.44 and 0.28; at 16 thousand a
+// whole host call to depth 1 took 0.27 ms with one and 0.30 with two)
 constexpr int32_t kRingThreadsFrom = 1 << 15;
 inline void build_cage_rings(const cc_Mesh *m, CageRings &r, bool threads = false) {
     for (bool &x : r.part_ok) x = false;
